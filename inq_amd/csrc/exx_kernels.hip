@@ -90,9 +90,9 @@ __device__ __forceinline__ void lds_row_fft_split(C *lds, int r, int q) {
   line_dit<N2, SIGN, C, S>(v, q);
   __builtin_amdgcn_wave_barrier();
   if (r < N1) {
-    const int o = M * line_part_out<S>(q);
+    const int o = line_out_q<N2, S>(q);
 #pragma unroll
-    for (int k = 0; k < M; ++k) row[k + o] = v[k];
+    for (int k = 0; k < M; ++k) row[line_out_j<N2, S>(k) + o] = v[k];
   }
 }
 
@@ -114,7 +114,7 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_f
   C *lds = reinterpret_cast<C *>(smem_raw);
   const int tid = threadIdx.x;
   const int line = (tid >> 6) * Cfg::LPW + (tid & 63) % Cfg::LPW;
-  const int q = (tid & 63) / Cfg::LPW, qo = line_part_out<S>(q);  // part of the line, its output position
+  const int q = (tid & 63) / Cfg::LPW, qo = line_out_q<N1, S>(q);  // part of the line, its output position
   // one work item per work-group, the grid being the work count: a grid-stride loop
   // here made the complex128 96-point kernels spill to scratch
   {
@@ -147,7 +147,7 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_f
       line_dit<N1, -1, C, S>(v, q);
       if (line < N2) {
 #pragma unroll
-        for (int k = 0; k < M1; ++k) lds[(k + qo * M1) * Cfg::STRIDE + z] = v[k];
+        for (int k = 0; k < M1; ++k) lds[(line_out_j<N1, S>(k) + qo) * Cfg::STRIDE + z] = v[k];
       }
     }
     __syncthreads();
@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(256) k_pair_xline(PairDev<T> d, int total) {
   const int NGRP = (NTILE + 3) / 4;
   const long N = (long)N0 * NP;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform per wave
-  const int q = lane / LPW, qo = line_part_out<S>(q);  // part of the line, its output position
+  const int q = lane / LPW, qo = line_out_q<N0, S>(q);  // part of the line, its output position
   // one work item per work-group, the grid being the work count: a grid-stride loop
   // here made the complex128 96-point kernels spill to scratch
   {
@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(256) k_pair_xline(PairDev<T> d, int total) {
     for (int n = 0; n < M; ++n) bload(rs, voff, (unsigned)(S * n * NP * sizeof(C)), v[n]);
     line_dit<N0, -1, C, S>(v, q);
     __builtin_amdgcn_sched_barrier(0);  // keep the kernel factors out of the FFT's live range
-    // frequency f = k + qo N0/S; G + q = m0 b0 + (m1 b1 + m2 b2 + q)
+    // frequency f = line_out_j(k) + qo; G + q = m0 b0 + (m1 b1 + m2 b2 + q)
     const int i1 = Lc / N2, i2 = Lc - (Lc / N2) * N2;
     const T m1 = (T)(i1 >= (N1 + 1) / 2 ? i1 - N1 : i1), m2 = (T)(i2 >= (N2 + 1) / 2 ? i2 - N2 : i2);
     T u[3];
@@ -213,8 +213,9 @@ __global__ void __launch_bounds__(256) k_pair_xline(PairDev<T> d, int total) {
     for (int c = 0; c < 3; ++c) u[c] = m1 * d.b[1][c] + m2 * d.b[2][c] + d.q[c];
 #pragma unroll
     for (int k = 0; k < M; ++k) {
-      const int f = k + qo * M;
-      const T m0 = (T)(f >= (N0 + 1) / 2 ? f - N0 : f);
+      // with swapped stages the register alone decides the half of the line
+      const int j = line_out_j<N0, S>(k), f = j + qo;
+      const T m0 = (T)(line_swapped<N0, S>() ? (j >= N0 / 2 ? f - N0 : f) : (f >= (N0 + 1) / 2 ? f - N0 : f));
       const T g0 = m0 * d.b[0][0] + u[0], g1 = m0 * d.b[0][1] + u[1], g2 = m0 * d.b[0][2] + u[2];
       const T gg = g0 * g0 + g1 * g1 + g2 * g2;
       const T fct = gg < (T)1e-6 ? d.zero : d.scal * rcp_t(gg);
@@ -244,7 +245,7 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_i
   C *lds = reinterpret_cast<C *>(smem_raw);
   const int tid = threadIdx.x;
   const int line = (tid >> 6) * Cfg::LPW + (tid & 63) % Cfg::LPW;
-  const int q = (tid & 63) / Cfg::LPW, qo = line_part_out<S>(q);
+  const int q = (tid & 63) / Cfg::LPW, qo = line_out_q<N1, S>(q);
   // one work item per work-group, the grid being the work count: a grid-stride loop
   // here made the complex128 96-point kernels spill to scratch
   {
@@ -265,7 +266,7 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_i
       line_dit<N1, +1, C, S>(v, q);
       if (line < N2) {
 #pragma unroll
-        for (int k = 0; k < M1; ++k) lds[(k + qo * M1) * Cfg::STRIDE + z] = v[k];
+        for (int k = 0; k < M1; ++k) lds[(line_out_j<N1, S>(k) + qo) * Cfg::STRIDE + z] = v[k];
       }
     }
     __syncthreads();
@@ -337,7 +338,7 @@ __global__ void __launch_bounds__(256) k_pair_cols(PairDev<T> d, int total) {
     fft_split<N1, SIGN, C>::dit(v, half != 0);
     if (ok) {
 #pragma unroll
-      for (int k = 0; k < H1; ++k) tp[(k + half * H1) * n2 + z] = v[k];
+      for (int k = 0; k < H1; ++k) tp[(line_out_j<N1, 2>(k) + line_out_q<N1, 2>(half)) * n2 + z] = v[k];
     }
   }
 }
@@ -367,7 +368,7 @@ __global__ void __launch_bounds__(256) k_pair_rows(PairDev<T> d, int total) {
     fft_split<N2, SIGN, C>::dit(v, half != 0);
     if (ok) {
 #pragma unroll
-      for (int k = 0; k < H2; ++k) row[k + half * H2] = v[k];
+      for (int k = 0; k < H2; ++k) row[line_out_j<N2, 2>(k) + line_out_q<N2, 2>(half)] = v[k];
     }
   }
 }

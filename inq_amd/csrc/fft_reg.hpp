@@ -222,141 +222,250 @@ template <int N, int SIGN, typename C> struct fft_line {
   }
 };
 
-// ---------------------------------------------------------------- lines split over lane pairs
-// A line of even length N is shared by lane l < 32 ("lower") and lane l + 32
-// ("upper") of a wave, N/2 values each, so a lane holds half the registers of
-// fft_line.  One radix-2 stage crosses the pair; v_permlane32_swap hands each
-// lane both values of its pair (no LDS traffic).
+// ---------------------------------------------------------------- lines split over lanes
+// A line of N values is shared by S lanes of a wave, N/S values each, so a lane
+// holds 1/S of the registers of fft_line: S = 2, lanes l and l + 32 (part 0 and
+// 1), or S = 4, lanes l + 16 q (part q).  Radix-2 stages cross the lanes through
+// v_permlane32_swap and v_permlane16_swap, which exchange the upper part's value
+// of one register with the lower part's value of another: swapping v[k] with
+// v[k + M/2] (M values per lane) hands each lane BOTH operands of a butterfly for
+// half of the butterflies.  A stage then costs one swap per two registers and
+// one full butterfly per two values.  Giving both lanes both operands of every
+// butterfly, as the stages for odd M below still do, costs a swap and a move per
+// register and a half butterfly with its own twiddle per value.  The transforms
+// are VALU bound as much as memory bound, so this shows in every pass: H on 128
+// states at 72^3 418.9 -> 395.6 us in complex64 and 1065 -> 927 us in complex128
+// (whose plane passes also lose the 16-lane shuffles through the LDS crossbar).
+//
+// Order of the values, dit in / dif out: part q holds x[S n + q].  dit out / dif
+// in: register j of part q holds X[line_out_j<N, S>(j) + line_out_q<N, S>(q)].
 
-// the values held by the lower and the upper lane of the pair, on both lanes
-__device__ __forceinline__ void pair_vals(float v, float &lo, float &hi) {
-  const unsigned u = __float_as_uint(v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  lo = __uint_as_float(r[0]);
-  hi = __uint_as_float(r[1]);
+__host__ __device__ constexpr int quad_rev(int q) { return ((q & 1) << 1) | (q >> 1); }
+
+// even values per lane: the swapped stages run
+template <int N, int S> __host__ __device__ constexpr bool line_swapped() { return (N / S) % 2 == 0; }
+template <int N, int S> __host__ __device__ constexpr int line_out_j(int j) {
+  constexpr int M = N / S;
+  return line_swapped<N, S>() && j >= M / 2 ? j - M / 2 + N / 2 : j;
 }
-__device__ __forceinline__ void pair_vals(double v, double &lo, double &hi) {
-  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  const unsigned a = (unsigned)u, b = (unsigned)(u >> 32);
-  const auto ra = __builtin_amdgcn_permlane32_swap(a, a, false, false);
-  const auto rb = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-  lo = __longlong_as_double((long long)(((unsigned long long)rb[0] << 32) | ra[0]));
-  hi = __longlong_as_double((long long)(((unsigned long long)rb[1] << 32) | ra[1]));
+template <int N, int S> __host__ __device__ constexpr int line_out_q(int q) {
+  constexpr int M = N / S;
+  if (!line_swapped<N, S>()) return M * (S == 2 ? q : quad_rev(q));
+  return S == 2 ? q * (M / 2) : (q >> 1) * (M / 2) + (q & 1) * M;
 }
+
+// parts 32 lanes apart: a <- (lower part's a, lower part's b), b <- (upper part's a, upper part's b)
+__device__ __forceinline__ void swap32(float &a, float &b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+// the same for parts 16 lanes apart (even and odd rows of 16 lanes)
+__device__ __forceinline__ void swap16(float &a, float &b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap32(double &a, double &b) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(a), v = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)v, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(v >> 32), false, false);
+  a = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+  b = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+__device__ __forceinline__ void swap16(double &a, double &b) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(a), v = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)v, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(v >> 32), false, false);
+  a = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0]));
+  b = __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+template <typename C> __device__ __forceinline__ void cswap32(C &a, C &b) {
+  swap32(a.x, b.x);
+  swap32(a.y, b.y);
+}
+template <typename C> __device__ __forceinline__ void cswap16(C &a, C &b) {
+  swap16(a.x, b.x);
+  swap16(a.y, b.y);
+}
+// the values held by the lower and the upper part, on both
 template <typename C> __device__ __forceinline__ void pair_vals(C v, C &lo, C &hi) {
-  pair_vals(v.x, lo.x, hi.x);
-  pair_vals(v.y, lo.y, hi.y);
+  lo = hi = v;
+  cswap32(lo, hi);
+}
+template <typename C> __device__ __forceinline__ void pair_vals16(C v, C &lo, C &hi) {
+  lo = hi = v;
+  cswap16(lo, hi);
+}
+
+// up ? (SIGN i) t : t
+template <int SIGN, typename C> __device__ __forceinline__ C quarter_if(C t, bool up) {
+  return SIGN > 0 ? C{up ? -t.y : t.x, up ? t.x : t.y} : C{up ? t.y : t.x, up ? -t.x : t.y};
 }
 
 template <int N, int SIGN, typename C> struct fft_split {
   static_assert(N % 2 == 0, "split lines need an even length");
   static constexpr int H = N / 2;
   using T = decltype(C{}.x);
-  // decimation in time: lower lanes hold x[2n], upper lanes x[2n+1] (n < H);
-  // afterwards lower lanes hold X[k], upper lanes X[k + H] (k < H)
+  // decimation in time: lower lanes hold x[2n], upper lanes x[2n+1] (n < H)
   static __device__ __forceinline__ void dit(C (&v)[H], bool upper) {
     fft_line<H, SIGN, C>::run(v);
-    const T sg = upper ? (T)-1 : (T)1;
+    if constexpr (H % 2 == 0) {
+      // lower lanes take the butterflies k < H/2, upper lanes k + H/2, whose
+      // twiddle W^(k + N/4) is a quarter turn further
 #pragma unroll
-    for (int k = 0; k < H; ++k) {
-      C a, b;
-      pair_vals(v[k], a, b);
-      const C t = twmul<N, SIGN>(b, k);
-      v[k] = C{a.x + sg * t.x, a.y + sg * t.y};
+      for (int k = 0; k < H / 2; ++k) {
+        C e = v[k], o = v[k + H / 2];
+        cswap32(e, o);
+        const C t = quarter_if<SIGN>(twmul<N, SIGN>(o, k), upper);
+        v[k] = cadd(e, t);
+        v[k + H / 2] = csub(e, t);
+      }
+    } else {
+      const T sg = upper ? (T)-1 : (T)1;
+#pragma unroll
+      for (int k = 0; k < H; ++k) {
+        C a, b;
+        pair_vals(v[k], a, b);
+        const C t = twmul<N, SIGN>(b, k);
+        v[k] = C{a.x + sg * t.x, a.y + sg * t.y};
+      }
     }
   }
-  // decimation in frequency: lower lanes hold x[n], upper lanes x[n + H];
-  // afterwards lower lanes hold X[2k], upper lanes X[2k + 1]
+  // decimation in frequency, the mirror: afterwards lower lanes hold X[2k], upper lanes X[2k + 1]
   static __device__ __forceinline__ void dif(C (&v)[H], bool upper) {
-    const T sg = upper ? (T)-1 : (T)1;
+    if constexpr (H % 2 == 0) {
 #pragma unroll
-    for (int n = 0; n < H; ++n) {
-      C a, b;
-      pair_vals(v[n], a, b);
-      const C d{a.x + sg * b.x, a.y + sg * b.y};
-      const C t = twmul<N, SIGN>(d, n);
-      v[n] = upper ? t : d;
+      for (int k = 0; k < H / 2; ++k) {
+        C s = cadd(v[k], v[k + H / 2]);
+        C d = quarter_if<SIGN>(twmul<N, SIGN>(csub(v[k], v[k + H / 2]), k), upper);
+        cswap32(s, d);
+        v[k] = s;
+        v[k + H / 2] = d;
+      }
+    } else {
+      const T sg = upper ? (T)-1 : (T)1;
+#pragma unroll
+      for (int n = 0; n < H; ++n) {
+        C a, b;
+        pair_vals(v[n], a, b);
+        const C d{a.x + sg * b.x, a.y + sg * b.y};
+        const C t = twmul<N, SIGN>(d, n);
+        v[n] = upper ? t : d;
+      }
     }
     fft_line<H, SIGN, C>::run(v);
   }
 };
 
-// ---------------------------------------------------------------- lines split over four lanes
-// A line of length N (a multiple of 4) is shared by the lanes l, l + 16, l + 32
-// and l + 48 of a wave (part q = lane / 16), N/4 values each: a quarter of the
-// registers of fft_line.  Two radix-2 stages cross the lanes: parts q and q ^ 2
-// (32 lanes apart, v_permlane32_swap as in fft_split) and parts q and q ^ 1
-// (16 lanes apart, a lane shuffle within each half-wave).
-
-// the value of lane l ^ 16
-__device__ __forceinline__ float xor16(float v) { return __shfl_xor(v, 16); }
-__device__ __forceinline__ double xor16(double v) { return __shfl_xor(v, 16); }
-
-// output position of part q: the values of part q are X[k + (N/4) quad_rev(q)]
-__host__ __device__ constexpr int quad_rev(int q) { return ((q & 1) << 1) | (q >> 1); }
-
 template <int N, int SIGN, typename C> struct fft_quad {
   static_assert(N % 4 == 0, "four-lane lines need a length divisible by 4");
   static constexpr int Q = N / 4;
   using T = decltype(C{}.x);
-  // decimation in time: part q holds x[4n + q] (n < Q); afterwards it holds
-  // X[k + Q quad_rev(q)] (k < Q)
+  // W_8^(q >> 1) (SIGN i)^(q & 1): what part q's last butterflies turn by beyond W_N^k
+  static __device__ __forceinline__ C part_turn(int q) {
+    const T r = (T)0.70710678118654752440;
+    const C w = q >= 2 ? C{r, (T)SIGN * r} : C{(T)1, (T)0};
+    return quarter_if<SIGN>(w, (q & 1) != 0);
+  }
+  // decimation in time: part q holds x[4n + q] (n < Q)
   static __device__ __forceinline__ void dit(C (&v)[Q], int q) {
     fft_line<Q, SIGN, C>::run(v);  // Y_q[k], the transform of x[4n + q]
-    // parts q, q ^ 2 hold the even and odd samples of x[2m + (q & 1)]: their
-    // length-N/2 transform, E (q & 1 = 0) or O (q & 1 = 1), at k (q < 2) and k + Q (q >= 2)
-    const T sa = q >= 2 ? (T)-1 : (T)1;
-#pragma unroll
-    for (int k = 0; k < Q; ++k) {
-      C a, b;
-      pair_vals(v[k], a, b);
-      const C t = twmul<N / 2, SIGN>(b, k);
-      v[k] = C{a.x + sa * t.x, a.y + sa * t.y};
-    }
-    // parts q, q ^ 1 hold E[m] and O[m], m = k + Q (q >> 1): X[m] = E + W^m O on
-    // the even part, X[m + N/2] = E - W^m O on the odd part
     const bool odd = (q & 1) != 0, hi = q >= 2;
-    const T sb = odd ? (T)-1 : (T)1;
+    if constexpr (Q % 2 == 0) {
+      // parts q, q ^ 2 hold the even and odd samples of x[2m + (q & 1)]: their
+      // length-N/2 transform at m = k + (Q/2)(q >> 1) and at m + Q
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
-      const C w{xor16(v[k].x), xor16(v[k].y)};
-      const C e = odd ? w : v[k], o = odd ? v[k] : w;
-      C t = twmul<N, SIGN>(o, k);
-      if (hi) t = SIGN > 0 ? C{-t.y, t.x} : C{t.y, -t.x};  // W^(k + N/4) = W^k (SIGN i)
-      v[k] = C{e.x + sb * t.x, e.y + sb * t.y};
+      for (int k = 0; k < Q / 2; ++k) {
+        C e = v[k], o = v[k + Q / 2];
+        cswap32(e, o);
+        const C t = quarter_if<SIGN>(twmul<N / 2, SIGN>(o, k), hi);
+        v[k] = cadd(e, t);
+        v[k + Q / 2] = csub(e, t);
+      }
+      // parts q, q ^ 1 hold those of the even and the odd samples, E[m] and O[m]:
+      // X[m] = E + W_N^m O and X[m + N/2] = E - W_N^m O, m now plus Q on odd parts
+      const C rho = part_turn(q);
+#pragma unroll
+      for (int k = 0; k < Q / 2; ++k) {
+        C e = v[k], o = v[k + Q / 2];
+        cswap16(e, o);
+        const C t = twmul<N, SIGN>(cmul(o, rho), k);
+        v[k] = cadd(e, t);
+        v[k + Q / 2] = csub(e, t);
+      }
+    } else {
+      const T sa = hi ? (T)-1 : (T)1, sb = odd ? (T)-1 : (T)1;
+#pragma unroll
+      for (int k = 0; k < Q; ++k) {
+        C a, b;
+        pair_vals(v[k], a, b);
+        const C t = twmul<N / 2, SIGN>(b, k);
+        v[k] = C{a.x + sa * t.x, a.y + sa * t.y};
+      }
+      // part q: X[k + Q quad_rev(q)]
+#pragma unroll
+      for (int k = 0; k < Q; ++k) {
+        C e, o;
+        pair_vals16(v[k], e, o);
+        const C t = quarter_if<SIGN>(twmul<N, SIGN>(o, k), hi);  // W^(k + N/4) = W^k (SIGN i)
+        v[k] = C{e.x + sb * t.x, e.y + sb * t.y};
+      }
     }
   }
-  // decimation in frequency, the mirror of dit: part q holds x[m + Q quad_rev(q)]
-  // (m < Q); afterwards it holds X[4k + q] (k < Q).  With chunk p = p0 + 2 p1
-  // in part q (p0 = q >> 1, p1 = q & 1) and frequency t = t0 + 2 t1,
-  // X[4k + t] = sum_m W_Q^(mk) W_N^(mt) sum_p x[m + Q p] W_4^(pt), the inner sum
-  // taken over p1 (parts q, q ^ 1) and then over p0 (parts q, q ^ 2)
+  // decimation in frequency, the mirror: afterwards part q holds X[4k + q] (k < Q)
   static __device__ __forceinline__ void dif(C (&v)[Q], int q) {
     const bool odd = (q & 1) != 0, hi = q >= 2;
-    // u = x[m + Q p0] + (-1)^t0 x[m + Q (p0 + 2)], t0 = q & 1
+    if constexpr (Q % 2 == 0) {
+      // even parts take the sums x[m] + x[m + N/2] (the even frequencies), odd
+      // parts the differences times W_N^m
+      const C rho = part_turn(q);
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
-      const C w{xor16(v[k].x), xor16(v[k].y)};
-      const C a = odd ? w : v[k], b = odd ? v[k] : w;
-      v[k] = odd ? C{a.x - b.x, a.y - b.y} : C{a.x + b.x, a.y + b.y};
-    }
-    // z = u(p0 = 0) + (-1)^t1 W_4^t0 u(p0 = 1), t1 = q >> 1
+      for (int k = 0; k < Q / 2; ++k) {
+        C s = cadd(v[k], v[k + Q / 2]);
+        C d = twmul<N, SIGN>(cmul(csub(v[k], v[k + Q / 2]), rho), k);
+        cswap16(s, d);
+        v[k] = s;
+        v[k + Q / 2] = d;
+      }
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
-      C a, b;
-      pair_vals(v[k], a, b);
-      if (odd) b = SIGN > 0 ? C{-b.y, b.x} : C{b.y, -b.x};  // W_4 = SIGN i
-      v[k] = hi ? C{a.x - b.x, a.y - b.y} : C{a.x + b.x, a.y + b.y};
-    }
-    // W_N^(m q), then the length-Q transform
+      for (int k = 0; k < Q / 2; ++k) {
+        C s = cadd(v[k], v[k + Q / 2]);
+        C d = quarter_if<SIGN>(twmul<N / 2, SIGN>(csub(v[k], v[k + Q / 2]), k), hi);
+        cswap32(s, d);
+        v[k] = s;
+        v[k + Q / 2] = d;
+      }
+    } else {
+      // part q holds x[m + Q quad_rev(q)]; with chunk p = p0 + 2 p1 in part q (p0 =
+      // q >> 1, p1 = q & 1) and frequency t = t0 + 2 t1,
+      // X[4k + t] = sum_m W_Q^(mk) W_N^(mt) sum_p x[m + Q p] W_4^(pt), the inner sum
+      // taken over p1 (parts q, q ^ 1) and then over p0 (parts q, q ^ 2)
+      // u = x[m + Q p0] + (-1)^t0 x[m + Q (p0 + 2)], t0 = q & 1
 #pragma unroll
-    for (int m = 0; m < Q; ++m) {
-      const T c = q == 0 ? (T)1 : q == 1 ? (T)kTw<N>.c[m % N] : q == 2 ? (T)kTw<N>.c[(2 * m) % N] : (T)kTw<N>.c[(3 * m) % N];
-      const T sn = q == 0 ? (T)0
-                          : (T)SIGN * (q == 1   ? (T)kTw<N>.s[m % N]
-                                       : q == 2 ? (T)kTw<N>.s[(2 * m) % N]
-                                                : (T)kTw<N>.s[(3 * m) % N]);
-      v[m] = C{v[m].x * c - v[m].y * sn, v[m].x * sn + v[m].y * c};
+      for (int k = 0; k < Q; ++k) {
+        C a, b;
+        pair_vals16(v[k], a, b);
+        v[k] = odd ? C{a.x - b.x, a.y - b.y} : C{a.x + b.x, a.y + b.y};
+      }
+      // z = u(p0 = 0) + (-1)^t1 W_4^t0 u(p0 = 1), t1 = q >> 1
+#pragma unroll
+      for (int k = 0; k < Q; ++k) {
+        C a, b;
+        pair_vals(v[k], a, b);
+        b = quarter_if<SIGN>(b, odd);  // W_4 = SIGN i
+        v[k] = hi ? C{a.x - b.x, a.y - b.y} : C{a.x + b.x, a.y + b.y};
+      }
+      // W_N^(m q), then the length-Q transform
+#pragma unroll
+      for (int m = 0; m < Q; ++m) {
+        const T c = q == 0 ? (T)1 : q == 1 ? (T)kTw<N>.c[m % N] : q == 2 ? (T)kTw<N>.c[(2 * m) % N] : (T)kTw<N>.c[(3 * m) % N];
+        const T sn = q == 0 ? (T)0
+                            : (T)SIGN * (q == 1   ? (T)kTw<N>.s[m % N]
+                                         : q == 2 ? (T)kTw<N>.s[(2 * m) % N]
+                                                  : (T)kTw<N>.s[(3 * m) % N]);
+        v[m] = C{v[m].x * c - v[m].y * sn, v[m].x * sn + v[m].y * c};
+      }
     }
     fft_line<Q, SIGN, C>::run(v);
   }

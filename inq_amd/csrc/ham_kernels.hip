@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(256) k_plane_inverse(const SphereBlock<T> *blo
   const int tid = threadIdx.x, nth = blockDim.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane / LPW, ll = lane % LPW;  // part of the line, line of the wave
-  const int qo = line_part_out<S>(q);
+  const int qo = line_out_q<N1, S>(q);
   {  // one work item per work-group: the grid is the work count
     const int wg = blockIdx.x;
     if (wg >= total) return;
@@ -155,11 +155,11 @@ __global__ void __launch_bounds__(256) k_plane_inverse(const SphereBlock<T> *blo
         v[n] = row_in_plane<N1>(y, wlo, nwin) ? lds[(y < N1 / 2 ? bA : bB) + S * n * (N2 + 1)] : C{0, 0};
       }
       line_dit<N1, +1, C, S>(v, q);
-      // v[k] is row k + qo N1/S; lanes past the last column store out of range
-      // (dropped), no branch
-      const unsigned vo = ok ? (unsigned)(((size_t)p * pstride + z + qo * (N1 / S) * N2) * sizeof(C)) : kOOB;
+      // v[k] is row line_out_j(k) + qo; lanes past the last column store out of
+      // range (dropped), no branch
+      const unsigned vo = ok ? (unsigned)(((size_t)p * pstride + z + qo * N2) * sizeof(C)) : kOOB;
 #pragma unroll
-      for (int k = 0; k < N1 / S; ++k) bstore(rt, vo, (unsigned)(k * N2 * sizeof(C)), v[k]);
+      for (int k = 0; k < N1 / S; ++k) bstore(rt, vo, (unsigned)(line_out_j<N1, S>(k) * N2 * sizeof(C)), v[k]);
     }
     __syncthreads();
   }
@@ -180,7 +180,7 @@ k_plane_forward(const SphereBlock<T> *blocks, const int *prefix, int nblocks, in
   const int tid = threadIdx.x, nth = blockDim.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane / LPW, ll = lane % LPW;  // part of the line, line of the wave
-  const int qo = line_part_out<S>(q);
+  const int qo = line_out_q<N1, S>(q);
   {  // one work item per work-group: the grid is the work count
     const int wg = blockIdx.x;
     if (wg >= total) return;
@@ -215,15 +215,17 @@ k_plane_forward(const SphereBlock<T> *blocks, const int *prefix, int nblocks, in
 #pragma unroll
       for (int n = 0; n < N1 / S; ++n) bload(rt, vo, (unsigned)(S * n * N2 * sizeof(C)), v[n]);
       line_dit<N1, -1, C, S>(v, q);
-      // v[k] is row y = k + qo N1/S (complex64: the lower lanes hold y < N1/2,
-      // the upper lanes y >= N1/2); in the window layout rows outside the window
-      // are not stored
-      const int sb = p * pstr + z + plane_row<N1>(qo * (N1 / S), wlo) * (N2 + 1);
+      // v[k] is row y = line_out_j(k) + qo; in the window layout rows outside the
+      // window are not stored.  Row y >= N1/2 stands for y - N1: with swapped
+      // stages the register decides it, else the lane
+      const int sb = p * pstr + z + (qo - wlo + 1) * (N2 + 1);
+      const int wrap = !line_swapped<N1, S>() && qo >= N1 / 2 ? N1 : 0;
       if (ok) {
 #pragma unroll
         for (int k = 0; k < N1 / S; ++k) {
-          const int y = k + qo * (N1 / S);
-          if (row_in_plane<N1>(y, wlo, nwin)) lds[sb + k * (N2 + 1)] = v[k];
+          const int j = line_out_j<N1, S>(k);
+          const int d = j - (line_swapped<N1, S>() ? (j >= N1 / 2 ? N1 : 0) : wrap);
+          if ((unsigned)(d + qo - wlo) < (unsigned)nwin) lds[sb + d * (N2 + 1)] = v[k];
         }
       }
     }
@@ -265,13 +267,13 @@ k_plane_forward(const SphereBlock<T> *blocks, const int *prefix, int nblocks, in
 template <int N> constexpr int sym_of(int i) { return i >= (N + 1) / 2 ? i - N : i; }
 
 
-// A line (i1,i2) along i0 is shared by a lane pair (lane, lane + 32): the
-// lower lane holds i0 in [0, N0/2), the upper lane [N0/2, N0) after an
-// inverse transform, and the even / odd i0 before it.  t1 is state-major
+// A line (i1,i2) along i0 is shared by a lane pair (lane, lane + 32): the even
+// and odd i0 before an inverse transform, i0 = line_out_j(k) + line_out_q(half)
+// after it.  t1 is state-major
 // [state][slot][i1][i2]; slot j holds the symmetric plane index m_lo + j.
 //
 // loads the plane slots i0 = 2n + half of the pair's line (zero outside the
-// slot range) and transforms along i0: afterwards v[k] = x[k + half N0/2]
+// slot range) and transforms along i0: afterwards v[k] = x[line_out_j(k) + line_out_q(half)]
 template <typename T, int N0>
 __device__ __forceinline__ void load_line_slots_split(const SphereBlock<T> &B, int n12, int s, int Lc, bool upper,
                                                       cplx<T> (&v)[N0 / 2]) {
@@ -352,21 +354,38 @@ template <int N0> __device__ __forceinline__ LineMask<N0> load_line_mask(const u
   return r;
 }
 
-// the lane's half of a line's point mask as bits 0..N0/2-1 (bit k: i0 = k +
-// half N0/2 holds a sphere point), and the number of points of the line
-// before that half plus the tile's points on earlier lines
-template <int N0>
-__device__ __forceinline__ unsigned long long half_mask(const LineMask<N0> &lm, bool upper, int &cnt0) {
-  constexpr int H = N0 / 2;
-  static_assert(H <= 64, "lines up to 128 points");
-  const unsigned long long lo = (unsigned long long)lm.m[0] | ((unsigned long long)lm.m[1] << 32);  // bits 0..63
-  unsigned long long hi = lm.m[2];                                                                 // bits 64..
-  if constexpr (N0 > 96) hi |= (unsigned long long)lm.m[3] << 32;
-  const unsigned long long keep = H >= 64 ? ~0ull : (1ull << (H & 63)) - 1ull;
-  const unsigned long long ml = lo & keep;
-  const unsigned long long mu = H >= 64 ? hi : ((lo >> (H & 63)) | (hi << ((64 - H) & 63))) & keep;
-  cnt0 = lm.base + (upper ? __popcll(ml) : 0);
-  return upper ? mu : ml;
+// the lane's part of a line's point mask, in the order of its values after an
+// inverse transform: NP runs of L consecutive i0 (two quarters of the line with
+// swapped stages, else one half); bit k of m[e] is value e L + k, and cnt[e] the
+// number of the tile's points before run e
+template <int N0> struct LaneMask {
+  static constexpr int NP = line_swapped<N0, 2>() ? 2 : 1, L = N0 / 2 / NP;
+  static_assert(L <= 32, "lines up to 128 points");
+  uint32_t m[NP];
+  int cnt[NP];
+};
+template <int N0> __device__ __forceinline__ LaneMask<N0> lane_mask(const LineMask<N0> &lm, bool upper, bool valid) {
+  using LM = LaneMask<N0>;
+  constexpr int L = LM::L;
+  constexpr uint32_t keep = L >= 32 ? ~0u : (1u << (L & 31)) - 1u;
+  LM r;
+  int c = lm.base;
+#pragma unroll
+  for (int e = 0; e < LM::NP; ++e) {
+    uint32_t run[2];  // the lower and the upper lane's run: the L bits from 2 e L and from (2 e + 1) L
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int b = (2 * e + h) * L, w = b >> 5, o = b & 31;
+      uint32_t x = lm.m[w] >> o;
+      if (o + L > 32 && w + 1 < mask_words<N0>()) x |= lm.m[w + 1] << ((32 - o) & 31);
+      run[h] = valid ? x & keep : 0u;
+    }
+    const int c0 = __popc(run[0]);
+    r.m[e] = upper ? run[1] : run[0];
+    r.cnt[e] = c + (upper ? c0 : 0);
+    c += c0 + __popc(run[1]);
+  }
+  return r;
 }
 
 __device__ __forceinline__ void lds_add(float *p, float v) { atomicAdd(p, v); }
@@ -454,15 +473,13 @@ __global__ void __launch_bounds__(xpass_threads<T>(N0)) k_xpass_project(const Sp
       // every value goes out: the line's sphere points to their compact
       // slots, the others (and lanes past the last line) to the trash slot
       // pts[npts + 1], so the stores need no branches
-      int cnt;
-      const unsigned long long mh = valid ? half_mask<N0>(lm, upper, cnt) : 0ull;
-      if (!valid) cnt = 0;
+      LaneMask<N0> mh = lane_mask<N0>(lm, upper, valid);
       const int trash = npts + 1;
 #pragma unroll
       for (int k = 0; k < H; ++k) {
-        const int bit = (int)((mh >> k) & 1ull);
-        pts[bit ? cnt : trash] = v[k];
-        cnt += bit;
+        const int e = k / LaneMask<N0>::L, bit = (int)((mh.m[e] >> (k % LaneMask<N0>::L)) & 1u);
+        pts[bit ? mh.cnt[e] : trash] = v[k];
+        mh.cnt[e] += bit;
       }
     }
     __syncthreads();  // entry records in LDS, sphere points staged
@@ -720,13 +737,14 @@ __global__ void __launch_bounds__(xpass_threads<T>(N0)) k_xpass_apply(const Sphe
       }
       fft_split<N0, +1, C>::dit(v, upper);
       if (B.dip) {
-        // sum |u|^2 and sum f0 |u|^2 along the lane's half line, f0 = sym(i0)/n0
+        // sum |u|^2 and sum f0 |u|^2 along the lane's part of the line, f0 = sym(i0)/n0
         double s0 = 0.0, s1 = 0.0;
         if (valid) {
 #pragma unroll
           for (int k = 0; k < H; ++k) {
             const double x2 = (double)v[k].x * (double)v[k].x + (double)v[k].y * (double)v[k].y;
-            const double f0 = upper ? (double)sym_of<N0>(k + H) / (double)N0 : (double)sym_of<N0>(k) / (double)N0;
+            const int j = line_out_j<N0, 2>(k);
+            const double f0 = upper ? (double)sym_of<N0>(j + line_out_q<N0, 2>(1)) / (double)N0 : (double)sym_of<N0>(j) / (double)N0;
             s0 += x2;
             s1 += x2 * f0;
           }
@@ -751,11 +769,11 @@ __global__ void __launch_bounds__(xpass_threads<T>(N0)) k_xpass_apply(const Sphe
     }
     __syncthreads();  // V tile, entry records and D P in LDS
     if (act) {
-      // V/N at i0 = k + half N0/2
-      const T *vrow = sv + (upper ? H * kTile : 0) + (lane & 31);
+      // V/N at i0 = line_out_j(k) + line_out_q(half)
+      const T *vrow = sv + (upper ? line_out_q<N0, 2>(1) * kTile : 0) + (lane & 31);
 #pragma unroll
       for (int k = 0; k < H; ++k) {
-        const T vv = vrow[k * kTile];
+        const T vv = vrow[line_out_j<N0, 2>(k) * kTile];
         v[k].x *= vv;
         v[k].y *= vv;
       }
@@ -808,14 +826,12 @@ __global__ void __launch_bounds__(xpass_threads<T>(N0)) k_xpass_apply(const Sphe
       if (npts > 0) {
         // every value reads: its compact point, or the zero slot pts[npts]
         // (no branches, so the reads are in flight together)
-        int cnt;
-        const unsigned long long mh = valid ? half_mask<N0>(lm, upper, cnt) : 0ull;
-        if (!valid) cnt = 0;
+        LaneMask<N0> mh = lane_mask<N0>(lm, upper, valid);
 #pragma unroll
         for (int k = 0; k < H; ++k) {
-          const int bit = (int)((mh >> k) & 1ull);
-          v[k] = cadd(v[k], pts[bit ? cnt : npts]);
-          cnt += bit;
+          const int e = k / LaneMask<N0>::L, bit = (int)((mh.m[e] >> (k % LaneMask<N0>::L)) & 1u);
+          v[k] = cadd(v[k], pts[bit ? mh.cnt[e] : npts]);
+          mh.cnt[e] += bit;
         }
       }
       fft_split<N0, -1, C>::dif(v, upper);
@@ -1347,14 +1363,16 @@ __global__ void __launch_bounds__(256) k_line_to_real(const SphereBlock<T> *bloc
     if (B.rs_layout == 0) {
       const unsigned pl = (unsigned)(n12 * sizeof(C));
       const auto rs = make_rsrc(B.rs + (size_t)s * N0 * n12, (unsigned)N0 * pl);
-      const unsigned vo = L < n12 ? (unsigned)(L * sizeof(C)) + (upper ? (unsigned)H * pl : 0u) : kOOB;
+      const unsigned vo = L < n12 ? (unsigned)(L * sizeof(C)) + (upper ? (unsigned)line_out_q<N0, 2>(1) * pl : 0u) : kOOB;
 #pragma unroll
-      for (int k = 0; k < H; ++k) bstore(rs, vo, (unsigned)k * pl, C{v[k].x * scale, v[k].y * scale});
+      for (int k = 0; k < H; ++k)
+        bstore(rs, vo, (unsigned)line_out_j<N0, 2>(k) * pl, C{v[k].x * scale, v[k].y * scale});
     } else if (L < n12) {
       {
-        GAS C *out = gw(B.rs) + ((size_t)L + (upper ? (size_t)H * n12 : 0)) * B.nst + s;
+        GAS C *out = gw(B.rs) + ((size_t)L + (upper ? (size_t)line_out_q<N0, 2>(1) * n12 : 0)) * B.nst + s;
 #pragma unroll
-        for (int k = 0; k < H; ++k) out[(size_t)k * n12 * B.nst] = C{v[k].x * scale, v[k].y * scale};
+        for (int k = 0; k < H; ++k)
+          out[(size_t)line_out_j<N0, 2>(k) * n12 * B.nst] = C{v[k].x * scale, v[k].y * scale};
       }
     }
   }
@@ -1386,13 +1404,13 @@ __global__ void __launch_bounds__(256) k_line_from_real(const SphereBlock<T> *bl
     if (B.rs_layout == 0) {
       const unsigned pl = (unsigned)(n12 * sizeof(C));
       const auto rs = make_rsrc(B.rs + (size_t)s * N0 * n12, (unsigned)N0 * pl);
-      const unsigned vo = (unsigned)(Lc * sizeof(C)) + (upper ? (unsigned)H * pl : 0u);
+      const unsigned vo = (unsigned)(Lc * sizeof(C)) + (upper ? (unsigned)line_out_q<N0, 2>(1) * pl : 0u);
 #pragma unroll
-      for (int k = 0; k < H; ++k) bload(rs, vo, (unsigned)k * pl, v[k]);
+      for (int k = 0; k < H; ++k) bload(rs, vo, (unsigned)line_out_j<N0, 2>(k) * pl, v[k]);
     } else {
-      const GAS C *in = gp(B.rs) + ((size_t)Lc + (upper ? (size_t)H * n12 : 0)) * B.nst + s;
+      const GAS C *in = gp(B.rs) + ((size_t)Lc + (upper ? (size_t)line_out_q<N0, 2>(1) * n12 : 0)) * B.nst + s;
 #pragma unroll
-      for (int k = 0; k < H; ++k) v[k] = in[(size_t)k * n12 * B.nst];
+      for (int k = 0; k < H; ++k) v[k] = in[(size_t)line_out_j<N0, 2>(k) * n12 * B.nst];
     }
     fft_split<N0, -1, C>::dif(v, upper);
     store_line_slots_split<T, N0>(B, n12, s, L, upper, L < n12, v);

@@ -124,20 +124,18 @@ __device__ __forceinline__ void plane_row_split(C *row, bool upper, bool ok) {
   __builtin_amdgcn_wave_barrier();
   if (ok) {
 #pragma unroll
-    for (int k = 0; k < H; ++k) row[k + (upper ? H : 0)] = v[k];
+    for (int k = 0; k < H; ++k) row[line_out_j<N, 2>(k) + line_out_q<N, 2>(upper ? 1 : 0)] = v[k];
   }
 }
 
 // the transform of a line split over S lanes (part q of the line): input
-// x[S n + q], output X[k + (N/S) line_part_out<S>(q)]
+// x[S n + q], output order line_out_j + line_out_q (fft_reg.hpp)
 template <int N, int SIGN, typename C, int S>
 __device__ __forceinline__ void line_dit(C (&v)[N / S], int q) {
   if constexpr (S == 2) fft_split<N, SIGN, C>::dit(v, q != 0);
   else fft_quad<N, SIGN, C>::dit(v, q);
 }
-template <int S> __device__ __forceinline__ int line_part_out(int q) { return S == 2 ? q : quad_rev(q); }
-// the mirror: input X[k + (N/S) line_part_out<S>(q)] (line_dit's output order),
-// output x[S k + q] (line_dit's input order)
+// the mirror: input in line_dit's output order, output x[S k + q] (line_dit's input order)
 template <int N, int SIGN, typename C, int S>
 __device__ __forceinline__ void line_dif(C (&v)[N / S], int q) {
   if constexpr (S == 2) fft_split<N, SIGN, C>::dif(v, q != 0);
@@ -158,9 +156,9 @@ __device__ __forceinline__ void plane_row_lanes(C *row, int q, bool ok) {
     line_dit<N, SIGN, C, S>(v, q);
     __builtin_amdgcn_wave_barrier();
     if (ok) {
-      const int o = M * line_part_out<S>(q);
+      const int o = line_out_q<N, S>(q);
 #pragma unroll
-      for (int k = 0; k < M; ++k) row[k + o] = v[k];
+      for (int k = 0; k < M; ++k) row[line_out_j<N, S>(k) + o] = v[k];
     }
   }
 }

@@ -115,16 +115,16 @@ __global__ void __launch_bounds__(256) k_plane_cols(const SphereBlock<T> *blocks
     const bool ok = li < np * n2;
     const int lc = ok ? li : np * n2 - 1;
     const int p = div_rcp(lc, n2, rn2), z = lc - p * n2;
-    // rows y = 2n + half in, rows y = k + half N1/2 out
+    // rows y = 2n + half in, rows y = line_out_j(k) + line_out_q(half) out
     const unsigned vi = (unsigned)(((size_t)p * pstride + z + half * n2) * sizeof(C));
     C v[N1 / 2];
 #pragma unroll
     for (int n = 0; n < N1 / 2; ++n) bload(rt, vi, (unsigned)(2 * n * n2 * (int)sizeof(C)), v[n]);
     fft_split<N1, SIGN, C>::dit(v, upper);
     // lanes past the last column store out of range (dropped)
-    const unsigned vo = ok ? (unsigned)(((size_t)p * pstride + z + half * (N1 / 2) * n2) * sizeof(C)) : kOOB;
+    const unsigned vo = ok ? (unsigned)(((size_t)p * pstride + z + line_out_q<N1, 2>(half) * n2) * sizeof(C)) : kOOB;
 #pragma unroll
-    for (int k = 0; k < N1 / 2; ++k) bstore(rt, vo, (unsigned)(k * n2 * (int)sizeof(C)), v[k]);
+    for (int k = 0; k < N1 / 2; ++k) bstore(rt, vo, (unsigned)(line_out_j<N1, 2>(k) * n2 * (int)sizeof(C)), v[k]);
   }
 }
 
