@@ -887,6 +887,11 @@ int inqx_invert_triangular(inqx_ctx ctx, int n, const void *L, void *Linv) {
   API_END(ctx)
 }
 
+// phi <- phi Linv^H (Linv lower triangular) in place
+static void rotate_lower(inqx_ctx ctx, int precision, int n, long npw, const double *Linv, void *phi) {
+  launch_rotate(ctx->c, precision, n, n, npw, Linv, 0, 1.0, 0.0, phi, phi, 0.0, 0.0, ctx->c.ws_ops, true);
+}
+
 // phi <- M phi through a temporary (rows of the output depend on all rows of phi)
 static void rotate_inplace(inqx_ctx ctx, int precision, int n, long npw, const double *R, int mode, void *phi) {
   const size_t cs = precision == INQX_FP64 ? 16 : 8;
@@ -921,7 +926,7 @@ static void orthogonalize_impl(inqx_ctx ctx, int precision, int n, long npw, dou
   const int info = cholesky_impl(ctx, n, S);
   INQX_CHECK(info == 0, INQX_ERR_NOT_PD, "orthogonalize: overlap not positive definite (minor " + std::to_string(info) + ")");
   launch_trinv(ctx->c, n, S, X);
-  rotate_inplace(ctx, precision, n, npw, X, 0, phi);  // phi <- phi Linv^H
+  rotate_lower(ctx, precision, n, npw, X, phi);  // phi <- phi Linv^H
 }
 
 int inqx_orthogonalize(inqx_ctx ctx, int precision, int n, long npw, double vol_el, void *phi) {
@@ -1476,7 +1481,7 @@ static double ace_build_impl(inqx_ham h, Basis &B, int nst, int precision, const
   const int info = cholesky_impl(ctx, nst, S);
   INQX_CHECK(info == 0, INQX_ERR_NOT_PD, "ACE: exchange matrix not positive definite (minor " + std::to_string(info) + ")");
   launch_trinv(ctx->c, nst, S, X);
-  rotate_inplace(ctx, precision, nst, npw, X, 0, xi);  // xi <- W L^{-H} (rotate_trs)
+  rotate_lower(ctx, precision, nst, npw, X, xi);  // xi <- W L^{-H} (rotate_trs)
   return en;
 }
 

@@ -347,9 +347,11 @@ void launch_rect_forward(Ctx &cx, const SphereBlock<T> *blk, const int *pref, in
 void launch_overlap(Ctx &cx, int prec, int n1, int n2, long K, const void *A, const void *B, double vol, double *S,
                     DevMem &partial);
 // Out[nr][K] = M C (+ beta Out), C [nc][K]; M from R by mode (0: conj(R), 2: R, both square;
-// 1: alpha R^T with R [nc][nr])
+// 1: alpha R^T with R [nc][nr]).  lower: M is lower triangular, and Out may be C.  info: a
+// device status word; the product is skipped where it is not 0 when the kernel runs
 void launch_rotate(Ctx &cx, int prec, int nr, int nc, long K, const double *R, int mode, double ar, double ai,
-                   const void *Cm, void *Out, double br, double bi, DevMem &ops);
+                   const void *Cm, void *Out, double br, double bi, DevMem &ops, bool lower = false,
+                   const int *info = nullptr);
 void launch_cholesky(Ctx &cx, int n, double *S, int *info);
 void launch_trinv(Ctx &cx, int n, const double *L, double *X);
 void launch_stream_copy(Ctx &cx, const void *src, void *dst, size_t bytes);

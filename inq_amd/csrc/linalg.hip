@@ -3,27 +3,25 @@
 //
 //   overlap   S = vol * A^H B   (operations::overlap, src/operations/overlap.hpp:26-41)
 //             A [n1][K], B [n2][K] complex; split-K over K with
-//             v_mfma_{f32,f64}_16x16x4 on the interleaved (re, im) storage read
-//             as a real K' = 2K contraction:
-//               Re S = sum_k' A'[i][k'] B'[j][k'],
-//               Im S = sum_k' A'[i][k'] B''[j][k'],  B''[j][k'] = (+/-) B'[j][k' ^ 1]
-//             Partial tiles are reduced in FP64 in a fixed order.
+//             matrix-core products of the complex values' real and imaginary parts;
+//             partial tiles are reduced in FP64 in a fixed order.
 //   rotate    Out = M C (+ beta Out): C [n][K] complex, M [n][n] complex
-//             (operations::rotate, src/operations/rotate.hpp:26-156), MFMA with
-//             the real operands A' = [Mr, -Mi], A'' = [Mi, Mr] interleaved along j.
+//             (operations::rotate, src/operations/rotate.hpp:26-156) on the matrix
+//             cores; half of it, in place, for a triangular M.
 //   cholesky  FP64 lower Cholesky S = L L^H, upper zeroed (matrix::cholesky,
 //             src/matrix/cholesky.hpp:28-100), blocked in 32-wide panels.
 //   trinv     FP64 inverse of a lower-triangular matrix (matrix::invert_triangular,
 //             src/matrix/invert_triangular.hpp:20-50), blocked by 32x32 block rows.
 //
-// MFMA 16x16x4 lane layout (CDNA4): lane l supplies A[l%16][l/16] and
-// B[l/16][l%16] and receives column l%16 of D in its four accumulators; the
-// accumulator-to-row map differs between the f32 and f64 forms (mfma_t::row),
-// and tests/test_gpu_linalg.py checks both against numpy.
+// MFMA lane layouts (CDNA4), checked against numpy by tests/test_gpu_linalg.py: 16x16x4
+// lane l supplies A[l%16][l/16] and B[l/16][l%16] and receives column l%16 of D in
+// its four accumulators; the accumulator-to-row map differs between the f32 and f64
+// forms (mm_t::row).
 #include "internal.hpp"
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #if defined(__HIP_DEVICE_COMPILE__)
 #define GAS __attribute__((address_space(1)))
@@ -44,162 +42,332 @@ typedef double doublex4 __attribute__((ext_vector_type(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef double doublex2 __attribute__((ext_vector_type(2)));
 
-// row of the 16x16 output tile held in accumulator r of a lane (column = lane % 16)
 template <typename T> struct mfma_t;
 template <> struct mfma_t<float> {
-  using acc = floatx4;
   using pair = floatx2;
-  using v16 = floatx4;
+};
+template <> struct mfma_t<double> {
+  using pair = doublex2;
+};
+template <typename T> struct Vec16;  // 16 bytes of values
+template <> struct Vec16<float> {
+  typedef floatx4 type;
+};
+template <> struct Vec16<double> {
+  typedef doublex2 type;
+};
+
+// ------------------------------------------------------------------------ matrix-core blocks
+// Both contractions run 64 x 64 output tiles on four waves, each wave a 32 x 32
+// complex block of 2 x 2 16x16x4 products (eight independent accumulators per
+// wave keep the matrix cores at 153 of 157 TFLOP/s FP32 and 67 TFLOP/s FP64 in a
+// register-only loop; two 32x32x2 accumulators reach 140).  A stage
+// is kStage bytes (128) of complex values along the contraction per row.  Any
+// order of the contraction index is the same sum, so a lane takes contiguous
+// complex values of its row (16-byte LDS reads) and uses real and imaginary
+// parts in separate steps: no operand is stored twice or sign-flipped in memory.
+constexpr int kMT = 64;                          // output tile edge
+constexpr int kStageBytes = 128;                 // of one row, per stage
+constexpr int kRowStride = kStageBytes + 16;     // LDS row stride: 16 rows of 16-byte reads cover all banks
+template <typename T> constexpr int kStage = kStageBytes / (2 * (int)sizeof(T));  // complex values: 16 or 8
+
+// 16 bytes of complex values, and the same at the alignment of one complex value
+// (rows of an odd count of complex64 values start at 8 bytes)
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+template <typename T> struct chunk16;
+template <> struct chunk16<float> {
+  typedef uintx4 type __attribute__((aligned(8)));
+};
+template <> struct chunk16<double> {
+  typedef uintx4 type;
+};
+template <typename T> __device__ __forceinline__ uintx4 load16(const GAS cplx<T> *p) {
+  return *(const GAS typename chunk16<T>::type *)p;
+}
+// the first m complex values at p, zero after them
+template <typename T> __device__ __forceinline__ uintx4 load16_part(const GAS cplx<T> *p, long m) {
+  constexpr int W = (int)sizeof(cplx<T>) / 4;
+  uintx4 v{};
+#pragma unroll
+  for (int q = 0; q < 4 / W; ++q)
+    if (q < m)
+#pragma unroll
+      for (int i = 0; i < W; ++i) v[W * q + i] = ((const GAS unsigned *)(p + q))[i];
+  return v;
+}
+
+template <typename T> struct mm_t;
+template <> struct mm_t<float> {
+  typedef floatx4 acc;
   static __device__ __forceinline__ acc run(float a, float b, acc c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+  static __device__ __forceinline__ int row(int lane, int i) { return 4 * (lane >> 4) + i; }
 };
-template <> struct mfma_t<double> {
-  using acc = doublex4;
-  using pair = doublex2;
-  using v16 = doublex2;
+template <> struct mm_t<double> {
+  typedef doublex4 acc;
   static __device__ __forceinline__ acc run(double a, double b, acc c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
+  static __device__ __forceinline__ int row(int lane, int i) { return (lane >> 4) + 4 * i; }
 };
 
-// ------------------------------------------------------------------------ overlap
-constexpr int kOvTile = 64;   // output tile edge per work-group
-constexpr int kOvKC = 32;     // real K per LDS stage
-constexpr int kOvChunkMax = 2048;  // real K per work-group (split K), upper bound
-constexpr int kOvChunkMin = 256;   // lower bound when few output tiles call for more chunks
-constexpr int kOvGridTarget = 1024;  // work-groups that keep every CU busy with 4 of them
-
-constexpr size_t kOvPartialMax = size_t(1) << 30;  // bytes of partial tiles at most
-
-// real K per work-group: the full 2048 when the output has enough tiles, else
-// shorter chunks (a multiple of the LDS stage) so that the grid fills the chip;
-// longer ones when the partial tiles (nchunk x tiles x 64 x 64 complex) would
-// pass kOvPartialMax (thousands of states over a long K)
-static long overlap_chunk(long K2, int tiles, size_t es) {
-  const long want = std::max<long>(1, (kOvGridTarget + tiles - 1) / tiles);
-  long c = (K2 + want - 1) / want;
-  c = std::min<long>(kOvChunkMax, std::max<long>(kOvChunkMin, c));
-  const size_t tile_bytes = es * (size_t)tiles * kOvTile * kOvTile * 2;
-  const long nchunk_max = std::max<long>(1, (long)(kOvPartialMax / tile_bytes));
-  c = std::max<long>(c, (K2 + nchunk_max - 1) / nchunk_max);
-  return (c + kOvKC - 1) / kOvKC * kOvKC;
-}
-
-// partial[chunk][tile_i][tile_j] holds a 64x64 complex tile in T.  Each stage
-// loads (re, im) pairs (rows start at even real offsets, so pairs are aligned),
-// and the next stage's pairs are loaded into registers while the matrix cores
-// work on the current one.
-template <typename T>
-__global__ void __launch_bounds__(256) k_overlap_partial(const T *A, const T *B, int n1, int n2, long K2,
-                                                         int tiles_i, int tiles_j, int kchunk, T *partial) {
-  using M = mfma_t<T>;
-  using P2 = typename M::pair;
-  __shared__ T At[kOvTile][kOvKC + 1];
-  __shared__ T Bt[kOvTile][kOvKC + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int tj = blockIdx.x % tiles_j, ti = (blockIdx.x / tiles_j) % tiles_i, chunk = blockIdx.x / (tiles_j * tiles_i);
-  const long k_begin = (long)chunk * kchunk;
-  const long k_end = min(k_begin + kchunk, K2);
-  const int i0 = ti * kOvTile, j0 = tj * kOvTile;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;  // wave sub-tile 32x32
-  typename M::acc re[2][2], im[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      re[a][b] = typename M::acc{0, 0, 0, 0};
-      im[a][b] = typename M::acc{0, 0, 0, 0};
-    }
-  const GAS T *Ag = lgp(A), *Bg = lgp(B);
-  // stage = 64 rows x 32 real k' of A and of B = 64 x 16 pairs each, 4 pairs per lane;
-  // K2 and kchunk are even, so k < k_end implies k + 1 < k_end
-  constexpr int kPairs = kOvTile * kOvKC / 2 / 256;
-  P2 ra[kPairs], rb[kPairs];
-  auto load_stage = [&](long kb) {
-#pragma unroll
-    for (int q = 0; q < kPairs; ++q) {
-      const int e = tid + 256 * q, r = e >> 4;
-      const long k = kb + 2 * (e & 15);
-      const int ia = i0 + r, jb = j0 + r;
-      ra[q] = (ia < n1 && k < k_end) ? *(const GAS P2 *)(Ag + (long)ia * K2 + k) : P2{0, 0};
-      rb[q] = (jb < n2 && k < k_end) ? *(const GAS P2 *)(Bg + (long)jb * K2 + k) : P2{0, 0};
-    }
+// the wave's 32 x 32 complex block as 2 x 2 sub-tiles; value r = 8 x + 4 y + i is
+// accumulator i of sub-tile (x, y), at row(lane, r), col(lane, r)
+template <typename T> struct Block {
+  using M = mm_t<T>;
+  static constexpr int kAcc = 16;
+  static constexpr int CL = kStage<T> / 4;           // complex values per lane and stage: 4 or 2
+  static constexpr int W = 2 * (int)sizeof(T) * CL;  // their bytes: 32
+  typename M::acc re[2][2] = {}, im[2][2] = {};
+  struct Frag {
+    T v[2][2 * CL];
   };
-  load_stage(k_begin);
-  for (long kb = k_begin; kb < k_end; kb += kOvKC) {
+  static __device__ __forceinline__ int row(int lane, int r) { return 16 * (r >> 3) + M::row(lane, r & 3); }
+  static __device__ __forceinline__ int col(int lane, int r) { return 16 * ((r >> 2) & 1) + (lane & 15); }
+  __device__ __forceinline__ T vr(int r) const { return re[r >> 3][(r >> 2) & 1][r & 3]; }
+  __device__ __forceinline__ T vi(int r) const { return im[r >> 3][(r >> 2) & 1][r & 3]; }
+  // rows of an LDS tile [row][kStage complex]
+  static __device__ __forceinline__ Frag rows(const unsigned char *tile, int lane) {
+    using V = typename Vec16<T>::type;
+    constexpr int PV = 16 / (int)sizeof(T);
+    Frag f;
 #pragma unroll
-    for (int q = 0; q < kPairs; ++q) {
-      const int e = tid + 256 * q, r = e >> 4, c = 2 * (e & 15);
-      At[r][c] = ra[q].x;
-      At[r][c + 1] = ra[q].y;
-      Bt[r][c] = rb[q].x;
-      Bt[r][c + 1] = rb[q].y;
-    }
-    __syncthreads();
-    if (kb + kOvKC < k_end) load_stage(kb + kOvKC);
+    for (int x = 0; x < 2; ++x) {
+      const V *p = reinterpret_cast<const V *>(tile + (16 * x + (lane & 15)) * kRowStride + (lane >> 4) * W);
 #pragma unroll
-    for (int ks = 0; ks < kOvKC; ks += 4) {
-      const int kk = ks + (lane >> 4);
-      const T sgn = (kk & 1) ? (T)-1 : (T)1;
-      T a[2], bp[2], bq[2];
+      for (int u = 0; u < W / 16; ++u) {
+        const V q = p[u];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        a[t] = At[wr + 16 * t + (lane & 15)][kk];
-        bp[t] = Bt[wc + 16 * t + (lane & 15)][kk];
-        bq[t] = sgn * Bt[wc + 16 * t + (lane & 15)][kk ^ 1];
+        for (int i = 0; i < PV; ++i) f.v[x][PV * u + i] = q[i];
       }
+    }
+    return f;
+  }
+  // columns c0 .. c0 + 31 of an LDS tile [kStage][64 complex]
+  static __device__ __forceinline__ Frag cols(const unsigned char *tile, int c0, int lane) {
+    using P = typename mfma_t<T>::pair;
+    Frag f;
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const P *p = reinterpret_cast<const P *>(tile) + (lane >> 4) * CL * kMT + c0 + 16 * x + (lane & 15);
+#pragma unroll
+      for (int u = 0; u < CL; ++u) {
+        const P q = p[u * kMT];
+        f.v[x][2 * u] = q.x;
+        f.v[x][2 * u + 1] = q.y;
+      }
+    }
+    return f;
+  }
+  // += conj(a) b over the stage (CONJ) or a b; eight independent sums follow one another
+  template <bool CONJ> __device__ __forceinline__ void mac(const Frag &a, const Frag &b) {
+#pragma unroll
+    for (int u = 0; u < CL; ++u) {
 #pragma unroll
       for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) {
-          re[x][y] = M::run(a[x], bp[y], re[x][y]);
-          im[x][y] = M::run(a[x], bq[y], im[x][y]);
+          re[x][y] = M::run(a.v[x][2 * u], b.v[y][2 * u], re[x][y]);
+          im[x][y] = M::run(a.v[x][2 * u], b.v[y][2 * u + 1], im[x][y]);
+        }
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          const T ai = a.v[x][2 * u + 1];
+          re[x][y] = M::run(CONJ ? ai : -ai, b.v[y][2 * u + 1], re[x][y]);
+          im[x][y] = M::run(CONJ ? -ai : ai, b.v[y][2 * u], im[x][y]);
         }
     }
+  }
+};
+
+// Work-groups are dealt round-robin to the 8 XCDs; renumber so that each XCD runs
+// a contiguous range, whose neighbours read the same rows through the same L2.
+__device__ __forceinline__ int xcd_logical(int b, int G) {
+  const int xq = G / 8, xr = G % 8, x = b % 8;
+  return (x < xr ? x * (xq + 1) : xr * (xq + 1) + (x - xr) * xq) + b / 8;
+}
+
+// ------------------------------------------------------------------------ overlap
+// S = vol A^H B split over K: a work-group sums one chunk of K for one 64 x 64
+// tile.  The grid is sized to run as one round of equal work-groups (up to four
+// per CU), so none waits for a last partial round.  FP32 products accumulate over
+// at most kOvRun complex values before they are added in FP64 (WIDE: chunks
+// longer than that keep FP64 sums in registers and write FP64 partial tiles).
+// HERM (A and B the same states): only the tiles on and below the diagonal.
+// Measured, before -> now: 432 states x 228487 with themselves, complex64, 3.38 ->
+// 1.87 ms (112 TFLOP/s over the products done); 128 x 67691 93 -> 67 us complex64,
+// two different blocks of it in complex128 176 -> 166 us (53 of 67 TFLOP/s).
+constexpr int kOvRun = 1024;        // complex values per FP32 accumulation
+constexpr int kOvChunkMin = 128;    // complex values per work-group at least
+constexpr int kOvChunkGood = 256;   // enough stages to hide a work-group's start and end
+
+struct OvPlan {
+  int tiles_i, tiles_j, tiles;  // tiles: all, or those on and below the diagonal
+  int nchunk;
+  long chunk;  // complex values, a multiple of the stage
+};
+// work-groups per CU in the one round: what the registers hold
+static int overlap_slots(bool f64, bool wide) { return f64 || wide ? 3 : 4; }
+static OvPlan overlap_plan(int n1, int n2, long K, bool herm, int cus, bool f64) {
+  OvPlan p;
+  p.tiles_i = (n1 + kMT - 1) / kMT;
+  p.tiles_j = (n2 + kMT - 1) / kMT;
+  p.tiles = herm ? p.tiles_i * (p.tiles_i + 1) / 2 : p.tiles_i * p.tiles_j;
+  const int stage = f64 ? kStage<double> : kStage<float>;
+  for (int m = 4; m >= 1; --m) {
+    const long want = std::max<long>(1, (long)m * cus / p.tiles);
+    if (m > overlap_slots(f64, K > want * kOvRun)) continue;
+    long c = std::max<long>((K + want - 1) / want, kOvChunkMin);
+    p.chunk = (c + stage - 1) / stage * stage;
+    if (p.chunk >= kOvChunkGood) break;
+  }
+  p.nchunk = (int)((K + p.chunk - 1) / p.chunk);
+  return p;
+}
+
+// tile t of the list on and below the diagonal
+__device__ __forceinline__ void lower_tile(int t, int &ti, int &tj) {
+  int i = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+  while ((i + 1) * (i + 2) / 2 <= t) ++i;
+  while (i * (i + 1) / 2 > t) --i;
+  ti = i;
+  tj = t - i * (i + 1) / 2;
+}
+
+template <typename T, typename P, bool WIDE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WIDE || sizeof(T) == 8 ? 3 : 4)))
+k_overlap_partial(const T *A, const T *B, int n1, int n2, long K, int tiles,
+                                                         int tiles_j, int herm, long chunk, P *partial) {
+  constexpr int KC = kStage<T>, CV = 16 / (2 * (int)sizeof(T)), kTile = kMT * kRowStride;
+  __shared__ __align__(16) unsigned char sm[2][2][kTile];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int id = xcd_logical(blockIdx.x, gridDim.x);
+  const int c = id / tiles, t = id - c * tiles;
+  int ti, tj;
+  if (herm) {
+    lower_tile(t, ti, tj);
+  } else {
+    ti = t / tiles_j;
+    tj = t - ti * tiles_j;
+  }
+  const int i0 = ti * kMT, j0 = tj * kMT, wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  const long k0 = (long)c * chunk, k1 = min(k0 + chunk, K);
+  // this thread's 16 bytes of rows lr and lr + 32 of both tiles, chunk lc (rows past
+  // the last state repeat it: their outputs are not used).  The pipelined loop runs
+  // over whole stages with plain loads; the last chunk's odd stage follows it
+  const int lr = tid >> 3, lc = tid & 7;
+  const GAS cplx<T> *pa[2], *pb[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    pa[h] = (const GAS cplx<T> *)lgp(A) + (long)min(i0 + 32 * h + lr, n1 - 1) * K + lc * CV;
+    pb[h] = (const GAS cplx<T> *)lgp(B) + (long)min(j0 + 32 * h + lr, n2 - 1) * K + lc * CV;
+  }
+  uintx4 ra[2], rb[2];
+  auto load = [&](long k) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      ra[h] = load16<T>(pa[h] + k);
+      rb[h] = load16<T>(pb[h] + k);
+    }
+  };
+  auto store = [&](int b) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      *reinterpret_cast<uintx4 *>(&sm[b][0][(32 * h + lr) * kRowStride + 16 * lc]) = ra[h];
+      *reinterpret_cast<uintx4 *>(&sm[b][1][(32 * h + lr) * kRowStride + 16 * lc]) = rb[h];
+    }
+  };
+  Block<T> acc;
+  double wre[WIDE ? 16 : 1] = {}, wim[WIDE ? 16 : 1] = {};
+  auto mac = [&](int b) {
+    const auto a = Block<T>::rows(&sm[b][0][wr * kRowStride], lane);
+    const auto c = Block<T>::rows(&sm[b][1][wc * kRowStride], lane);
+    acc.template mac<true>(a, c);
+  };
+  auto widen = [&]() {
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        wre[r] += (double)acc.vr(r);
+        wim[r] += (double)acc.vi(r);
+      }
+      acc = Block<T>();
+    }
+  };
+  const long kw = k0 + (k1 - k0) / KC * KC;  // end of the whole stages
+  int buf = 0, run = 0;
+  if (k0 < kw) {
+    load(k0);
+    store(0);
     __syncthreads();
   }
-  // write the 64x64 complex partial tile: row i = wr + 16x + 4(l/16) + r, col j = wc + 16y + l%16
-  GAS T *P = lgw(partial) + ((long)blockIdx.x) * kOvTile * kOvTile * 2;
+  for (long k = k0; k < kw; k += KC) {
+    const bool more = k + KC < kw;
+    if (more) load(k + KC);
+    mac(buf);
+    if (WIDE && (run += KC) >= kOvRun) {
+      run = 0;
+      widen();
+    }
+    buf ^= 1;
+    if (more) store(buf);
+    __syncthreads();
+  }
+  if (kw < k1) {
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+    for (int h = 0; h < 2; ++h) {
+      ra[h] = load16_part<T>(pa[h] + kw, k1 - kw - lc * CV);
+      rb[h] = load16_part<T>(pb[h] + kw, k1 - kw - lc * CV);
+    }
+    store(buf);
+    __syncthreads();
+    mac(buf);
+  }
+  widen();
+  GAS P *out = lgw(partial) + (long)id * kMT * kMT * 2;
 #pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = wr + 16 * x + M::row(lane, r), j = wc + 16 * y + (lane & 15);
-        P[(i * kOvTile + j) * 2 + 0] = re[x][y][r];
-        P[(i * kOvTile + j) * 2 + 1] = im[x][y][r];
-      }
+  for (int r = 0; r < Block<T>::kAcc; ++r) {
+    const int e = (wr + Block<T>::row(lane, r)) * kMT + wc + Block<T>::col(lane, r);
+    out[2 * e] = WIDE ? (P)wre[WIDE ? r : 0] : (P)acc.vr(r);
+    out[2 * e + 1] = WIDE ? (P)wim[WIDE ? r : 0] : (P)acc.vi(r);
+  }
 }
 
 // S[i][j] = vol * sum_chunks partial in FP64, in a fixed order: work-group = one
 // 64-wide row of one output tile; lane group g (of 4) sums chunks g, g+4, g+8, ...
-// in ascending order, and the four group sums are added g = 0..3.
+// in ascending order, and the four group sums are added g = 0..3.  herm: the
+// tiles below the diagonal also give S[j][i], the conjugate.
 constexpr int kOvRedGroups = 4;
-template <typename T>
-__global__ void __launch_bounds__(256) k_overlap_reduce(const T *partial, int n1, int n2, int tiles_i, int tiles_j,
-                                                        int nchunk, double vol, double *S) {
-  using P2 = typename mfma_t<T>::pair;
-  __shared__ double red[kOvRedGroups][kOvTile][2];
-  const int jj = threadIdx.x & (kOvTile - 1), g = threadIdx.x >> 6;
-  const int ii = blockIdx.x % kOvTile, tile = blockIdx.x / kOvTile;
-  const int tj = tile % tiles_j, ti = tile / tiles_j;
-  const long tile_stride = (long)tiles_i * tiles_j * kOvTile * kOvTile;  // P2 per chunk
-  const GAS P2 *P = (const GAS P2 *)lgp(partial) + (long)tile * kOvTile * kOvTile + ii * kOvTile + jj;
+template <typename P>
+__global__ void __launch_bounds__(256) k_overlap_reduce(const P *partial, int n1, int n2, int tiles, int tiles_j,
+                                                        int herm, int nchunk, double vol, double *S) {
+  using P2 = typename mfma_t<P>::pair;
+  __shared__ double red[kOvRedGroups][kMT][2];
+  const int jj = threadIdx.x & (kMT - 1), g = threadIdx.x >> 6;
+  const int ii = blockIdx.x % kMT, tile = blockIdx.x / kMT;
+  int ti, tj;
+  if (herm) {
+    lower_tile(tile, ti, tj);
+  } else {
+    ti = tile / tiles_j;
+    tj = tile - ti * tiles_j;
+  }
+  const long tile_stride = (long)tiles * kMT * kMT;  // P2 per chunk
+  const GAS P2 *p = (const GAS P2 *)lgp(partial) + (long)tile * kMT * kMT + ii * kMT + jj;
   double sr = 0.0, si = 0.0;
 #pragma unroll 8
   for (int c = g; c < nchunk; c += kOvRedGroups) {
-    const P2 v = P[(long)c * tile_stride];
+    const P2 v = p[(long)c * tile_stride];
     sr += (double)v.x;
     si += (double)v.y;
   }
   red[g][jj][0] = sr;
   red[g][jj][1] = si;
   __syncthreads();
-  const int i = ti * kOvTile + ii, j = tj * kOvTile + jj;
+  const int i = ti * kMT + ii, j = tj * kMT + jj;
   if (g == 0 && i < n1 && j < n2) {
     double tr = red[0][jj][0], tim = red[0][jj][1];
 #pragma unroll
@@ -210,133 +378,120 @@ __global__ void __launch_bounds__(256) k_overlap_reduce(const T *partial, int n1
     GAS double *Sg = lgw(S);
     Sg[2 * ((long)i * n2 + j)] = vol * tr;
     Sg[2 * ((long)i * n2 + j) + 1] = vol * tim;
+    if (herm && ti != tj) {
+      Sg[2 * ((long)j * n2 + i)] = vol * tr;
+      Sg[2 * ((long)j * n2 + i) + 1] = -vol * tim;
+    }
   }
 }
 
 // ------------------------------------------------------------------------ rotate
-// operand matrices Ap = [Mr, -Mi], Aq = [Mi, Mr] interleaved along j: [nr_pad][ld] in T,
-// rows padded to a multiple of 64 and ld = 2 nc rounded up to 32, the padding zero
+// operand matrix M [nr_pad][ld] complex in T, rows padded to a multiple of 64 and
+// ld to a multiple of 16, the padding zero
 // mode 0: M = conj(R) (Phi <- Phi R^H);  mode 1: M = alpha R^T (5-argument rotate,
 // R is [nc][nr]); mode 2: M = R
 template <typename T>
-__global__ void k_rot_prep(const double *R, int nr, int nc, int mode, double ar, double ai, int nr_pad, int ld, T *Ap,
-                           T *Aq) {
+__global__ void k_rot_prep(const double *R, int nr, int nc, int mode, double ar, double ai, int nr_pad, int ld,
+                           cplx<T> *M) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int half = ld / 2;
-  if (idx >= (long)nr_pad * half) return;
-  const int i = (int)(idx / half), j = (int)(idx - (long)i * half);
+  if (idx >= (long)nr_pad * ld) return;
+  const int i = (int)(idx / ld), j = (int)(idx - (long)i * ld);
   double mr = 0.0, mi = 0.0;
   if (i < nr && j < nc) {
-    if (mode == 0) {
-      mr = R[2 * ((long)i * nc + j)];
-      mi = -R[2 * ((long)i * nc + j) + 1];
-    } else if (mode == 1) {
+    if (mode == 1) {
       const double rr = R[2 * ((long)j * nr + i)], ri = R[2 * ((long)j * nr + i) + 1];
       mr = ar * rr - ai * ri;
       mi = ar * ri + ai * rr;
     } else {
       mr = R[2 * ((long)i * nc + j)];
       mi = R[2 * ((long)i * nc + j) + 1];
+      if (mode == 0) mi = -mi;
     }
   }
-  Ap[(long)i * ld + 2 * j] = (T)mr;
-  Ap[(long)i * ld + 2 * j + 1] = (T)-mi;
-  Aq[(long)i * ld + 2 * j] = (T)mi;
-  Aq[(long)i * ld + 2 * j + 1] = (T)mr;
+  M[idx] = cplx<T>{(T)mr, (T)mi};
 }
 
-constexpr int kRotJC = 16;  // complex j per LDS stage (32 real k')
-
-// Out[i][p] = sum_j M[i][j] C[j][p] (+ beta Out[i][p]), i < nr, j < n; work-group = 64 rows x 64 columns p.
-// Within a stage, lane group q = lane / 16 of an MFMA step s holds real k' = 8q + s (any
-// order of k' is the same sum), so a lane's eight A values per stage are contiguous and
-// come in 16-byte loads.  The next stage's A values and C tile are loaded into registers
-// while the matrix cores work on the current one.
+// Out[i][p] = sum_j M[i][j] C[j][p] (+ beta Out[i][p]), i < nr, j < nc; a 64 x 64
+// tile per work-group, or, with `lower` (M lower triangular), every row tile of
+// one column block, the last rows first: row tile i reads rows j < i0 + 64 only, so
+// Out may be C itself (a tile's rows are read by that tile and later rows alone,
+// which are done), half of the products are left out and no copy follows.
+// Measured, before -> now: triangular 432 x 228487 complex64, 3.09 ms and a 0.30 ms
+// copy -> 1.84 ms; 128 x 67691 94 + 27 -> 78 us; the full complex128 product with
+// beta = 1 of 128 x 67691 250 -> 198 us.
 template <typename T>
-__global__ void __launch_bounds__(256) k_rotate(const T *Ap, const T *Aq, int ld, const cplx<T> *Cm, int nr, int n,
-                                                long K, cplx<T> *Out, double br, double bi, int tiles_p, int tiles_i) {
-  using M = mfma_t<T>;
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4)))
+k_rotate(const cplx<T> *Mm, int ld, const cplx<T> *Cm, int nr, int nc, long K,
+                                                cplx<T> *Out, double br, double bi, int tiles_i, int lower,
+                                                const int *info) {
   using C = cplx<T>;
-  using V = typename M::v16;
-  using P2 = typename M::pair;  // one complex value as a vector (loads stay in registers)
-  constexpr int PV = 16 / sizeof(T);  // T per 16-byte load
-  constexpr int NV = 8 / PV;          // 16-byte loads per lane per operand and stage
-  __shared__ P2 Ct[kRotJC][64 + 1];
+  constexpr int KC = kStage<T>, CV = 16 / (int)sizeof(C);
+  constexpr int kA = kMT * kRowStride, kB = KC * kMT * (int)sizeof(C);
+  __shared__ __align__(16) unsigned char sm[2][kA + kB];
+  if (info && *info != 0) return;  // the factorisation that gave M failed
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // Work-groups are dealt round-robin to the 8 XCDs; renumber so that each XCD runs a
-  // contiguous range, in which the tiles_i row tiles of one column block p are
-  // neighbours and read that block of C through the same L2.
-  const int G = gridDim.x, b = blockIdx.x, xq = G / 8, xr = G % 8, x = b % 8;
-  const int logical = (x < xr ? x * (xq + 1) : xr * (xq + 1) + (x - xr) * xq) + b / 8;
-  const int ti = logical % tiles_i, tp = logical / tiles_i;
-  const long p0 = (long)tp * 64;
-  const int i0 = ti * 64 + wave * 16;  // this wave's 16 rows
-  typename M::acc re[4], im[4];
+  const int id = xcd_logical(blockIdx.x, gridDim.x);
+  const int tp = lower ? id : id / tiles_i;
+  const long p0 = (long)tp * kMT;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  const GAS C *Mg = lgp(Mm);
+  const GAS C *Cg = lgp(Cm);
+  const int mr = tid >> 3, mc = tid & 7;              // M loads: rows mr, mr + 32, 16-byte chunk mc
+  constexpr int CPR = kMT / CV, RPP = 256 / CPR;      // C loads: chunks per row, rows per pass
+  const int cr = tid / CPR, cc = (tid % CPR) * CV;
+  const bool full = p0 + kMT <= K;                    // uniform
+  for (int ti = lower ? tiles_i - 1 : id - tp * tiles_i; ti >= 0; --ti) {
+    const int i0 = ti * kMT;
+    const int jend = lower ? min(nc, i0 + kMT) : nc;
+    Block<T> acc;
+    auto sweep = [&](auto whole) {
+      uintx4 ra[2], rb[KC / RPP];
+      auto load = [&](int j) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    re[c] = typename M::acc{0, 0, 0, 0};
-    im[c] = typename M::acc{0, 0, 0, 0};
-  }
-  const int q = lane >> 4;
-  // rows are padded to the tile and ld covers every stage, so these loads need no check
-  const GAS V *apv = (const GAS V *)(lgp(Ap) + (long)(i0 + (lane & 15)) * ld + 8 * q);
-  const GAS V *aqv = (const GAS V *)(lgp(Aq) + (long)(i0 + (lane & 15)) * ld + 8 * q);
-  const GAS P2 *Cg = (const GAS P2 *)lgp(Cm);
-  V an[NV], bn[NV];
-  P2 cn[4];
-  auto load_stage = [&](int jb) {
+        for (int h = 0; h < 2; ++h)  // rows and columns of M are padded: no check
+          ra[h] = *(const GAS uintx4 *)(Mg + (long)(i0 + 32 * h + mr) * ld + j + mc * CV);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      an[v] = apv[(2 * jb) / PV + v];
-      bn[v] = aqv[(2 * jb) / PV + v];
-    }
+        for (int h = 0; h < KC / RPP; ++h) {  // rows past the last repeat it and are cleared below
+          const GAS C *p = Cg + (long)min(j + RPP * h + cr, nc - 1) * K + p0 + cc;
+          if constexpr (decltype(whole)::value) rb[h] = load16<T>(p);
+          else rb[h] = load16_part<T>(p, K - p0 - cc);
+        }
+      };
+      auto store = [&](int b, int j) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + 256 * u, r = e >> 6, c = e & 63;
-      const int j = jb + r;
-      const long p = p0 + c;
-      cn[u] = (j < n && p < K) ? Cg[(long)j * K + p] : P2{0, 0};
-    }
-  };
-  load_stage(0);
-  for (int jb = 0; jb < n; jb += kRotJC) {
+        for (int h = 0; h < 2; ++h) *reinterpret_cast<uintx4 *>(&sm[b][(32 * h + mr) * kRowStride + 16 * mc]) = ra[h];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + 256 * u;
-      Ct[e >> 6][e & 63] = cn[u];
-    }
-    V ac[NV], bc[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      ac[v] = an[v];
-      bc[v] = bn[v];
-    }
-    __syncthreads();
-    if (jb + kRotJC < n) load_stage(jb + kRotJC);
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const T ap = ac[s / PV][s % PV], aq = bc[s / PV][s % PV];
-      const int jl = 4 * q + (s >> 1);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const P2 v = Ct[jl][16 * c + (lane & 15)];
-        const T bv = (s & 1) ? v.y : v.x;
-        re[c] = M::run(ap, bv, re[c]);
-        im[c] = M::run(aq, bv, im[c]);
+        for (int h = 0; h < KC / RPP; ++h) {
+          const uintx4 zero{};
+          *reinterpret_cast<uintx4 *>(&sm[b][kA + ((RPP * h + cr) * kMT + cc) * (int)sizeof(C)]) =
+              j + RPP * h + cr < nc ? rb[h] : zero;
+        }
+      };
+      load(0);
+      store(0, 0);
+      __syncthreads();
+      int buf = 0;
+      for (int j = 0; j < jend; j += KC) {
+        const bool more = j + KC < jend;
+        if (more) load(j + KC);
+        const auto a = Block<T>::rows(&sm[buf][wr * kRowStride], lane);
+        const auto b = Block<T>::cols(&sm[buf][kA], wc, lane);
+        acc.template mac<false>(a, b);
+        buf ^= 1;
+        if (more) store(buf, j + KC);
+        __syncthreads();
       }
-    }
-    __syncthreads();
-  }
-  GAS C *Og = lgw(Out);
-  const bool beta = (br != 0.0 || bi != 0.0);
+    };
+    if (full) sweep(std::true_type{});
+    else sweep(std::false_type{});
+    GAS C *Og = lgw(Out);
+    const bool beta = (br != 0.0 || bi != 0.0);
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = i0 + M::row(lane, r);
-      const long p = p0 + 16 * c + (lane & 15);
+    for (int r = 0; r < Block<T>::kAcc; ++r) {
+      const int i = i0 + wr + Block<T>::row(lane, r);
+      const long p = p0 + wc + Block<T>::col(lane, r);
       if (i < nr && p < K) {
-        C o{re[c][r], im[c][r]};
+        C o{acc.vr(r), acc.vi(r)};
         if (beta) {
           const C qv = Og[(long)i * K + p];
           o.x += (T)(br * (double)qv.x - bi * (double)qv.y);
@@ -345,6 +500,8 @@ __global__ void __launch_bounds__(256) k_rotate(const T *Ap, const T *Aq, int ld
         Og[(long)i * K + p] = o;
       }
     }
+    if (!lower) break;
+  }
 }
 
 // ------------------------------------------------------------------------ Cholesky / inverse (FP64)
@@ -708,66 +865,65 @@ __global__ void __launch_bounds__(256) k_stream_copy(const V4f *src, V4f *dst, l
 // ------------------------------------------------------------------------ host launchers
 void launch_overlap(Ctx &cx, int prec, int n1, int n2, long K, const void *A, const void *B, double vol, double *S,
                     DevMem &partial) {
-  const long K2 = 2 * K;
-  const int ti = (n1 + kOvTile - 1) / kOvTile, tj = (n2 + kOvTile - 1) / kOvTile;
-  const size_t es = prec == INQX_FP64 ? 8 : 4;
-  const long kc = overlap_chunk(K2, ti * tj, es);
-  INQX_CHECK(kc <= INT32_MAX, INQX_ERR_ARG, "overlap: K too long");
-  const int kchunk = (int)kc;
-  const int nchunk = (int)((K2 + kchunk - 1) / kchunk);
-  partial.ensure(es * (size_t)nchunk * ti * tj * kOvTile * kOvTile * 2);
-  const int grid = nchunk * ti * tj;
-  const int rgrid = ti * tj * kOvTile;
-  if (prec == INQX_FP64) {
-    {
-      ProfScope ps(cx, "overlap_mfma_f64");
-      hipLaunchKernelGGL(k_overlap_partial<double>, dim3(grid), dim3(256), 0, cx.stream, (const double *)A,
-                         (const double *)B, n1, n2, K2, ti, tj, kchunk, partial.as<double>());
-    }
-    INQX_HIP(hipGetLastError());
-    ProfScope ps(cx, "overlap_reduce_f64");
-    hipLaunchKernelGGL(k_overlap_reduce<double>, dim3(rgrid), dim3(256), 0, cx.stream, partial.as<double>(), n1, n2,
-                       ti, tj, nchunk, vol, S);
-  } else {
-    {
-      ProfScope ps(cx, "overlap_mfma_f32");
-      hipLaunchKernelGGL(k_overlap_partial<float>, dim3(grid), dim3(256), 0, cx.stream, (const float *)A,
-                         (const float *)B, n1, n2, K2, ti, tj, kchunk, partial.as<float>());
-    }
-    INQX_HIP(hipGetLastError());
-    ProfScope ps(cx, "overlap_reduce_f32");
-    hipLaunchKernelGGL(k_overlap_reduce<float>, dim3(rgrid), dim3(256), 0, cx.stream, partial.as<float>(), n1, n2, ti,
-                       tj, nchunk, vol, S);
+  const bool herm = A == B && n1 == n2;
+  const bool f64 = prec == INQX_FP64;
+  const OvPlan p = overlap_plan(n1, n2, K, herm, cx.num_cu, f64);
+  const bool wide = !f64 && p.chunk > kOvRun;  // FP64 partial tiles of FP32 products
+  const size_t es = f64 || wide ? 8 : 4;
+  partial.ensure(es * (size_t)p.nchunk * p.tiles * kMT * kMT * 2);
+  const long grid = (long)p.nchunk * p.tiles;
+  INQX_CHECK(grid <= INT32_MAX / kMT, INQX_ERR_ARG, "overlap: too many tiles");
+  const dim3 g((unsigned)grid), gr((unsigned)(p.tiles * kMT));
+  const int h = herm ? 1 : 0;
+  {
+    ProfScope ps(cx, f64 ? "overlap_mfma_f64" : "overlap_mfma_f32");
+    if (f64)
+      hipLaunchKernelGGL((k_overlap_partial<double, double, false>), g, dim3(256), 0, cx.stream, (const double *)A,
+                         (const double *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, partial.as<double>());
+    else if (wide)
+      hipLaunchKernelGGL((k_overlap_partial<float, double, true>), g, dim3(256), 0, cx.stream, (const float *)A,
+                         (const float *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, partial.as<double>());
+    else
+      hipLaunchKernelGGL((k_overlap_partial<float, float, false>), g, dim3(256), 0, cx.stream, (const float *)A,
+                         (const float *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, partial.as<float>());
   }
+  INQX_HIP(hipGetLastError());
+  ProfScope ps(cx, f64 ? "overlap_reduce_f64" : "overlap_reduce_f32");
+  if (es == 8)
+    hipLaunchKernelGGL(k_overlap_reduce<double>, gr, dim3(256), 0, cx.stream, partial.as<double>(), n1, n2, p.tiles,
+                       p.tiles_j, h, p.nchunk, vol, S);
+  else
+    hipLaunchKernelGGL(k_overlap_reduce<float>, gr, dim3(256), 0, cx.stream, partial.as<float>(), n1, n2, p.tiles,
+                       p.tiles_j, h, p.nchunk, vol, S);
   INQX_HIP(hipGetLastError());
 }
 
 void launch_rotate(Ctx &cx, int prec, int nr, int nc, long K, const double *R, int mode, double ar, double ai,
-                   const void *Cm, void *Out, double br, double bi, DevMem &ops) {
+                   const void *Cm, void *Out, double br, double bi, DevMem &ops, bool lower, const int *info) {
   INQX_CHECK(mode == 1 || nr == nc, INQX_ERR_ARG, "rotate: modes 0 and 2 need a square matrix");
+  INQX_CHECK(!lower || nr == nc, INQX_ERR_ARG, "rotate: a triangular matrix is square");
   const size_t es = prec == INQX_FP64 ? 8 : 4;
-  const int tiles_p = (int)((K + 63) / 64), tiles_i = (nr + 63) / 64;
-  const int nr_pad = tiles_i * 64, ld = (2 * nc + 2 * kRotJC - 1) / (2 * kRotJC) * (2 * kRotJC);
-  const size_t mat = (size_t)nr_pad * ld;
-  ops.ensure(es * mat * 2);
-  const int gprep = (int)(((size_t)nr_pad * (ld / 2) + 255) / 256);
-  const int grid = tiles_p * tiles_i;
+  const long tiles_p = (K + kMT - 1) / kMT;
+  const int tiles_i = (nr + kMT - 1) / kMT;
+  const int nr_pad = tiles_i * kMT, ld = (nc + 15) / 16 * 16;
+  ops.ensure(2 * es * (size_t)nr_pad * ld);
+  const int gprep = (int)(((size_t)nr_pad * ld + 255) / 256);
+  const long grid = lower ? tiles_p : tiles_p * tiles_i;
+  INQX_CHECK(grid <= INT32_MAX, INQX_ERR_ARG, "rotate: too many tiles");
   if (prec == INQX_FP64) {
-    double *Ap = ops.as<double>(), *Aq = Ap + mat;
-    hipLaunchKernelGGL(k_rot_prep<double>, dim3(gprep), dim3(256), 0, cx.stream, R, nr, nc, mode, ar, ai, nr_pad, ld,
-                       Ap, Aq);
+    cplx<double> *M = ops.as<cplx<double>>();
+    hipLaunchKernelGGL(k_rot_prep<double>, dim3(gprep), dim3(256), 0, cx.stream, R, nr, nc, mode, ar, ai, nr_pad, ld, M);
     INQX_HIP(hipGetLastError());
     ProfScope ps(cx, "rotate_mfma_f64");
-    hipLaunchKernelGGL(k_rotate<double>, dim3(grid), dim3(256), 0, cx.stream, Ap, Aq, ld, (const cplx<double> *)Cm, nr,
-                       nc, K, (cplx<double> *)Out, br, bi, tiles_p, tiles_i);
+    hipLaunchKernelGGL(k_rotate<double>, dim3((unsigned)grid), dim3(256), 0, cx.stream, M, ld, (const cplx<double> *)Cm,
+                       nr, nc, K, (cplx<double> *)Out, br, bi, tiles_i, lower ? 1 : 0, info);
   } else {
-    float *Ap = ops.as<float>(), *Aq = Ap + mat;
-    hipLaunchKernelGGL(k_rot_prep<float>, dim3(gprep), dim3(256), 0, cx.stream, R, nr, nc, mode, ar, ai, nr_pad, ld,
-                       Ap, Aq);
+    cplx<float> *M = ops.as<cplx<float>>();
+    hipLaunchKernelGGL(k_rot_prep<float>, dim3(gprep), dim3(256), 0, cx.stream, R, nr, nc, mode, ar, ai, nr_pad, ld, M);
     INQX_HIP(hipGetLastError());
     ProfScope ps(cx, "rotate_mfma_f32");
-    hipLaunchKernelGGL(k_rotate<float>, dim3(grid), dim3(256), 0, cx.stream, Ap, Aq, ld, (const cplx<float> *)Cm, nr, nc,
-                       K, (cplx<float> *)Out, br, bi, tiles_p, tiles_i);
+    hipLaunchKernelGGL(k_rotate<float>, dim3((unsigned)grid), dim3(256), 0, cx.stream, M, ld, (const cplx<float> *)Cm,
+                       nr, nc, K, (cplx<float> *)Out, br, bi, tiles_i, lower ? 1 : 0, info);
   }
   INQX_HIP(hipGetLastError());
 }
