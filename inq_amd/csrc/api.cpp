@@ -863,9 +863,14 @@ int inqx_overlap_diagonal(inqx_ctx ctx, int precision, int n, long npw, double v
   API_END(ctx)
 }
 
-static int cholesky_impl(inqx_ctx ctx, int n, double *S) {
+static int *launch_cholesky_info(inqx_ctx ctx, int n, double *S) {
   ctx->c.ws_info.ensure(sizeof(int));
   launch_cholesky(ctx->c, n, S, ctx->c.ws_info.as<int>());
+  return ctx->c.ws_info.as<int>();
+}
+
+// the status word of the last factorisation (waits for it)
+static int cholesky_status(inqx_ctx ctx) {
   int info = 0;
   INQX_HIP(hipMemcpyAsync(&info, ctx->c.ws_info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->c.stream));
   INQX_HIP(hipStreamSynchronize(ctx->c.stream));
@@ -875,7 +880,8 @@ static int cholesky_impl(inqx_ctx ctx, int n, double *S) {
 int inqx_cholesky(inqx_ctx ctx, int n, void *S) {
   API_BEGIN
   INQX_CHECK(ctx && !ctx->c.host_only && S && n > 0, INQX_ERR_ARG, "bad arguments");
-  const int info = cholesky_impl(ctx, n, (double *)S);
+  launch_cholesky_info(ctx, n, (double *)S);
+  const int info = cholesky_status(ctx);
   INQX_CHECK(info == 0, INQX_ERR_NOT_PD, "Cholesky: leading minor " + std::to_string(info) + " is not positive definite");
   API_END(ctx)
 }
@@ -883,13 +889,18 @@ int inqx_cholesky(inqx_ctx ctx, int n, void *S) {
 int inqx_invert_triangular(inqx_ctx ctx, int n, const void *L, void *Linv) {
   API_BEGIN
   INQX_CHECK(ctx && !ctx->c.host_only && L && Linv && n > 0 && L != Linv, INQX_ERR_ARG, "bad arguments");
-  launch_trinv(ctx->c, n, (const double *)L, (double *)Linv);
+  launch_trinv(ctx->c, n, (const double *)L, (double *)Linv, ctx->c.ws_partial);
   API_END(ctx)
 }
 
-// phi <- phi Linv^H (Linv lower triangular) in place
-static void rotate_lower(inqx_ctx ctx, int precision, int n, long npw, const double *Linv, void *phi) {
-  launch_rotate(ctx->c, precision, n, n, npw, Linv, 0, 1.0, 0.0, phi, phi, 0.0, 0.0, ctx->c.ws_ops, true);
+// S = L L^H, phi <- phi L^{-H} in place, without a host wait between the two: the
+// rotation checks the factorisation's status on the device and leaves phi as it
+// is when S is not positive definite.  Returns the status.
+static int cholesky_rotate(inqx_ctx ctx, int precision, int n, long npw, double *S, double *X, void *phi) {
+  const int *info = launch_cholesky_info(ctx, n, S);
+  launch_trinv(ctx->c, n, S, X, ctx->c.ws_partial);
+  launch_rotate(ctx->c, precision, n, n, npw, X, 0, 1.0, 0.0, phi, phi, 0.0, 0.0, ctx->c.ws_ops, true, info);
+  return cholesky_status(ctx);
 }
 
 // phi <- M phi through a temporary (rows of the output depend on all rows of phi)
@@ -923,10 +934,8 @@ static void orthogonalize_impl(inqx_ctx ctx, int precision, int n, long npw, dou
   ctx->c.ws_X.ensure(16 * (size_t)n * n);
   double *S = ctx->c.ws_S.as<double>(), *X = ctx->c.ws_X.as<double>();
   launch_overlap(ctx->c, precision, n, n, npw, phi, phi, vol_el, S, ctx->c.ws_partial);
-  const int info = cholesky_impl(ctx, n, S);
+  const int info = cholesky_rotate(ctx, precision, n, npw, S, X, phi);
   INQX_CHECK(info == 0, INQX_ERR_NOT_PD, "orthogonalize: overlap not positive definite (minor " + std::to_string(info) + ")");
-  launch_trinv(ctx->c, n, S, X);
-  rotate_lower(ctx, precision, n, npw, X, phi);  // phi <- phi Linv^H
 }
 
 int inqx_orthogonalize(inqx_ctx ctx, int precision, int n, long npw, double vol_el, void *phi) {
@@ -1478,10 +1487,8 @@ static double ace_build_impl(inqx_ham h, Basis &B, int nst, int precision, const
   INQX_HIP(hipStreamSynchronize(ctx->c.stream));
   double en = 0.0;  // -1/2 sum occ_i M_ii (exchange_operator.hpp:108)
   for (int i = 0; i < nst; ++i) en += -0.5 * occ[i] * m[(size_t)i * nst + i].real();
-  const int info = cholesky_impl(ctx, nst, S);
+  const int info = cholesky_rotate(ctx, precision, nst, npw, S, X, xi);  // xi <- W L^{-H} (rotate_trs)
   INQX_CHECK(info == 0, INQX_ERR_NOT_PD, "ACE: exchange matrix not positive definite (minor " + std::to_string(info) + ")");
-  launch_trinv(ctx->c, nst, S, X);
-  rotate_lower(ctx, precision, nst, npw, X, xi);  // xi <- W L^{-H} (rotate_trs)
   return en;
 }
 

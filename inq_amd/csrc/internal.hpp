@@ -353,7 +353,8 @@ void launch_rotate(Ctx &cx, int prec, int nr, int nc, long K, const double *R, i
                    const void *Cm, void *Out, double br, double bi, DevMem &ops, bool lower = false,
                    const int *info = nullptr);
 void launch_cholesky(Ctx &cx, int n, double *S, int *info);
-void launch_trinv(Ctx &cx, int n, const double *L, double *X);
+// X = L^{-1}; work: a workspace that grows to n x n complex values
+void launch_trinv(Ctx &cx, int n, const double *L, double *X, DevMem &work);
 void launch_stream_copy(Ctx &cx, const void *src, void *dst, size_t bytes);
 void launch_fill_zero(Ctx &cx, void *p, size_t bytes);
 void launch_randomize(Ctx &cx, int type, long npoints, int nst, int index, int layout, void *out);
