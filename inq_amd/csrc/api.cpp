@@ -1014,31 +1014,20 @@ static void ensure_g2h(inqx_ham h, Basis &b) {
   INQX_HIP(hipStreamSynchronize(h->ctx->c.stream));
 }
 
-// scalar workspace: dot partials, then per state the (H phi, phi) and (phi, phi)
-// pair, the preconditioner pair, the four residual overlaps and lambda
+// partial sums per (state, chunk): the energy sums of the current and the next
+// step, the preconditioner's and the four residual overlaps
 struct SdScal {
-  double *part, *en, *kn, *m03, *lam;
+  double *en[2], *kn, *m03;
 };
 static SdScal sd_scalars(inqx_ham h, int nst, long npw) {
-  const size_t pb = (sd_dots_partial_bytes(nst, npw) + 255) / 256 * 256;
-  const size_t per = (size_t)nst * sizeof(double);
-  h->sd_scal.ensure(pb + per * (4 + 4 + 8 + 1));
-  char *base = (char *)h->sd_scal.p;
+  const size_t per = (size_t)nst * sd_chunks(npw);
+  h->sd_scal.ensure(per * (4 + 4 + 2 + 8) * sizeof(double));
   SdScal r;
-  r.part = (double *)base;
-  r.en = (double *)(base + pb);
-  r.kn = r.en + 4 * (size_t)nst;
-  r.m03 = r.kn + 4 * (size_t)nst;
-  r.lam = r.m03 + 8 * (size_t)nst;
+  r.en[0] = (double *)h->sd_scal.p;
+  r.en[1] = r.en[0] + 4 * per;
+  r.kn = r.en[1] + 4 * per;
+  r.m03 = r.kn + 2 * per;
   return r;
-}
-
-static void precondition_impl(inqx_ham h, Basis &B, int nst, int prec, void *phi, const SdScal &sc) {
-  Ctx &cx = h->ctx->c;
-  ensure_g2h(h, B);
-  const void *a[2] = {phi, phi};
-  launch_sd_dots(cx, prec, nst, B.npw, 2, a, a, B.d_g2h.as<double>(), 1, 1.0, sc.part, sc.kn);
-  launch_tpa_scale(cx, prec, nst, B.npw, phi, B.d_g2h.as<double>(), sc.kn);
 }
 
 static void check_sd(inqx_ham h, inqx_basis bs, int nst, int precision, const void *phi) {
@@ -1053,7 +1042,11 @@ int inqx_precondition(inqx_ham h, inqx_basis bs, int nst, int precision, void *p
   inqx_ctx ctx = h ? h->ctx : nullptr;
   API_BEGIN
   check_sd(h, bs, nst, precision, phi);
-  precondition_impl(h, bs->b, nst, precision, phi, sd_scalars(h, nst, bs->b.npw));
+  const SdScal sc = sd_scalars(h, nst, bs->b.npw);
+  ensure_g2h(h, bs->b);
+  const double *g2h = bs->b.d_g2h.as<double>();
+  launch_tpa_sums(ctx->c, precision, nst, bs->b.npw, phi, g2h, sc.kn);
+  launch_tpa_scale(ctx->c, precision, nst, bs->b.npw, phi, g2h, sc.kn);
   API_END(ctx)
 }
 
@@ -1079,18 +1072,22 @@ int inqx_steepest_descent(inqx_ham h, inqx_basis bs, int nst, int precision, int
     if (precision == INQX_FP64) launch_apply<double>(h, 1, &bb, &nst, &in, &out);
     else launch_apply<float>(h, 1, &bb, &nst, &in, &out);
   };
+  const double *g2h = nullptr;
+  if (precondition) {
+    ensure_g2h(h, B);
+    g2h = B.d_g2h.as<double>();
+  }
   apply(phi, hphi);
+  if (num_steps > 0) launch_sd_energy(cx, precision, nst, npw, phi, hphi, sc.en[0]);
   for (int step = 0; step < num_steps; ++step) {
-    // eigenvalue (H phi, phi) and norm (phi, phi), then the residual
-    const void *a1[2] = {hphi, phi}, *b1[2] = {phi, phi};
-    launch_sd_dots(cx, precision, nst, npw, 2, a1, b1, nullptr, 0, vol, sc.part, sc.en);
-    launch_sd_residual(cx, precision, nst, npw, phi, hphi, res, sc.en);
-    if (precondition) precondition_impl(h, B, nst, precision, res, sc);
+    const double *en = sc.en[step & 1];
+    launch_sd_residual(cx, precision, nst, npw, phi, hphi, res, en, vol, g2h, sc.kn);
+    if (precondition) launch_tpa_scale(cx, precision, nst, npw, res, g2h, sc.kn);
     apply(res, hres);
-    const void *a2[4] = {res, phi, res, phi}, *b2[4] = {res, res, hres, hres};
-    launch_sd_dots(cx, precision, nst, npw, 4, a2, b2, nullptr, 0, vol, sc.part, sc.m03);
-    launch_sd_lambda(cx, nst, sc.m03, sc.en, sc.lam);
-    launch_sd_update(cx, precision, nst, npw, phi, step != num_steps - 1 ? hphi : nullptr, res, hres, sc.lam);
+    launch_sd_cross(cx, precision, nst, npw, phi, res, hres, sc.m03);
+    const bool last = step == num_steps - 1;
+    launch_sd_update(cx, precision, nst, npw, phi, last ? nullptr : hphi, res, hres, sc.m03, en, vol,
+                     sc.en[(step + 1) & 1]);
   }
   orthogonalize_impl(ctx, precision, nst, npw, vol, phi);
   // complex64 states: a second Cholesky pass (CholeskyQR2).  After the line

@@ -2,15 +2,26 @@
 // eigensolver and of the Teter-Payne-Allan preconditioner on band-major sphere
 // states [nst][npw].
 //
-//   dots       d_k(s) = vol sum_G w_k(G) conj(a_k(s,G)) b_k(s,G), up to four
-//              pairs per pass (operations::overlap_diagonal,
-//              src/operations/overlap_diagonal.hpp:25-60); FP64 accumulation,
-//              partial sums over fixed 4096-point chunks added in chunk order,
-//              so the result does not depend on the launch.
-//   residual   r = H phi - (e / Re n) phi  (steepest_descent.hpp:37-49)
-//   tpa        r(G) *= K((1/2)|G|^2 / <T>)  (preconditioner.hpp:31-58)
-//   update     lambda from the six state overlaps, phi += lambda r and
-//              H phi += lambda H r  (steepest_descent.hpp:53-83)
+// Every pass is bound by HBM, so a step reads and writes each block as few times
+// as its dependencies allow, and a pass ends with the per-state sums that the
+// next one needs:
+//
+//   energy    (H phi, phi), (phi, phi)                         before the first step
+//   residual  r = H phi - (e / Re n) phi  (steepest_descent.hpp:37-49), with the
+//             preconditioner's sums of r
+//   tpa       r(G) *= K((1/2)|G|^2 / <T>)  (preconditioner.hpp:31-58)
+//   cross     (r, r), (phi, r), (r, H r), (phi, H r)            after H r
+//   update    lambda from the six state overlaps, phi += lambda r and
+//             H phi += lambda H r  (steepest_descent.hpp:53-83), with the energy
+//             sums of the next step
+//
+// One work-group takes 4096 points of one state: it adds the previous pass's
+// partial sums of its state itself (in chunk order, FP64) instead of waiting for
+// a kernel that does, and leaves its own, so sums do not depend on the launch.
+// The overlaps are those of operations::overlap_diagonal
+// (src/operations/overlap_diagonal.hpp:25-60).  128 states x 67691, complex64, per
+// step: ten launches and 290 us with separate dot, combine and lambda kernels, four
+// launches and 175 us now (a pass moves 138-414 MB: 23-69 us at 6 TB/s).
 #include "internal.hpp"
 
 #include <algorithm>
@@ -31,75 +42,123 @@ template <typename T> __device__ __forceinline__ GAS T *sgw(T *p) { return (GAS 
 constexpr int kChunk = 4096;
 constexpr int kThreads = 256;
 
-struct DotArgs {
-  const void *a[4];
-  const void *b[4];
-  const double *w;  // weight per sphere point for the pairs with bit k of wmask set
-  int wmask;
-  int n;
+// state and points of a work-group
+struct SdItem {
+  int s, c;
+  long p0, p1;
 };
+__device__ __forceinline__ SdItem sd_item(long K, int nch) {
+  SdItem it;
+  it.s = blockIdx.x / nch;
+  it.c = blockIdx.x - it.s * nch;
+  it.p0 = (long)it.c * kChunk;
+  it.p1 = it.p0 + kChunk < K ? it.p0 + kChunk : K;
+  return it;
+}
 
-// partial sums of one (state, chunk): part[(s * nch + c) * n + k] (re, im)
+// acc[0..N) summed over the work-group into part[(s nch + c) N + k], in a fixed order
+template <int N>
+__device__ __forceinline__ void sd_store_sums(double (&acc)[N], double *part, const SdItem &it, int nch) {
+  __shared__ double red[kThreads / 64][N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = acc[k];
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < N) {
+    double t = red[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kThreads / 64; ++w) t += red[w][threadIdx.x];
+    sgw(part)[((size_t)it.s * nch + it.c) * N + threadIdx.x] = t;
+  }
+}
+
+// the sums of one state over its chunks, in chunk order, on every thread
+template <int N> __device__ __forceinline__ void sd_load_sums(double (&out)[N], const double *part, int s, int nch) {
+  __shared__ double tot[N];
+  if ((int)threadIdx.x < N) {
+    const GAS double *q = sgp(part) + (size_t)s * nch * N + threadIdx.x;
+    double t = 0.0;
+#pragma unroll 4
+    for (int c = 0; c < nch; ++c) t += q[(size_t)c * N];
+    tot[threadIdx.x] = t;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) out[k] = tot[k];
+}
+
+// += conj(x) y in FP64
+template <typename C> __device__ __forceinline__ void dot_add(double &re, double &im, const C &x, const C &y) {
+  re += (double)x.x * y.x + (double)x.y * y.y;
+  im += (double)x.x * y.y - (double)x.y * y.x;
+}
+
+// sums {(H phi, phi), (phi, phi)}
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_sd_dots(DotArgs d, long K, int nch, double *part) {
+__global__ void __launch_bounds__(kThreads) k_sd_energy(const cplx<T> *phi, const cplx<T> *hphi, long K, int nch,
+                                                        double *part) {
   using C = cplx<T>;
-  __shared__ double red[8][kThreads];
-  const int tid = threadIdx.x;
-  const int c = blockIdx.x % nch, s = blockIdx.x / nch;
-  double acc[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = 0.0;
-  const long p0 = (long)c * kChunk;
-  const long p1 = p0 + kChunk < K ? p0 + kChunk : K;
-  for (long p = p0 + tid; p < p1; p += kThreads) {
-    const double wp = d.w ? sgp(d.w)[p] : 1.0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (k < d.n) {
-        const C x = sgp(reinterpret_cast<const C *>(d.a[k]))[(size_t)s * K + p];
-        const C y = sgp(reinterpret_cast<const C *>(d.b[k]))[(size_t)s * K + p];
-        const double wk = (d.wmask >> k) & 1 ? wp : 1.0;
-        acc[2 * k] += wk * ((double)x.x * y.x + (double)x.y * y.y);
-        acc[2 * k + 1] += wk * ((double)x.x * y.y - (double)x.y * y.x);
-      }
+  const SdItem it = sd_item(K, nch);
+  const GAS C *f = sgp(phi) + (size_t)it.s * K, *h = sgp(hphi) + (size_t)it.s * K;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (long p = it.p0 + threadIdx.x; p < it.p1; p += kThreads) {
+    const C x = f[p], y = h[p];
+    dot_add(acc[0], acc[1], y, x);
+    dot_add(acc[2], acc[3], x, x);
+  }
+  sd_store_sums(acc, part, it, nch);
+}
+
+// sums {sum g2h |r|^2, sum |r|^2}
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_tpa_sums(const cplx<T> *res, const double *g2h, long K, int nch,
+                                                       double *part) {
+  using C = cplx<T>;
+  const SdItem it = sd_item(K, nch);
+  const GAS C *r = sgp(res) + (size_t)it.s * K;
+  double acc[2] = {0.0, 0.0};
+#pragma unroll 4
+  for (long p = it.p0 + threadIdx.x; p < it.p1; p += kThreads) {
+    const C v = r[p];
+    const double n2 = (double)v.x * v.x + (double)v.y * v.y;
+    acc[0] += sgp(g2h)[p] * n2;
+    acc[1] += n2;
+  }
+  sd_store_sums(acc, part, it, nch);
+}
+
+// r = hphi - (e / Re n) phi with (e, n) the energy sums times vol; TPA: the
+// preconditioner's sums of r
+template <typename T, bool TPA>
+__global__ void __launch_bounds__(kThreads) k_sd_residual(const cplx<T> *__restrict__ phi,
+                                                          const cplx<T> *__restrict__ hphi, cplx<T> *__restrict__ res,
+                                                          long K, int nch, const double *part_e, double vol,
+                                                          const double *__restrict__ g2h, double *part_k) {
+  using C = cplx<T>;
+  const SdItem it = sd_item(K, nch);
+  double en[4];
+  sd_load_sums(en, part_e, it.s, nch);
+  const double nr = vol * en[2];
+  const T er = (T)(vol * en[0] / nr), ei = (T)(vol * en[1] / nr);
+  const GAS C *f = sgp(phi) + (size_t)it.s * K, *h = sgp(hphi) + (size_t)it.s * K;
+  GAS C *r = sgw(res) + (size_t)it.s * K;
+  double acc[2] = {0.0, 0.0};
+#pragma unroll 8
+  for (long p = it.p0 + threadIdx.x; p < it.p1; p += kThreads) {
+    const C x = f[p], y = h[p];
+    const C v{y.x - (er * x.x - ei * x.y), y.y - (er * x.y + ei * x.x)};
+    r[p] = v;
+    if constexpr (TPA) {
+      const double n2 = (double)v.x * v.x + (double)v.y * v.y;
+      acc[0] += sgp(g2h)[p] * n2;
+      acc[1] += n2;
     }
   }
-#pragma unroll
-  for (int k = 0; k < 8; ++k) red[k][tid] = acc[k];
-  __syncthreads();
-  for (int h = kThreads / 2; h > 0; h >>= 1) {
-    if (tid < h)
-#pragma unroll
-      for (int k = 0; k < 8; ++k) red[k][tid] += red[k][tid + h];
-    __syncthreads();
-  }
-  if (tid < 2 * d.n) sgw(part)[((size_t)s * nch + c) * 2 * d.n + tid] = red[tid][0];
-}
-
-// out[s * n + k] = vol * sum over chunks, in chunk order
-__global__ void __launch_bounds__(kThreads) k_sd_dots_combine(const double *part, int nst, int nch, int n, double vol,
-                                                              double *out) {
-  const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= nst * 2 * n) return;
-  const int s = i / (2 * n), r = i - s * 2 * n;
-  double acc = 0.0;
-  for (int c = 0; c < nch; ++c) acc += sgp(part)[((size_t)s * nch + c) * 2 * n + r];
-  sgw(out)[i] = vol * acc;
-}
-
-// r = hphi - (e / Re n) phi with e = en[2s], n = en[2s+1] (complex pairs)
-template <typename T>
-__global__ void __launch_bounds__(kThreads) k_sd_residual(const cplx<T> *phi, const cplx<T> *hphi, cplx<T> *res,
-                                                          const double *en, long K) {
-  using C = cplx<T>;
-  const int s = blockIdx.y;
-  const long p = (long)blockIdx.x * kThreads + threadIdx.x;
-  if (p >= K) return;
-  const GAS double *q = sgp(en) + 4 * (size_t)s;
-  const double nr = q[2];
-  const T er = (T)(q[0] / nr), ei = (T)(q[1] / nr);
-  const C f = sgp(phi)[(size_t)s * K + p], h = sgp(hphi)[(size_t)s * K + p];
-  sgw(res)[(size_t)s * K + p] = C{h.x - (er * f.x - ei * f.y), h.y - (er * f.y + ei * f.x)};
+  if constexpr (TPA) sd_store_sums(acc, part_k, it, nch);
 }
 
 __device__ __forceinline__ double tpa_k(double x) {
@@ -108,21 +167,46 @@ __device__ __forceinline__ double tpa_k(double x) {
   return num / den;
 }
 
-// r(G) *= K(g2h(G) / <T>_s), <T>_s = Re(kn[2s] / kn[2s+1]) (complex pairs)
+// r(G) *= K(g2h(G) / <T>), <T> = sum g2h |r|^2 / sum |r|^2
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_tpa_scale(cplx<T> *res, const double *g2h, const double *kn, long K) {
+__global__ void __launch_bounds__(kThreads) k_tpa_scale(cplx<T> *__restrict__ res,
+                                                        const double *__restrict__ g2h, long K, int nch,
+                                                        const double *part_k) {
   using C = cplx<T>;
-  const int s = blockIdx.y;
-  const long p = (long)blockIdx.x * kThreads + threadIdx.x;
-  if (p >= K) return;
-  const GAS double *q = sgp(kn) + 4 * (size_t)s;
-  // Re(a / b) for complex a, b
-  const double kin = (q[0] * q[2] + q[1] * q[3]) / (q[2] * q[2] + q[3] * q[3]);
-  const T f = (T)tpa_k(sgp(g2h)[p] / kin);
-  C v = sgp(res)[(size_t)s * K + p];
-  v.x *= f;
-  v.y *= f;
-  sgw(res)[(size_t)s * K + p] = v;
+  const SdItem it = sd_item(K, nch);
+  double kn[2];
+  sd_load_sums(kn, part_k, it.s, nch);
+  const double kin = kn[0] / kn[1];
+  GAS C *r = sgw(res) + (size_t)it.s * K;
+#pragma unroll 4
+  for (long p = it.p0 + threadIdx.x; p < it.p1; p += kThreads) {
+    const T f = (T)tpa_k(sgp(g2h)[p] / kin);
+    C v = r[p];
+    v.x *= f;
+    v.y *= f;
+    r[p] = v;
+  }
+}
+
+// sums {(r, r), (phi, r), (r, H r), (phi, H r)}
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_sd_cross(const cplx<T> *phi, const cplx<T> *res, const cplx<T> *hres,
+                                                       long K, int nch, double *part) {
+  using C = cplx<T>;
+  const SdItem it = sd_item(K, nch);
+  const GAS C *f = sgp(phi) + (size_t)it.s * K, *r = sgp(res) + (size_t)it.s * K, *h = sgp(hres) + (size_t)it.s * K;
+  double acc[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) acc[k] = 0.0;
+#pragma unroll 8
+  for (long p = it.p0 + threadIdx.x; p < it.p1; p += kThreads) {
+    const C x = f[p], y = r[p], z = h[p];
+    dot_add(acc[0], acc[1], y, y);
+    dot_add(acc[2], acc[3], x, y);
+    dot_add(acc[4], acc[5], y, z);
+    dot_add(acc[6], acc[7], x, z);
+  }
+  sd_store_sums(acc, part, it, nch);
 }
 
 __device__ __forceinline__ void cmul_d(double ar, double ai, double br, double bi, double &cr, double &ci) {
@@ -130,20 +214,18 @@ __device__ __forceinline__ void cmul_d(double ar, double ai, double br, double b
   ci = ar * bi + ai * br;
 }
 
-// lambda per state from m0..m3 = (r,r), (phi,r), (r,Hr), (phi,Hr) and m4, m5 = (Hphi,phi), (phi,phi)
-__global__ void __launch_bounds__(kThreads) k_sd_lambda(const double *m03, const double *m45, int nst, double *lam) {
-  const int s = blockIdx.x * kThreads + threadIdx.x;
-  if (s >= nst) return;
-  const GAS double *a = sgp(m03) + 8 * (size_t)s;
-  const GAS double *b = sgp(m45) + 4 * (size_t)s;
+// lambda of a state from m0..m3 = (r,r), (phi,r), (r,Hr), (phi,Hr) and m4, m5 = (Hphi,phi), (phi,phi)
+__device__ __forceinline__ double sd_lambda(const double (&m03)[8], const double (&m45)[4], double vol) {
   double m[6][2];
+#pragma unroll
   for (int k = 0; k < 4; ++k) {
-    m[k][0] = a[2 * k];
-    m[k][1] = a[2 * k + 1];
+    m[k][0] = vol * m03[2 * k];
+    m[k][1] = vol * m03[2 * k + 1];
   }
+#pragma unroll
   for (int k = 0; k < 2; ++k) {
-    m[4 + k][0] = b[2 * k];
-    m[4 + k][1] = b[2 * k + 1];
+    m[4 + k][0] = vol * m45[2 * k];
+    m[4 + k][1] = vol * m45[2 * k + 1];
   }
   double x, y, u, v;
   cmul_d(m[0][0], m[0][1], m[3][0], m[3][1], x, y);
@@ -156,102 +238,102 @@ __global__ void __launch_bounds__(kThreads) k_sd_lambda(const double *m03, const
   cmul_d(m[3][0], m[3][1], m[5][0], m[5][1], u, v);
   const double cc = x - u;
   const double den = cb + sqrt(cb * cb - 4.0 * ca * cc);
-  sgw(lam)[s] = fabs(den) < 1e-15 ? 0.0 : 2.0 * cc / den;
+  return fabs(den) < 1e-15 ? 0.0 : 2.0 * cc / den;
 }
 
-// phi += lambda r; hphi += lambda hr when hphi is given
+// phi += lambda r; with hphi, hphi += lambda hr and the energy sums of the result
+// (part_out: not part_e, which other work-groups of the state still read)
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_sd_update(cplx<T> *phi, cplx<T> *hphi, const cplx<T> *res,
-                                                        const cplx<T> *hres, const double *lam, long K) {
+__global__ void __launch_bounds__(kThreads) k_sd_update(cplx<T> *__restrict__ phi, cplx<T> *__restrict__ hphi,
+                                                        const cplx<T> *__restrict__ res,
+                                                        const cplx<T> *__restrict__ hres, long K, int nch,
+                                                        const double *part_m, const double *part_e, double vol,
+                                                        double *part_out) {
   using C = cplx<T>;
-  const int s = blockIdx.y;
-  const long p = (long)blockIdx.x * kThreads + threadIdx.x;
-  if (p >= K) return;
-  const T l = (T)sgp(lam)[s];
-  const size_t o = (size_t)s * K + p;
-  const C r = sgp(res)[o];
-  C f = sgp(phi)[o];
-  f.x += l * r.x;
-  f.y += l * r.y;
-  sgw(phi)[o] = f;
-  if (hphi) {
-    const C hr = sgp(hres)[o];
-    C h = sgp(hphi)[o];
-    h.x += l * hr.x;
-    h.y += l * hr.y;
-    sgw(hphi)[o] = h;
+  const SdItem it = sd_item(K, nch);
+  double m03[8], m45[4];
+  sd_load_sums(m03, part_m, it.s, nch);
+  sd_load_sums(m45, part_e, it.s, nch);
+  const T l = (T)sd_lambda(m03, m45, vol);
+  const size_t o = (size_t)it.s * K;
+  GAS C *f = sgw(phi) + o;
+  const GAS C *r = sgp(res) + o;
+  if (!hphi) {
+#pragma unroll 4
+    for (long p = it.p0 + threadIdx.x; p < it.p1; p += kThreads) {
+      const C y = r[p];
+      C x = f[p];
+      x.x += l * y.x;
+      x.y += l * y.y;
+      f[p] = x;
+    }
+    return;
   }
+  GAS C *h = sgw(hphi) + o;
+  const GAS C *hr = sgp(hres) + o;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (long p = it.p0 + threadIdx.x; p < it.p1; p += kThreads) {
+    const C y = r[p], z = hr[p];
+    C x = f[p], w = h[p];
+    x.x += l * y.x;
+    x.y += l * y.y;
+    w.x += l * z.x;
+    w.y += l * z.y;
+    f[p] = x;
+    h[p] = w;
+    dot_add(acc[0], acc[1], w, x);
+    dot_add(acc[2], acc[3], x, x);
+  }
+  sd_store_sums(acc, part_out, it, nch);
 }
-
-inline dim3 point_grid(int nst, long K) { return dim3((unsigned)((K + kThreads - 1) / kThreads), (unsigned)nst); }
 
 }  // namespace
 
-size_t sd_dots_partial_bytes(int nst, long K) { return (size_t)nst * ((K + kChunk - 1) / kChunk) * 8 * sizeof(double); }
+int sd_chunks(long K) { return (int)((K + kChunk - 1) / kChunk); }
 
-void launch_sd_dots(Ctx &cx, int prec, int nst, long K, int n, const void *const *a, const void *const *b,
-                    const double *w, int wmask, double vol, double *part, double *out) {
-  INQX_CHECK(n >= 1 && n <= 4, INQX_ERR_ARG, "one to four overlaps per pass");
-  DotArgs d{};
-  for (int k = 0; k < n; ++k) {
-    d.a[k] = a[k];
-    d.b[k] = b[k];
-  }
-  d.w = w;
-  d.wmask = w ? wmask : 0;
-  d.n = n;
-  const int nch = (int)((K + kChunk - 1) / kChunk);
-  ProfScope ps(cx, "sd_dots");
-  if (prec == INQX_FP64)
-    hipLaunchKernelGGL(k_sd_dots<double>, dim3((unsigned)(nst * nch)), dim3(kThreads), 0, cx.stream, d, K, nch, part);
-  else
-    hipLaunchKernelGGL(k_sd_dots<float>, dim3((unsigned)(nst * nch)), dim3(kThreads), 0, cx.stream, d, K, nch, part);
-  INQX_HIP(hipGetLastError());
-  const int tot = nst * 2 * n;
-  hipLaunchKernelGGL(k_sd_dots_combine, dim3((unsigned)((tot + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                     cx.stream, part, nst, nch, n, vol, out);
-  INQX_HIP(hipGetLastError());
+// KERNEL(ARGS) for the precision T over one work-group per (state, chunk)
+#define SD_LAUNCH(NAME, KERNEL, ...)                                                                      \
+  do {                                                                                                    \
+    const int nch = sd_chunks(K);                                                                         \
+    ProfScope ps(cx, NAME);                                                                               \
+    const dim3 grid((unsigned)(nst * nch));                                                               \
+    if (prec == INQX_FP64) {                                                                              \
+      using T = double;                                                                                   \
+      hipLaunchKernelGGL((KERNEL), grid, dim3(kThreads), 0, cx.stream, __VA_ARGS__);                      \
+    } else {                                                                                              \
+      using T = float;                                                                                    \
+      hipLaunchKernelGGL((KERNEL), grid, dim3(kThreads), 0, cx.stream, __VA_ARGS__);                      \
+    }                                                                                                     \
+    INQX_HIP(hipGetLastError());                                                                          \
+  } while (0)
+
+void launch_sd_energy(Ctx &cx, int prec, int nst, long K, const void *phi, const void *hphi, double *part) {
+  SD_LAUNCH("sd_energy", k_sd_energy<T>, (const cplx<T> *)phi, (const cplx<T> *)hphi, K, nch, part);
 }
-
+void launch_tpa_sums(Ctx &cx, int prec, int nst, long K, const void *res, const double *g2h, double *part) {
+  SD_LAUNCH("tpa_sums", k_tpa_sums<T>, (const cplx<T> *)res, g2h, K, nch, part);
+}
 void launch_sd_residual(Ctx &cx, int prec, int nst, long K, const void *phi, const void *hphi, void *res,
-                        const double *en) {
-  ProfScope ps(cx, "sd_residual");
-  if (prec == INQX_FP64)
-    hipLaunchKernelGGL(k_sd_residual<double>, point_grid(nst, K), dim3(kThreads), 0, cx.stream,
-                       (const cplx<double> *)phi, (const cplx<double> *)hphi, (cplx<double> *)res, en, K);
+                        const double *part_e, double vol, const double *g2h, double *part_k) {
+  if (g2h)
+    SD_LAUNCH("sd_residual", (k_sd_residual<T, true>), (const cplx<T> *)phi, (const cplx<T> *)hphi, (cplx<T> *)res, K,
+              nch, part_e, vol, g2h, part_k);
   else
-    hipLaunchKernelGGL(k_sd_residual<float>, point_grid(nst, K), dim3(kThreads), 0, cx.stream,
-                       (const cplx<float> *)phi, (const cplx<float> *)hphi, (cplx<float> *)res, en, K);
-  INQX_HIP(hipGetLastError());
+    SD_LAUNCH("sd_residual", (k_sd_residual<T, false>), (const cplx<T> *)phi, (const cplx<T> *)hphi, (cplx<T> *)res, K,
+              nch, part_e, vol, g2h, part_k);
 }
-
-void launch_tpa_scale(Ctx &cx, int prec, int nst, long K, void *res, const double *g2h, const double *kn) {
-  ProfScope ps(cx, "tpa_scale");
-  if (prec == INQX_FP64)
-    hipLaunchKernelGGL(k_tpa_scale<double>, point_grid(nst, K), dim3(kThreads), 0, cx.stream, (cplx<double> *)res,
-                       g2h, kn, K);
-  else
-    hipLaunchKernelGGL(k_tpa_scale<float>, point_grid(nst, K), dim3(kThreads), 0, cx.stream, (cplx<float> *)res, g2h,
-                       kn, K);
-  INQX_HIP(hipGetLastError());
+void launch_tpa_scale(Ctx &cx, int prec, int nst, long K, void *res, const double *g2h, const double *part_k) {
+  SD_LAUNCH("tpa_scale", k_tpa_scale<T>, (cplx<T> *)res, g2h, K, nch, part_k);
 }
-
-void launch_sd_lambda(Ctx &cx, int nst, const double *m03, const double *m45, double *lam) {
-  hipLaunchKernelGGL(k_sd_lambda, dim3((unsigned)((nst + kThreads - 1) / kThreads)), dim3(kThreads), 0, cx.stream,
-                     m03, m45, nst, lam);
-  INQX_HIP(hipGetLastError());
+void launch_sd_cross(Ctx &cx, int prec, int nst, long K, const void *phi, const void *res, const void *hres,
+                     double *part) {
+  SD_LAUNCH("sd_cross", k_sd_cross<T>, (const cplx<T> *)phi, (const cplx<T> *)res, (const cplx<T> *)hres, K, nch, part);
 }
-
 void launch_sd_update(Ctx &cx, int prec, int nst, long K, void *phi, void *hphi, const void *res, const void *hres,
-                      const double *lam) {
-  ProfScope ps(cx, "sd_update");
-  if (prec == INQX_FP64)
-    hipLaunchKernelGGL(k_sd_update<double>, point_grid(nst, K), dim3(kThreads), 0, cx.stream, (cplx<double> *)phi,
-                       (cplx<double> *)hphi, (const cplx<double> *)res, (const cplx<double> *)hres, lam, K);
-  else
-    hipLaunchKernelGGL(k_sd_update<float>, point_grid(nst, K), dim3(kThreads), 0, cx.stream, (cplx<float> *)phi,
-                       (cplx<float> *)hphi, (const cplx<float> *)res, (const cplx<float> *)hres, lam, K);
-  INQX_HIP(hipGetLastError());
+                      const double *part_m, const double *part_e, double vol, double *part_out) {
+  SD_LAUNCH("sd_update", k_sd_update<T>, (cplx<T> *)phi, (cplx<T> *)hphi, (const cplx<T> *)res, (const cplx<T> *)hres, K,
+            nch, part_m, part_e, vol, part_out);
 }
 
 }  // namespace inqx

@@ -363,18 +363,19 @@ void launch_overlap_diagonal(Ctx &cx, int prec, int n, long K, double vol, const
 void launch_density_add(Ctx &cx, int prec, const void *phi, const double *occ, int nst, long N, int ncomp,
                         int ispin, double *den);
 // eigensolver.hip: per-state passes of steepest descent and the TPA
-// preconditioner over band-major sphere states [nst][K].  Dots: out[s][k] =
-// vol sum_G w conj(a_k) b_k as (re, im), n <= 4 pairs, w applied to the pairs
-// in wmask; part holds sd_dots_partial_bytes(nst, K).
-size_t sd_dots_partial_bytes(int nst, long K);
-void launch_sd_dots(Ctx &cx, int prec, int nst, long K, int n, const void *const *a, const void *const *b,
-                    const double *w, int wmask, double vol, double *part, double *out);
+// preconditioner over band-major sphere states.  Partial sums of a pass are kept
+// per (state, chunk of 4096 points): part[(s nch + c) N + k], N = 4 (energy), 2
+// (tpa) or 8 (cross) doubles, nch = sd_chunks(K); vol multiplies the sums.
+int sd_chunks(long K);
+void launch_sd_energy(Ctx &cx, int prec, int nst, long K, const void *phi, const void *hphi, double *part);
+void launch_tpa_sums(Ctx &cx, int prec, int nst, long K, const void *res, const double *g2h, double *part);
 void launch_sd_residual(Ctx &cx, int prec, int nst, long K, const void *phi, const void *hphi, void *res,
-                        const double *en);
-void launch_tpa_scale(Ctx &cx, int prec, int nst, long K, void *res, const double *g2h, const double *kn);
-void launch_sd_lambda(Ctx &cx, int nst, const double *m03, const double *m45, double *lam);
+                        const double *part_e, double vol, const double *g2h, double *part_k);
+void launch_tpa_scale(Ctx &cx, int prec, int nst, long K, void *res, const double *g2h, const double *part_k);
+void launch_sd_cross(Ctx &cx, int prec, int nst, long K, const void *phi, const void *res, const void *hres,
+                     double *part);
 void launch_sd_update(Ctx &cx, int prec, int nst, long K, void *phi, void *hphi, const void *res, const void *hres,
-                      const double *lam);
+                      const double *part_m, const double *part_e, double vol, double *part_out);
 // exx_kernels.hip: batched pair-density Poisson solves on real-space arrays in
 // state-major layout [n][N].  With hf: for every chunk entry jj (hf index
 // j = jlist[jj]) and state i, rho = conj(hf_j) phi_i -> Poisson -> w_i +=
