@@ -668,7 +668,7 @@ static void tune_cache_write(const char *path, const std::string &key, int xw, i
   if (!path || !*path) return;
   FILE *f = std::fopen(path, "a");
   if (!f) return;  // an unwritable cache only costs the next run a search
-  std::fprintf(f, "%s %d %d %.6f\n", key.c_str(), xw, pb, ms);
+  std::fprintf(f, "%s %d %d %.9g\n", key.c_str(), xw, pb, ms);  // microseconds and below count
   std::fclose(f);
 }
 

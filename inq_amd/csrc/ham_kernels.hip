@@ -1137,14 +1137,90 @@ void build_kb_tables(inqx_ham_s *h) {
       base += 64L * rows;
       kb.maxchunk = std::max(kb.maxchunk, rows);
     }
+    // small grids (small_grid.hip): the entries by group at their offsets in the padded cube
+    if (dev && small_grid(g.n)) {
+      auto offset = [&](const Mem &m) {
+        const int L = m.tile * kTile + m.lane;
+        return (m.i0 * g.n[1] + L / g.n[2]) * (g.n[2] + 1) + L % g.n[2];
+      };
+      std::vector<std::vector<size_t>> by(kb.natoms);
+      for (size_t k = 0; k < mem.size(); ++k) by[mem[k].a].push_back(k);
+      std::vector<int> row(kb.natoms + 1, 0), off;
+      std::vector<float> v32;
+      std::vector<double> v64;
+      std::vector<float> spos;
+      for (int a = 0; a < kb.natoms; ++a) {
+        row[a] = (int)(off.size() / 64);
+        // the groups of a projector list the sphere's points in the same order
+        std::sort(by[a].begin(), by[a].end(), [&](size_t x, size_t y) { return mem[x].p < mem[y].p; });
+        for (size_t k : by[a]) {
+          off.push_back(offset(mem[k]));
+          for (int q = 0; q < kMaxNlm; ++q) {
+            v32.push_back(eb32[kMaxNlm * k + q]);
+            v64.push_back(eb64[kMaxNlm * k + q]);
+          }
+          for (int q = 0; q < 4; ++q) spos.push_back(epos[4 * k + q]);
+        }
+        while (off.size() % 64) {  // padding: offset -1, zero projector values
+          off.push_back(-1);
+          v32.insert(v32.end(), kMaxNlm, 0.0f);
+          v64.insert(v64.end(), kMaxNlm, 0.0);
+          spos.insert(spos.end(), 4, 0.0f);
+        }
+      }
+      row[kb.natoms] = (int)(off.size() / 64);
+      kb.sg_nrec = (long)off.size();
+      // classes of projectors that share no point, each projector in the first that takes it
+      std::vector<std::vector<char>> used;
+      std::vector<std::vector<int>> cls;
+      bool twice = false;
+      for (int a = 0; a < kb.natoms; a += sib[2 * a + 1]) {
+        std::vector<int> pts;
+        for (size_t k : by[a]) pts.push_back(offset(mem[k]));
+        std::vector<int> s = pts;
+        std::sort(s.begin(), s.end());
+        if (std::unique(s.begin(), s.end()) != s.end()) twice = true;
+        size_t c = 0;
+        for (; c < cls.size(); ++c)
+          if (std::none_of(pts.begin(), pts.end(), [&](int o) { return used[c][o] != 0; })) break;
+        if (c == cls.size()) {
+          cls.emplace_back();
+          used.emplace_back((size_t)g.n[0] * g.n[1] * (g.n[2] + 1), 0);
+        }
+        cls[c].push_back(a);
+        for (int o : pts) used[c][o] = 1;
+      }
+      std::vector<int> item, first(1, 0);
+      for (auto &list : cls) {
+        for (int a : list)
+          for (int r = row[a]; r < row[a + 1]; ++r) {
+            item.push_back(r);
+            item.push_back(a);
+            item.push_back(sib[2 * a + 1]);
+            item.push_back(row[a + 1] - row[a]);
+          }
+        first.push_back((int)(item.size() / 4));
+      }
+      kb.sg_classes = twice ? 0 : (int)cls.size();
+      upload(kb.sg_row, row, st);
+      upload(kb.sg_off, off, st);
+      kb.pos_host[1].swap(spos);
+      kb.pos[1].release();
+      upload(kb.sg_b32, v32, st);
+      upload(kb.sg_b64, v64, st);
+      upload(kb.sg_item, item, st);
+      upload(kb.sg_class, first, st);
+      INQX_HIP(hipStreamSynchronize(st));
+    }
     ent_cs.swap(cs2);
     eb32.swap(b32);
     eb64.swap(b64);
     epos.swap(pos2);
   }
   kb.nent = (long)ent_cs.size() / 2;
+  kb.pos_host[0].swap(epos);
+  kb.pos[0].release();
   ++kb.gen;
-  kb.pos_host = epos;
   std::vector<int> atom_slots(kb.natoms + 1, 0), atom_slot_list;
   for (int a = 0; a < kb.natoms; ++a) {
     atom_slots[a] = (int)atom_slot_list.size();
@@ -1197,6 +1273,15 @@ void ensure_basis_device(inqx_ham_s *h, Basis &b) {
         lw[q] = (Grid::sym(y, g.n[1]) - ss[4] + 1) * n2p + z;
       }
     }
+    std::vector<int> co, cr;  // offsets in the padded cube of a small grid
+    if (small_grid(g.n)) {
+      for (long i = 0; i < b.npw; ++i) co.push_back(b.gidx[i] / g.n[2] * n2p + b.gidx[i] % g.n[2]);
+      for (long i = 0; i < b.npw; ++i)
+        if (i == 0 || b.gidx[i] / g.n[2] != b.gidx[i - 1] / g.n[2]) cr.push_back(b.gidx[i] / g.n[2] * n2p);
+      b.ncube_rows = (int)cr.size();
+      upload(b.d_cube_off, co, st);
+      upload(b.d_cube_rows, cr, st);
+    }
     upload(b.d_slot_seg, b.slot_seg, st);
     upload(b.d_rows, b.rows, st);
     upload(b.d_pw_lw, lw, st);
@@ -1224,32 +1309,63 @@ void ensure_basis_device(inqx_ham_s *h, Basis &b) {
   }
 }
 
-// exp(+i (k+A).r_e) of every KB entry e for this basis' k and the current A,
-// with r_e the entry's float contravariant position as the reference keeps it
-// (projector_all.hpp:123,284): the phase depends on (k + A, entry) only, so it
-// is tabulated once instead of evaluated per (entry, state) in the x passes
-static void ensure_phase_table(inqx_ham_s *h, Basis &b) {
-  const KBTables &kb = h->kb;
-  if (b.ph_gen == kb.gen && b.ph_A[0] == h->A[0] && b.ph_A[1] == h->A[1] && b.ph_A[2] == h->A[2]) return;
-  INQX_CHECK(b.pinned == 0, INQX_ERR_STATE, "basis tables are pinned by a captured propagation graph");
-  const long nent = kb.nent;
-  std::vector<double> p64(2 * (size_t)std::max(1L, nent));
-  std::vector<float> p32(2 * (size_t)std::max(1L, nent));
-  const double kk[3] = {b.kcov[0] + h->A[0], b.kcov[1] + h->A[1], b.kcov[2] + h->A[2]};
-  for (long e = 0; e < nent; ++e) {
-    const float *r = &kb.pos_host[4 * (size_t)e];
-    const double arg = kk[0] * (double)r[0] + kk[1] * (double)r[1] + kk[2] * (double)r[2];
-    p64[2 * e] = std::cos(arg);
-    p64[2 * e + 1] = std::sin(arg);
-    p32[2 * e] = (float)p64[2 * e];
-    p32[2 * e + 1] = (float)p64[2 * e + 1];
+// exp(+i (k+A).r_e) of every KB record e for this basis' k and the current A,
+// with r_e the record's float contravariant position as the reference keeps it
+// (projector_all.hpp:123,284): the phase depends on (k + A, record) only, so it
+// is tabulated once per basis instead of evaluated per (record, state) in the
+// passes; first application of 128 blocks at 24^3 with the
+// tables from the host, two allocations and a wait each: 10.7 ms, now 0.65 ms
+template <typename T>
+__global__ void __launch_bounds__(256) k_phase_table(const float4 *pos, int n, double k0, double k1, double k2,
+                                                     cplx<T> *out) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  const float4 r = pos[e];
+  const double arg = k0 * (double)r.x + k1 * (double)r.y + k2 * (double)r.z;
+  double s, c;
+  sincos(arg, &s, &c);
+  gw(out)[e] = cplx<T>{(T)c, (T)s};
+}
+
+// the tables of the blocks with k + A != 0, in the x passes' record order or in
+// that of small_grid.hip.  The missing ones of a launch share one allocation (a
+// hipMalloc each was most of a batch's first application) and one wait, as a table
+// outlives a change of the context's stream.
+template <typename T>
+static void ensure_phase_tables(inqx_ham_s *h, int nblocks, Basis *const *bases, bool small) {
+  KBTables &kb = h->kb;
+  const int w = small ? 1 : 0, prec = std::is_same<T, double>::value ? INQX_FP64 : INQX_FP32;
+  const long n = small ? kb.sg_nrec : kb.nent;
+  std::vector<Basis *> todo;
+  for (int i = 0; i < nblocks; ++i) {
+    Basis &b = *bases[i];
+    const Basis::PhaseTable &t = b.ph[w][prec];
+    if (b.kcov[0] + h->A[0] == 0.0 && b.kcov[1] + h->A[1] == 0.0 && b.kcov[2] + h->A[2] == 0.0) continue;
+    if (t.gen == kb.gen && t.A[0] == h->A[0] && t.A[1] == h->A[1] && t.A[2] == h->A[2]) continue;
+    INQX_CHECK(b.pinned == 0, INQX_ERR_STATE, "basis tables are pinned by a captured propagation graph");
+    if (std::find(todo.begin(), todo.end(), &b) == todo.end()) todo.push_back(&b);
   }
-  hipStream_t st = h->ctx->c.stream;
-  upload(b.d_ph64, p64, st);
-  upload(b.d_ph32, p32, st);
-  INQX_HIP(hipStreamSynchronize(st));
-  b.ph_gen = kb.gen;
-  for (int d = 0; d < 3; ++d) b.ph_A[d] = h->A[d];
+  if (todo.empty()) return;
+  if (!kb.pos[w].p) upload(kb.pos[w], kb.pos_host[w], h->ctx->c.stream);
+  const size_t per = (std::max(1L, n) * sizeof(cplx<T>) + 255) / 256 * 256;
+  auto store = std::make_shared<DevMem>();
+  store->ensure(per * todo.size());
+  for (size_t i = 0; i < todo.size(); ++i) {
+    Basis &b = *todo[i];
+    Basis::PhaseTable &t = b.ph[w][prec];
+    t.store = store;
+    t.p = store->as<char>() + per * i;
+    t.gen = -1;
+    if (n > 0) {
+      hipLaunchKernelGGL(k_phase_table<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->ctx->c.stream,
+                         kb.pos[w].as<float4>(), (int)n, b.kcov[0] + h->A[0], b.kcov[1] + h->A[1],
+                         b.kcov[2] + h->A[2], static_cast<cplx<T> *>(t.p));
+      INQX_HIP(hipGetLastError());
+    }
+    t.gen = kb.gen;
+    for (int d = 0; d < 3; ++d) t.A[d] = h->A[d];
+  }
+  INQX_HIP(hipStreamSynchronize(h->ctx->c.stream));
 }
 
 void ensure_workspace(inqx_ham_s *h, Basis &b, int nst, int prec) {
@@ -1278,7 +1394,8 @@ struct LaunchKey {
 struct LaunchData {
   DevMem desc;  // SphereBlock array followed by 4 prefix arrays
   int total_plane = 0, total_x = 0, total_red = 0;
-  size_t off_pref[3] = {0, 0, 0};
+  bool small = false;                // one work-group per state (small_grid.hip): total_x states
+  size_t off_pref[3] = {0, 0, 0}, off_items = 0;
   int nwave = 4;
   int mode = 0;                      // ApplyOpts::mode
   int total_line = 0, ntile_line = 0;  // line passes of the transform modes
@@ -1589,6 +1706,12 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
     INQX_CHECK(opts->rs != nullptr, INQX_ERR_ARG, "transform without real-space arrays");
   }
   const bool has_kb = mode == 0 && h->kb.natoms > 0;
+  // a cube that fits the LDS runs as one work-group per state, whatever the number
+  // of states: fewer than the CUs leave some idle, but the five passes they would
+  // run instead are launch and latency bound there (16 states at 20^3 complex128
+  // 39 us against 25; 1024 states 190 against 97).  The energy record needs the x passes' dipole sums.
+  const bool small = mode == 0 && !opts->observables && small_grid_fits(g.n, prec, has_kb ? h->kb.natoms : 0) &&
+                     (!has_kb || h->kb.sg_classes > 0);
   LaunchKey key;
   key.k.push_back((uintptr_t)prec);
   key.k.push_back((uintptr_t)mode);
@@ -1598,12 +1721,10 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
   key.k.push_back((uintptr_t)h->plane_batch[prec]);
   if (mode != 0)
     for (int i = 0; i < nblocks; ++i) key.k.push_back((uintptr_t)opts->rs[i]);
+  if (has_kb) ensure_phase_tables<T>(h, nblocks, bases, small);
   for (int i = 0; i < nblocks; ++i) {
     ensure_basis_device(h, *bases[i]);
     ensure_workspace(h, *bases[i], nst[i], prec);
-    const double *kc = bases[i]->kcov;
-    const bool gamma_i = kc[0] + h->A[0] == 0.0 && kc[1] + h->A[1] == 0.0 && kc[2] + h->A[2] == 0.0;
-    if (has_kb && !gamma_i) ensure_phase_table(h, *bases[i]);
     key.k.push_back((uintptr_t)bases[i]);
     key.k.push_back((uintptr_t)nst[i]);
     key.k.push_back((uintptr_t)psi[i]);
@@ -1612,7 +1733,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
     key.k.push_back((uintptr_t)(opts->acc1 ? opts->acc1[i] : nullptr));
     key.k.push_back((uintptr_t)(opts->acc2 ? opts->acc2[i] : nullptr));
     key.k.push_back((uintptr_t)(opts->acc_wide ? 1 : 0));
-    key.k.push_back((uintptr_t)(prec == INQX_FP64 ? bases[i]->d_ph64.p : bases[i]->d_ph32.p));
+    key.k.push_back((uintptr_t)bases[i]->ph[small ? 1 : 0][prec].p);
   }
   key.k.push_back((uintptr_t)(opts->write_h ? 1 : 0));
   key.k.push_back((uintptr_t)(opts->observables ? 1 : 0));
@@ -1688,6 +1809,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
       ld->xlds_project = xp.wave0 + nw * xp.wave_bytes;
     }
     ld->nwave = nw;
+    ld->small = small;
     const double *Afull = h->A;
     for (int i = 0; i < nblocks; ++i) {
       Basis &B = *bases[i];
@@ -1705,6 +1827,9 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
       d.rs = mode != 0 ? reinterpret_cast<cplx<T> *>(opts->rs[i]) : nullptr;
       d.rs_layout = opts->rs_layout;
       d.accumulate = opts->accumulate ? 1 : 0;
+      d.cube_off = B.d_cube_off.as<int>();
+      d.cube_rows = B.d_cube_rows.as<int>();
+      d.ncube_rows = B.ncube_rows;
       d.acc1 = opts->acc1 ? reinterpret_cast<cplx<T> *>(opts->acc1[i]) : nullptr;
       d.acc2 = opts->acc2 ? reinterpret_cast<cplx<T> *>(opts->acc2[i]) : nullptr;
       d.acc_wide = opts->acc_wide && !std::is_same<T, double>::value ? 1 : 0;
@@ -1719,11 +1844,13 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
       d.m_lo = B.m_lo;
       for (int k = 0; k < 3; ++k) d.kcov[k] = B.kcov[k] + Afull[k];
       d.gamma = (d.kcov[0] == 0.0 && d.kcov[1] == 0.0 && d.kcov[2] == 0.0) ? 1 : 0;
-      d.kbph = (has_kb && !d.gamma)
-                   ? (prec == INQX_FP64 ? (const cplx<T> *)B.d_ph64.p : (const cplx<T> *)B.d_ph32.p)
-                   : nullptr;
+      const void *ph = has_kb && !d.gamma ? B.ph[small ? 1 : 0][prec].p : nullptr;
+      d.kbph = small ? nullptr : static_cast<const cplx<T> *>(ph);
+      d.sgph = small ? static_cast<const cplx<T> *>(ph) : nullptr;
       pp[i + 1] = pp[i] + d.nslot * ((nst[i] + plane_p - 1) / plane_p);
-      if (mode == 0)
+      if (ld->small)
+        px[i + 1] = px[i] + nst[i];
+      else if (mode == 0)
         px[i + 1] = px[i] + x_tiles_padded(h->kb.ntile) * ((nst[i] + nw - 1) / nw);
       else
         px[i + 1] = px[i] + ld->ntile_line * ((nst[i] + 3) / 4);
@@ -1741,12 +1868,21 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
     ld->off_pref[0] = bytes;
     ld->off_pref[1] = bytes + sizeof(int) * (nblocks + 1);
     ld->off_pref[2] = bytes + 2 * sizeof(int) * (nblocks + 1);
-    size_t tot = bytes + 3 * sizeof(int) * (nblocks + 1);
+    ld->off_items = (bytes + 3 * sizeof(int) * (nblocks + 1) + 15) & ~size_t(15);
+    std::vector<int> items;  // small grids: block and state of every work-group
+    if (ld->small)
+      for (int i = 0; i < nblocks; ++i)
+        for (int s = 0; s < nst[i]; ++s) {
+          items.push_back(i);
+          items.push_back(s);
+        }
+    size_t tot = ld->off_items + sizeof(int) * items.size();
     std::vector<char> host(tot);
     std::memcpy(host.data(), blk.data(), sizeof(SphereBlock<T>) * nblocks);
     std::memcpy(host.data() + ld->off_pref[0], pp.data(), sizeof(int) * (nblocks + 1));
     std::memcpy(host.data() + ld->off_pref[1], px.data(), sizeof(int) * (nblocks + 1));
     std::memcpy(host.data() + ld->off_pref[2], pr.data(), sizeof(int) * (nblocks + 1));
+    if (!items.empty()) std::memcpy(host.data() + ld->off_items, items.data(), sizeof(int) * items.size());
     ld->desc.ensure(tot);
     INQX_HIP(hipMemcpyAsync(ld->desc.p, host.data(), tot, hipMemcpyHostToDevice, h->ctx->c.stream));
     INQX_HIP(hipStreamSynchronize(h->ctx->c.stream));
@@ -1781,6 +1917,11 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
   for (int r = 0; r < 3; ++r)
     for (int c = 0; c < 3; ++c) hd.lat[3 * r + c] = g.a[r][c];
   const double cf[4] = {opts->c1r, opts->c1i, opts->c2r, opts->c2i};
+  if (ld.small) {
+    launch_small_apply<T>(h, ld.desc.as<SphereBlock<T>>(),
+                          reinterpret_cast<const int *>(ld.desc.as<char>() + ld.off_items), ld.total_x, has_kb, cf);
+    return;
+  }
   dispatch_passes<T>(g.n[0], g.n[1], g.n[2], h, ld, nblocks, hd, cf);
 }
 

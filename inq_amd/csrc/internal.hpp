@@ -185,7 +185,18 @@ struct KBTables {
   DevMem atom_slot_list;
   DevMem coeff;       // [natoms][kMaxNlm][kCoeffCols] double: group rows of the projector's D
   DevMem group_sib;   // [natoms] int2: first group of the group's projector, number of groups
-  std::vector<float> pos_host;  // [nent][4] the entry positions, for the per-basis phase tables
+  // the same records for grids whose cube fits the LDS (small_grid.hip): by group,
+  // each padded to rows of 64 (LDS offset; projector values; position), and the
+  // rows of the projectors (first group's row, first group, groups, rows between
+  // groups) in classes of projectors that share no point.  sg_classes = 0: a
+  // projector's sphere holds a point twice (periodic images), not offered
+  DevMem sg_row, sg_off, sg_b32, sg_b64, sg_item, sg_class;
+  int sg_classes = 0;
+  long sg_nrec = 0;
+  // float4 position of every record of the two orders, for the per-basis phase
+  // tables; on the device from the first table on
+  std::vector<float> pos_host[2];
+  DevMem pos[2];
 };
 
 // ------------------------------------------------------------------ device block descriptor
@@ -217,6 +228,10 @@ template <typename T> struct SphereBlock {
   C *rs;               // real-space states, [nst][N] (rs_layout 0) or [N][nst] (1)
   int rs_layout;
   int accumulate;      // plane_forward adds into hpsi instead of storing
+  const C *sgph;         // small grids: the KB phases in their record order
+  const int *cube_off;   // small grids: [npw] LDS offset of each sphere point in the cube,
+  const int *cube_rows;  // LDS offsets of the rows that hold sphere points
+  int ncube_rows;
 };
 
 // optional work fused into one H application
@@ -250,14 +265,19 @@ struct Basis {
   int nwin_max = 0;           // longest row window of a plane
   std::vector<int> rows, pw_yz;
   DevMem d_slot_seg, d_rows, d_pw_lw, d_kin64, d_kin32;
+  DevMem d_cube_off, d_cube_rows;  // small grids (small_grid.hip)
+  int ncube_rows = 0;
   DevMem d_g2h;  // (1/2)|G|^2 per sphere point, FP64, no k shift (preconditioner)
   DevMem d_gidx; // flattened FFT index per sphere point (layout conversions), on first use
   double kin_A[3] = {1e300, 0, 0};  // A for which d_kin* were built
-  // KB phases exp(+i (k+A).r_e) per KB entry e (FP64 and FP32 copies), built for
-  // the vector potential ph_A and the KB table generation ph_gen
-  DevMem d_ph64, d_ph32;
-  double ph_A[3] = {1e300, 0, 0};
-  int ph_gen = -1;
+  // KB phases exp(+i (k+A).r_e) per KB record e, built for the vector potential A
+  // and the KB table generation gen
+  struct PhaseTable {
+    std::shared_ptr<DevMem> store;  // shared by the blocks of one launch
+    void *p = nullptr;
+    double A[3] = {1e300, 0, 0};
+    int gen = -1;
+  } ph[2][2];  // [record order: x passes, small_grid.hip][precision]
   // workspaces per precision
   DevMem t1[2], partial[2], dp[2], dps[2], proj[2], dip, dots, hn[2][2], save[2];
   int ws_nst[2] = {0, 0};
@@ -343,6 +363,12 @@ void launch_rect_inverse(Ctx &cx, const SphereBlock<T> *blk, const int *pref, in
 template <typename T>
 void launch_rect_forward(Ctx &cx, const SphereBlock<T> *blk, const int *pref, int nblocks, int total, int pb,
                          int pstr, int n1, int n2, const double *cf);
+// small_grid.hip: H on blocks whose cube fits one work-group's LDS, a work-group per state
+bool small_grid(const int *n);
+bool small_grid_fits(const int *n, int prec, int natoms);
+template <typename T>
+void launch_small_apply(inqx_ham_s *h, const SphereBlock<T> *blk, const int *items, int total, bool has_kb,
+                        const double *cf);
 // linalg.hip
 void launch_overlap(Ctx &cx, int prec, int n1, int n2, long K, const void *A, const void *B, double vol, double *S,
                     DevMem &partial);
