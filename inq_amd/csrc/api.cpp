@@ -1220,14 +1220,21 @@ int inqx_density_add(inqx_ham h, inqx_basis bs, int nst, int precision, const vo
   API_BEGIN
   check_transform(h, bs, nst, precision, INQX_STATE_MAJOR);
   INQX_CHECK(phi && occ && density && ncomp > 0 && ispin >= 0 && ispin < ncomp, INQX_ERR_ARG, "bad arguments");
-  const size_t per = (precision == INQX_FP64 ? 16 : 8) * (size_t)h->g.N;
-  h->exx_phi.ensure(per * nst);
-  transform_impl(h, bs->b, nst, precision, 1, phi, h->exx_phi.p, INQX_STATE_MAJOR, false, nullptr);
-  std::vector<double> oc(occ, occ + nst);
-  upload(h->dens_occ, oc, ctx->c.stream);
-  INQX_HIP(hipStreamSynchronize(ctx->c.stream));
-  launch_density_add(ctx->c, precision, h->exx_phi.p, h->dens_occ.as<double>(), nst, h->g.N, ncomp, ispin,
-                     (double *)density);
+  h->dens_occ.ensure(sizeof(double) * (size_t)nst);
+  launch_put_occ(ctx->c, occ, nst, h->dens_occ.as<double>());
+  DensityOut d;
+  d.occ = h->dens_occ.as<double>();
+  d.ncomp = ncomp;
+  d.ispin = ispin;
+  d.den = (double *)density;
+  d.work = &h->dens_work;
+  ApplyOpts o;
+  o.mode = 3;
+  o.density = &d;
+  Basis *bb = &bs->b;
+  void *pout = nullptr;
+  if (precision == INQX_FP64) launch_apply<double>(h, 1, &bb, &nst, &phi, &pout, &o);
+  else launch_apply<float>(h, 1, &bb, &nst, &phi, &pout, &o);
   API_END(ctx)
 }
 

@@ -599,21 +599,24 @@ __global__ void __launch_bounds__(256) k_real_to_cplx(const double *r, double2 *
   if (p < N) gw(c)[p] = double2{gp(r)[p], 0.0};
 }
 
-// vh = Re(c); part[chunk] = sum over the chunk of rho vh (fixed tree order)
-__global__ void __launch_bounds__(256) k_hartree_out(const double2 *c, const double *rho, double *vh, long N,
+// vh = Re(c); part[chunk] = sum over the chunk of rho vh (fixed tree order).  A
+// chunk's loads are a chain of dependent round trips: 16 waves on it, 8 trips each
+// (4 waves and 32 trips: 18.6 us at 72^3, now 8.2)
+constexpr int kHThreads = 1024;
+__global__ void __launch_bounds__(kHThreads) k_hartree_out(const double2 *c, const double *rho, double *vh, long N,
                                                      double *part) {
-  __shared__ double red[256];
+  __shared__ double red[kHThreads];
   const int tid = threadIdx.x;
   const long p0 = (long)blockIdx.x * kHChunk;
   double acc = 0.0;
-  for (long p = p0 + tid; p < p0 + kHChunk && p < N; p += 256) {
+  for (long p = p0 + tid; p < p0 + kHChunk && p < N; p += kHThreads) {
     const double v = gp(c)[p].x;
     if (vh) gw(vh)[p] = v;
     acc += gp(rho)[p] * v;
   }
   red[tid] = acc;
   __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
+  for (int h = kHThreads / 2; h > 0; h >>= 1) {
     if (tid < h) red[tid] += red[tid + h];
     __syncthreads();
   }
@@ -699,7 +702,7 @@ void launch_hartree(inqx_ham_s *h, const double *rho, double *vh, void *work, do
   launch_pairs(h, INQX_FP64, a);
   {
     ProfScope ps(cx, "hartree_out");
-    hipLaunchKernelGGL(k_hartree_out, dim3((unsigned)hartree_chunks(N)), dim3(256), 0, cx.stream,
+    hipLaunchKernelGGL(k_hartree_out, dim3((unsigned)hartree_chunks(N)), dim3(kHThreads), 0, cx.stream,
                        reinterpret_cast<const double2 *>(work), rho, vh, N, part);
   }
   INQX_HIP(hipGetLastError());

@@ -1614,6 +1614,7 @@ static void run_passes(inqx_ham_s *h, LaunchData &ld, int nblocks, const HamDev 
     return;
   }
   plane_inv();
+  if (ld.mode == 3) return;  // launch_apply runs the density's line pass
   if (ld.mode == 1) {  // sphere -> real space
     const int grid_l = ld.total_line;
     ProfScope ps(cx, f64 ? "line_to_real_f64" : "line_to_real_f32");
@@ -1702,7 +1703,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
                      std::to_string(h->ncomp) + ")");
     if (!h->kb.built) build_kb_tables(h);
     if (prec == INQX_FP32 && !h->v32.p) INQX_CHECK(false, INQX_ERR_STATE, "potential not uploaded");
-  } else {
+  } else if (mode != 3) {
     INQX_CHECK(opts->rs != nullptr, INQX_ERR_ARG, "transform without real-space arrays");
   }
   const bool has_kb = mode == 0 && h->kb.natoms > 0;
@@ -1719,7 +1720,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
   key.k.push_back((uintptr_t)(opts->accumulate ? 1 : 0));
   key.k.push_back((uintptr_t)h->xwaves[prec]);
   key.k.push_back((uintptr_t)h->plane_batch[prec]);
-  if (mode != 0)
+  if (mode == 1 || mode == 2)
     for (int i = 0; i < nblocks; ++i) key.k.push_back((uintptr_t)opts->rs[i]);
   if (has_kb) ensure_phase_tables<T>(h, nblocks, bases, small);
   for (int i = 0; i < nblocks; ++i) {
@@ -1824,7 +1825,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
       d.rows = B.d_rows.as<int>();
       d.pw_lds = B.d_pw_lw.as<int>();
       d.kin = mode == 2 ? nullptr : prec == INQX_FP64 ? (const T *)B.d_kin64.p : (const T *)B.d_kin32.p;
-      d.rs = mode != 0 ? reinterpret_cast<cplx<T> *>(opts->rs[i]) : nullptr;
+      d.rs = mode == 1 || mode == 2 ? reinterpret_cast<cplx<T> *>(opts->rs[i]) : nullptr;
       d.rs_layout = opts->rs_layout;
       d.accumulate = opts->accumulate ? 1 : 0;
       d.cube_off = B.d_cube_off.as<int>();
@@ -1923,6 +1924,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
     return;
   }
   dispatch_passes<T>(g.n[0], g.n[1], g.n[2], h, ld, nblocks, hd, cf);
+  if (mode == 3) launch_line_density<T>(h, *bases[0], nst[0], *opts->density);
 }
 
 int dots_chunks(int npw) { return (npw + kDotChunk - 1) / kDotChunk; }

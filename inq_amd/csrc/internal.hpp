@@ -235,6 +235,15 @@ template <typename T> struct SphereBlock {
 };
 
 // optional work fused into one H application
+// den[N][ncomp] (component ispin) += sum_i occ_i |phi_i|^2; occ on the device, work
+// grows to what the launch needs
+struct DensityOut {
+  const double *occ = nullptr;
+  int ncomp = 1, ispin = 0;
+  double *den = nullptr;
+  DevMem *work = nullptr;
+};
+
 struct ApplyOpts {
   void *const *acc1 = nullptr;  // per block, acc1 += c1 (H psi)
   void *const *acc2 = nullptr;  // per block, acc2 += c2 (H psi)
@@ -243,8 +252,10 @@ struct ApplyOpts {
   bool write_h = true;
   bool observables = false;     // projections and dipole partials into the basis workspaces
   // mode 0: H application; 1: sphere -> real space (psi -> rs, x 1/N);
-  // 2: real space -> sphere (rs -> hpsi, masked forward FFT)
+  // 2: real space -> sphere (rs -> hpsi, masked forward FFT);
+  // 3: one block's density (psi -> *density)
   int mode = 0;
+  const DensityOut *density = nullptr;
   void *const *rs = nullptr;    // per block real-space arrays for modes 1 and 2
   int rs_layout = 0;            // 0: [nst][N], 1: [N][nst]
   bool accumulate = false;      // mode 2: hpsi += result
@@ -326,7 +337,7 @@ struct inqx_ham_s {
   inqx::DevMem exx_phi, exx_hf, exx_w, exx_t, exx_jlist, exx_coef;
   inqx::DevMem exx_wb, exx_occ;  // symmetric pairs: the conjugate-pair accumulator and occupied flags
   // real-space apply and density workspaces (sphere arrays of a full-cube basis, occupations)
-  inqx::DevMem rs_a, rs_b, dens_occ;
+  inqx::DevMem rs_a, rs_b, dens_occ, dens_work;
   inqx::DevMem lay_a, lay_b;  // band-major copies for inqx_ham_apply_layout
   // steepest-descent workspace: H phi, residual, H residual, dot partials and results
   inqx::DevMem sd_states, sd_scal;
@@ -346,6 +357,9 @@ namespace inqx {
 void build_kb_tables(inqx_ham_s *h);
 void invalidate_launch_cache(inqx_ham_s *h);
 void set_capture_keep(std::vector<std::shared_ptr<void>> *keep);
+// density.hip: the line pass of ApplyOpts::mode 3
+void launch_put_occ(Ctx &cx, const double *occ, int nst, double *dev);
+template <typename T> void launch_line_density(inqx_ham_s *h, const Basis &B, int nst, const DensityOut &o);
 template <typename T>
 void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *nst, const void *const *psi,
                   void *const *hpsi, const ApplyOpts *opts = nullptr);
@@ -386,8 +400,6 @@ void launch_fill_zero(Ctx &cx, void *p, size_t bytes);
 void launch_randomize(Ctx &cx, int type, long npoints, int nst, int index, int layout, void *out);
 void launch_overlap_diagonal(Ctx &cx, int prec, int n, long K, double vol, const void *A, const void *B,
                              int normalized, double *out);
-void launch_density_add(Ctx &cx, int prec, const void *phi, const double *occ, int nst, long N, int ncomp,
-                        int ispin, double *den);
 // eigensolver.hip: per-state passes of steepest descent and the TPA
 // preconditioner over band-major sphere states.  Partial sums of a pass are kept
 // per (state, chunk of 4096 points): part[(s nch + c) N + k], N = 4 (energy), 2

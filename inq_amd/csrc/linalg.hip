@@ -989,35 +989,6 @@ void launch_overlap_diagonal(Ctx &cx, int prec, int n, long K, double vol, const
   INQX_HIP(hipGetLastError());
 }
 
-// ------------------------------------------------------------------------ density
-// density[p][ncomp] (component ispin) += sum_i occ_i |phi_i(p)|^2, states
-// state-major [nst][N]; FP64, states summed in order
-template <typename T>
-__global__ void __launch_bounds__(256) k_density_add(const cplx<T> *phi, const double *occ, int nst, long N,
-                                                    int ncomp, int ispin, double *den) {
-  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < N; p += (long)gridDim.x * blockDim.x) {
-    double acc = 0.0;
-    for (int i = 0; i < nst; ++i) {
-      const cplx<T> v = lgp(phi)[(size_t)i * N + p];
-      acc += lgp(occ)[i] * ((double)v.x * v.x + (double)v.y * v.y);
-    }
-    lgw(den)[p * ncomp + ispin] += acc;
-  }
-}
-
-void launch_density_add(Ctx &cx, int prec, const void *phi, const double *occ, int nst, long N, int ncomp,
-                        int ispin, double *den) {
-  const int grid = (int)std::max<long>(1, std::min<long>((N + 255) / 256, (long)cx.num_cu * 16));
-  ProfScope ps(cx, "density_add");
-  if (prec == INQX_FP64)
-    hipLaunchKernelGGL(k_density_add<double>, dim3(grid), dim3(256), 0, cx.stream, (const cplx<double> *)phi, occ,
-                       nst, N, ncomp, ispin, den);
-  else
-    hipLaunchKernelGGL(k_density_add<float>, dim3(grid), dim3(256), 0, cx.stream, (const cplx<float> *)phi, occ,
-                       nst, N, ncomp, ispin, den);
-  INQX_HIP(hipGetLastError());
-}
-
 // ------------------------------------------------------------------------ randomize
 // operations::randomize (src/operations/randomize.hpp:48-70): value (ip, ist)
 // comes from pcg32 (64-bit LCG, XSH-RR output of the pre-step state) seeded

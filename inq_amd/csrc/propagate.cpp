@@ -315,24 +315,26 @@ void release_ks_work(inqx_ham_s *h) { g_ks_work.erase(h); }
 // spin density of every block's sphere states: den[N][ncomp] = sum occ |to_real(phi)|^2
 template <typename T>
 static void blocks_density(inqx_ham_s *h, int nb, Basis *const *bases, const int *nst, void *const *phi,
-                           const double *const *occ, DevMem &rs, double *den) {
+                           const double *const *occ, DevMem &work, double *den) {
   Ctx &cx = h->ctx->c;
   const long N = h->g.N;
   const int prec = std::is_same<T, double>::value ? INQX_FP64 : INQX_FP32;
   launch_fill_zero(cx, den, sizeof(double) * (size_t)N * h->ncomp);
   for (int i = 0; i < nb; ++i) {
     INQX_CHECK(bases[i]->spin < h->ncomp, INQX_ERR_ARG, "a block's spin index has no density component");
-    rs.ensure(sizeof(cplx<T>) * (size_t)nst[i] * N);
+    DensityOut d;
+    d.occ = occ[i];
+    d.ncomp = h->ncomp;
+    d.ispin = bases[i]->spin;
+    d.den = den;
+    d.work = &work;
     ApplyOpts o;
-    o.mode = 1;
-    void *rsp = rs.p;
-    o.rs = &rsp;
-    o.rs_layout = 0;
+    o.mode = 3;
+    o.density = &d;
     const void *pin = phi[i];
     void *pout = nullptr;
     Basis *b = bases[i];
     launch_apply<T>(h, 1, &b, &nst[i], &pin, &pout, &o);
-    launch_density_add(cx, prec, rs.p, occ[i], nst[i], N, h->ncomp, bases[i]->spin, den);
   }
 }
 
