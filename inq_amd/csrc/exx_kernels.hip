@@ -18,8 +18,8 @@
 //                    registers, Poisson kernel, inverse FFT along i0, in place
 //   pair_plane_inv   per (j, plane i0, i): 2-D inverse FFT of the plane of t
 //   pair_reduce      w_i += sum_j coef_j hf_j t_ji in j order (deterministic;
-//                    chunks of j give the same bits); pair_reduce_sym adds the
-//                    conjugate pairs' terms when hf = phi
+//                    chunks of j give the same bits); with hf = phi
+//                    pair_reduce_both also sums the conjugate pairs' terms
 //
 // Planes with n1 != n2 run the 2-D transforms as a column kernel and a row
 // kernel in place in t (pair_cols, pair_rows) instead of pair_plane_fwd/inv.
@@ -44,7 +44,7 @@ template <typename T> struct PairDev {
   int n0, n1, n2;      // grid (the plane passes take n0 at run time, the line pass n1 and n2)
   // symmetric pairs (hf = phi, no shift): pair (j, i) with i occupied and
   // i > j is not solved; its potential is conj of pair (i, j)'s, added into
-  // wb by k_pair_reduce_sym.  occ: [nst] 1 for an occupied state, or null.
+  // wb by k_pair_reduce_both.  occ: [nst] 1 for an occupied state, or null.
   const int *occ;
   cplx<T> *wb;         // [nst][N]
   T b[3][3];           // reciprocal lattice vectors (rows, cartesian, 2 pi included)
@@ -96,6 +96,18 @@ __device__ __forceinline__ void lds_row_fft_split(C *lds, int r, int q) {
   }
 }
 
+// pair plane (chunk entry jj, plane i0, state i) of work-group wg in the passes that
+// form the pair densities: planes outermost, so that plane i0 of every state stays
+// in the caches while all pairs read it (5.3 MB of 128 states at 72^3 complex64,
+// an eighth of the states on each XCD; with the pairs outermost each hf state
+// read the whole block of 382 MB again: 13.4 -> 11.7 ms for 8256 pairs)
+__device__ __forceinline__ void pair_product_item(int wg, int nst, int nj, int &jj, int &i0, int &i) {
+  i = wg % nst;
+  const int r = wg / nst;
+  jj = r % nj;
+  i0 = r / nj;
+}
+
 template <int N> __host__ __device__ constexpr int symi(int i) { return i >= (N + 1) / 2 ? i - N : i; }
 
 // reciprocal: the hardware approximation (1 ulp) for the complex64 path, an
@@ -120,10 +132,8 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_f
   {
     const int wg = blockIdx.x;
     if (wg >= total) return;
-    const int i = wg % d.nst;
-    const int r = wg / d.nst;
-    const int i0 = r % d.n0;
-    const int jj = r / d.n0;
+    int jj, i0, i;
+    pair_product_item(wg, d.nst, d.nj, jj, i0, i);
     if (pair_skipped(d, jj, i)) return;  // uniform over the work-group
     const size_t plane = (size_t)i0 * NP;
     const GAS C *ph = gp(d.phi) + (size_t)i * N + plane;
@@ -307,7 +317,8 @@ __global__ void __launch_bounds__(256) k_pair_cols(PairDev<T> d, int total) {
   const int wg = blockIdx.x;
   if (wg >= total) return;
   int jj, i0, i;
-  pair_plane_item(wg, d.nst, d.n0, jj, i0, i);
+  if (PROD) pair_product_item(wg, d.nst, d.nj, jj, i0, i);
+  else pair_plane_item(wg, d.nst, d.n0, jj, i0, i);
   if (pair_skipped(d, jj, i)) return;  // uniform over the work-group
   const size_t plane = (size_t)i0 * NP;
   GAS C *tp = gw(d.t) + ((size_t)jj * d.nst + i) * N + plane;
@@ -433,7 +444,6 @@ __global__ void __launch_bounds__(256) k_pair_reduce(PairDev<T> d, long nvec) {
   }
   for (int jj = 0; jj < d.nj; ++jj) {
     const int j = gp(d.jlist)[jj];
-    if (d.occ && i > j && gp(d.occ)[i] != 0) continue;  // pair not solved: k_pair_reduce_sym adds it
     const T c = (T)gp(d.coef)[j];
     V x[U], h[U];
 #pragma unroll
@@ -454,56 +464,114 @@ __global__ void __launch_bounds__(256) k_pair_reduce(PairDev<T> d, long nvec) {
   }
 }
 
-// acc += c h conj(t)
-__device__ __forceinline__ void cmac_conj(float4 &a, float c, const float4 &h, const float4 &t) {
-  a.x += c * (h.x * t.x + h.y * t.y);
-  a.y += c * (h.y * t.x - h.x * t.y);
-  a.z += c * (h.z * t.z + h.w * t.w);
-  a.w += c * (h.w * t.z - h.z * t.w);
-}
-__device__ __forceinline__ void cmac_conj(double2 &a, double c, const double2 &h, const double2 &t) {
-  a.x += c * (h.x * t.x + h.y * t.y);
-  a.y += c * (h.y * t.x - h.x * t.y);
-}
+// symmetric mode, both sums from one read of the solved pairs:
+//   w_i  += sum_jj c_j hf_j t[jj][i]           over the pairs solved for state i
+//   wb_j  = sum_{s < j, occupied} c_s phi_s conj(t[jj][s]),
+// the terms of w_j whose pair (j, s) was not solved (its potential is the conjugate
+// of pair (s, j)'s, exchange_operator.hpp:144-160 with real kernels).
+//
+// The bound is the read of t, 3 MB a pair at 72^3 complex64; two kernels, one for
+// each sum, read it twice.  A work-group holds 64 points; wave k holds the states
+// i = base + u kRedWaves + k (u < U): their values and their w sums stay in
+// registers while the rows jj stream by, a row's loads all in flight at once.  The
+// waves' parts of wb_j meet in LDS every kRedRows rows.  w_i is added in jj order
+// and wb_j belongs to one chunk, so splitting the j range into chunks gives the
+// same bits.  128 states, 72^3 complex64 (8256 pairs): 12.9 -> 6.7 ms.
+constexpr int kRedWaves = 8;
+template <typename T> constexpr int red_rows() { return sizeof(T) == 4 ? 8 : 4; }
 
-// symmetric mode: for every chunk entry jj (an occupied state j),
-// wb_j = sum over occupied states s < j, in s order, of c_s phi_s conj(t[jj][s])
-// -- the terms of w_j whose pair (j, s) was not solved (its potential is the
-// conjugate of pair (s, j)'s, exchange_operator.hpp:144-160 with real kernels).
-// Every w_j's terms land in one chunk, so wb needs no accumulation across chunks.
-template <typename T>
-__global__ void __launch_bounds__(256) k_pair_reduce_sym(PairDev<T> d, long nvec) {
-  using V = typename Vec16<T>::type;
-  constexpr int U = 4;
-  const int jj = (int)(blockIdx.x % (unsigned)d.nj);
-  const long v0 = (long)(blockIdx.x / (unsigned)d.nj) * 256 * U + threadIdx.x;
-  const int j = gp(d.jlist)[jj];
-  const GAS V *tv = gp(reinterpret_cast<const V *>(d.t)) + (size_t)jj * d.nst * nvec;
-  const GAS V *hv = gp(reinterpret_cast<const V *>(d.hf));
-  V acc[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) acc[u] = V{};
-  for (int s = 0; s < j; ++s) {
-    if (gp(d.occ)[s] == 0) continue;
-    const T c = (T)gp(d.coef)[s];
-    V x[U], h[U];
+template <typename T, int U>
+__global__ void __launch_bounds__(64 * kRedWaves) k_pair_reduce_both(PairDev<T> d, long N) {
+  using C = cplx<T>;
+  constexpr int W = kRedWaves, R = red_rows<T>();
+  __shared__ C part[R][W][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long p = (long)blockIdx.x * 64 + lane, pc = p < N ? p : N - 1;
+  const unsigned voff = (unsigned)(pc * sizeof(C)), row = (unsigned)(N * sizeof(C));
+  const GAS C *hf = gp(d.hf);
+  for (int base = 0; base < d.nst; base += W * U) {
+    C acc[U], ph[U];
+    unsigned occ = 0, valid = 0;  // bit u: state u of this wave
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const long v = v0 + u * 256;
-      if (v < nvec) {
-        x[u] = tv[(size_t)s * nvec + v];
-        h[u] = hv[(size_t)s * nvec + v];
-      }
+      const int i = base + u * W + wave, ic = i < d.nst ? i : d.nst - 1;
+      if (i < d.nst) valid |= 1u << u;
+      const bool o = i < d.nst && gp(d.occ)[ic] != 0;
+      if (o) occ |= 1u << u;
+      acc[u] = gw(d.w)[(size_t)ic * N + pc];
+      const C x = hf[(size_t)ic * N + pc];
+      const T c = o ? (T)gp(d.coef)[ic] : (T)0;
+      ph[u] = C{c * x.x, c * x.y};
     }
+    for (int r0 = 0; r0 < d.nj; r0 += R) {
+      const int r1 = min(r0 + R, d.nj);
+      for (int jj = r0; jj < r1; ++jj) {
+        const int j = gp(d.jlist)[jj];
+        // states i <= j and i < j of this wave as bits u
+        const int le = j - base - wave;
+        const unsigned mle = le < 0 ? 0u : le / W >= U - 1 ? ~0u : (2u << (le / W)) - 1u;
+        const unsigned mlt = le < 1 ? 0u : (le - 1) / W >= U - 1 ? ~0u : (2u << ((le - 1) / W)) - 1u;
+        const unsigned act = valid & (~occ | mle), conj = occ & mlt;
+        const C *tj = d.t + ((size_t)jj * d.nst + base + wave) * N;
+        C x[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) cmac_conj(acc[u], c, h[u], x[u]);
-  }
-  GAS V *bv = gw(reinterpret_cast<V *>(d.wb)) + (size_t)j * nvec;
+        for (int u = 0; u < U; ++u) {  // a pair that was not solved reads an empty buffer
+          const bool on = (act >> u) & 1u;
+          bload(make_rsrc(on ? tj + (size_t)u * W * N : d.t, on ? row : 0u), voff, 0u, x[u]);
+        }
+        const C h = hf[(size_t)j * N + pc];
+        const T c = (T)gp(d.coef)[j];
+        const C ch{c * h.x, c * h.y};
+        C b{0, 0};
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const long v = v0 + u * 256;
-    if (v < nvec) bv[v] = acc[u];
+        for (int u = 0; u < U; ++u) {
+          if ((act >> u) & 1u) {  // uniform
+            acc[u].x += ch.x * x[u].x - ch.y * x[u].y;
+            acc[u].y += ch.x * x[u].y + ch.y * x[u].x;
+          }
+          if ((conj >> u) & 1u) {
+            b.x += ph[u].x * x[u].x + ph[u].y * x[u].y;
+            b.y += ph[u].y * x[u].x - ph[u].x * x[u].y;
+          }
+        }
+        part[jj - r0][wave][lane] = b;
+      }
+      __syncthreads();
+      // wave k adds row r0 + k of the tile
+      const int jj = r0 + wave;
+      if (wave < R && jj < r1) {
+        const int j = gp(d.jlist)[jj];
+        if (j > base && p < N) {
+          C s = gw(d.wb)[(size_t)j * N + p];
+#pragma unroll
+          for (int k = 0; k < W; ++k) {
+            s.x += part[wave][k][lane].x;
+            s.y += part[wave][k][lane].y;
+          }
+          gw(d.wb)[(size_t)j * N + p] = s;
+        }
+      }
+      __syncthreads();
+    }
+    if (p < N) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if ((valid >> u) & 1u) gw(d.w)[(size_t)(base + u * W + wave) * N + p] = acc[u];
+    }
   }
+}
+
+// states per wave: enough for the block in one pass over the rows (more would be
+// empty loads), at most what the registers hold; further states take further passes
+template <typename T> void launch_pair_reduce_both(Ctx &cx, const PairDev<T> &d, long N) {
+  constexpr int UMAX = sizeof(T) == 4 ? 16 : 8;
+  const dim3 grid((unsigned)((N + 63) / 64)), wg(64 * kRedWaves);
+  const int need = (d.nst + kRedWaves - 1) / kRedWaves;
+  if (need <= 2) hipLaunchKernelGGL((k_pair_reduce_both<T, 2>), grid, wg, 0, cx.stream, d, N);
+  else if (need <= 4) hipLaunchKernelGGL((k_pair_reduce_both<T, 4>), grid, wg, 0, cx.stream, d, N);
+  else if (need <= 8) hipLaunchKernelGGL((k_pair_reduce_both<T, 8>), grid, wg, 0, cx.stream, d, N);
+  else hipLaunchKernelGGL((k_pair_reduce_both<T, UMAX>), grid, wg, 0, cx.stream, d, N);
+  INQX_HIP(hipGetLastError());
 }
 
 // S0: line length along i0; S > 0: square planes S x S (pair_plane_fwd /
@@ -569,22 +637,16 @@ template <typename T, int S0, int S> void run_pairs(inqx_ham_s *h, const PairArg
       pair_planes_rect<T, +1, false>(cx, d, tot1);
   }
   INQX_HIP(hipGetLastError());
-  if (d.hf) {
+  if (d.occ) {
+    ProfScope ps(cx, f64 ? "pair_reduce_both_f64" : "pair_reduce_both_f32");
+    launch_pair_reduce_both<T>(cx, d, g.N);
+  } else if (d.hf) {
     // 16-byte vectors per state: N complex values of 2 sizeof(T) bytes
     const long nvec = (long)g.N * 2 * (long)sizeof(T) / 16;
-    const long per = (nvec + 1023) / 1024;
-    const long tot4 = per * d.nst;
-    {
-      ProfScope ps(cx, f64 ? "pair_reduce_f64" : "pair_reduce_f32");
-      hipLaunchKernelGGL((k_pair_reduce<T>), dim3((unsigned)tot4), dim3(256), 0, cx.stream, d, nvec);
-    }
+    const long tot4 = (nvec + 1023) / 1024 * d.nst;
+    ProfScope ps(cx, f64 ? "pair_reduce_f64" : "pair_reduce_f32");
+    hipLaunchKernelGGL((k_pair_reduce<T>), dim3((unsigned)tot4), dim3(256), 0, cx.stream, d, nvec);
     INQX_HIP(hipGetLastError());
-    if (d.occ) {
-      const long tot5 = per * d.nj;
-      ProfScope ps(cx, f64 ? "pair_reduce_sym_f64" : "pair_reduce_sym_f32");
-      hipLaunchKernelGGL((k_pair_reduce_sym<T>), dim3((unsigned)tot5), dim3(256), 0, cx.stream, d, nvec);
-      INQX_HIP(hipGetLastError());
-    }
   }
 }
 
