@@ -12,11 +12,12 @@
 // real-space arrays in state-major layout [state][i0][i1][i2]:
 //
 //   pair_plane_fwd   per (j, plane i0, i): forms rho on the fly from the two
-//                    planes, 2-D forward FFT along i1 (registers, a column
-//                    per lane pair) then i2 (LDS rows), stores the plane of t
+//                    planes, 2-D forward FFT along i1 (memory to LDS) then i2
+//                    (LDS to memory), stores the plane of t transposed
 //   pair_xline       per (j, i, 128 lines (i1,i2)): forward FFT along i0 in
 //                    registers, Poisson kernel, inverse FFT along i0, in place
-//   pair_plane_inv   per (j, plane i0, i): 2-D inverse FFT of the plane of t
+//   pair_plane_inv   per (j, plane i0, i): 2-D inverse FFT of the plane of t, along
+//                    i2 (memory to LDS) then i1 (LDS to memory, i1 major again)
 //   pair_reduce      w_i += sum_j coef_j hf_j t_ji in j order (deterministic;
 //                    chunks of j give the same bits); with hf = phi
 //                    pair_reduce_both also sums the conjugate pairs' terms
@@ -47,6 +48,7 @@ template <typename T> struct PairDev {
   // wb by k_pair_reduce_both.  occ: [nst] 1 for an occupied state, or null.
   const int *occ;
   cplx<T> *wb;         // [nst][N]
+  int transposed;      // between the plane passes a plane of t is [f2][f1]
   T b[3][3];           // reciprocal lattice vectors (rows, cartesian, 2 pi included)
   T q[3];              // cartesian shift added to G
   T scal;              // 4 pi / N
@@ -55,19 +57,28 @@ template <typename T> struct PairDev {
 
 // a plane pass works on one N1 x N2 plane in LDS (rows padded to N2 + 1); every
 // row or column of the plane is split over LANES lanes of a wave (a lane pair
-// (l, l + 32), or the four lanes l + 16 q for complex128 planes from 72
-// points, whose planes fill the LDS of a CU: four lanes per line give that
-// one work-group twice the waves), so a wave covers 64 / LANES lines
+// (l, l + 32), or the four lanes l + 16 q from 72 points, where a plane takes so
+// much of the LDS that few work-groups share a CU: four lanes per line give them
+// 5/3 to 2 times the waves; forward pass of 8256 pairs at 72^3 complex64 11.6 ->
+// 10.4 ms), so a wave covers 64 / LANES lines
 template <typename T, int N1, int N2> struct PairPlaneCfg {
   static constexpr int STRIDE = N2 + 1;
   static constexpr int NL = N1 > N2 ? N1 : N2;
-  static constexpr int LANES = sizeof(T) == 8 && N1 % 4 == 0 && N2 % 4 == 0 && NL >= 72 ? 4 : 2;
+  static constexpr int LANES = N1 % 4 == 0 && N2 % 4 == 0 && NL >= 72 ? 4 : 2;
   static constexpr int LPW = 64 / LANES;
   static constexpr int THREADS = (NL + LPW - 1) / LPW * 64;
   static_assert(THREADS <= 512, "plane pass sized for at most 8 waves");
   // the launch bound: 256 keeps up to 512 VGPRs per lane-pair thread
   static constexpr int MAXT = THREADS <= 256 ? 256 : 512;
-  static constexpr int LDS = N1 * STRIDE * (int)sizeof(cplx<T>);
+  // the plane crosses LDS in one piece, or, where fewer than four whole planes fit a
+  // CU, real and imaginary parts one after the other through half the LDS (three
+  // barriers instead of one).  One Poisson solve in pieces against whole:
+  // complex64 72^3 3.58 / 3.55 us (the exchange pass over 8256 pairs 9.9 / 10.4 ms),
+  // 108^3 12.4 / 13.8; complex128 72^3 7.15 / 7.23, 128^3 38 / 80 us (a whole plane
+  // does not fit there and the column and row kernels of n1 != n2 run); smaller
+  // planes within 1 %
+  static constexpr bool HALVES = N1 * STRIDE * (int)sizeof(cplx<T>) > 40 * 1024;
+  static constexpr int LDS = N1 * STRIDE * (int)sizeof(cplx<T>) / (HALVES ? 2 : 1);
 };
 template <typename T, int N1, int N2> constexpr int pair_plane_maxt() { return PairPlaneCfg<T, N1, N2>::MAXT; }
 
@@ -75,25 +86,6 @@ template <typename T, int N1, int N2> constexpr int pair_plane_maxt() { return P
 // when both are occupied and i > j (the potential of pair (i, j) stands for it)
 template <typename T> __device__ __forceinline__ bool pair_skipped(const PairDev<T> &d, int jj, int i) {
   return d.occ && i > gp(d.jlist)[jj] && gp(d.occ)[i] != 0;
-}
-
-// FFT along i2 of row r of the LDS plane, split over S lanes (part q of the
-// row); rows >= N1 run on a clamped row and do not store
-template <typename C, int N1, int N2, int SIGN, int S>
-__device__ __forceinline__ void lds_row_fft_split(C *lds, int r, int q) {
-  constexpr int M = N2 / S;
-  const int rc = r < N1 ? r : N1 - 1;
-  C *row = lds + rc * (N2 + 1);
-  C v[M];
-#pragma unroll
-  for (int n = 0; n < M; ++n) v[n] = row[S * n + q];
-  line_dit<N2, SIGN, C, S>(v, q);
-  __builtin_amdgcn_wave_barrier();
-  if (r < N1) {
-    const int o = line_out_q<N2, S>(q);
-#pragma unroll
-    for (int k = 0; k < M; ++k) row[line_out_j<N2, S>(k) + o] = v[k];
-  }
 }
 
 // pair plane (chunk entry jj, plane i0, state i) of work-group wg in the passes that
@@ -108,6 +100,40 @@ __device__ __forceinline__ void pair_product_item(int wg, int nst, int nj, int &
   i0 = r / nj;
 }
 
+// the transposition between a plane's two transforms: value k of v goes to LDS
+// element wr + wk(k) (lanes with ok), value n of w comes from rd + rn(n)
+template <typename T, bool HALVES, int K, int M, typename FW, typename FR>
+__device__ __forceinline__ void lds_exchange(unsigned char *lds, const cplx<T> (&v)[K], bool ok, int wr, FW wk, int rd,
+                                             FR rn, cplx<T> (&w)[M]) {
+  if constexpr (HALVES) {
+    T *u = reinterpret_cast<T *>(lds);
+    if (ok) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) u[wr + wk(k)] = v[k].x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < M; ++n) w[n].x = u[rd + rn(n)];
+    __syncthreads();
+    if (ok) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) u[wr + wk(k)] = v[k].y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < M; ++n) w[n].y = u[rd + rn(n)];
+  } else {
+    cplx<T> *u = reinterpret_cast<cplx<T> *>(lds);
+    if (ok) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) u[wr + wk(k)] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < M; ++n) w[n] = u[rd + rn(n)];
+  }
+}
+
 template <int N> __host__ __device__ constexpr int symi(int i) { return i >= (N + 1) / 2 ? i - N : i; }
 
 // reciprocal: the hardware approximation (1 ulp) for the complex64 path, an
@@ -115,15 +141,22 @@ template <int N> __host__ __device__ constexpr int symi(int i) { return i >= (N 
 __device__ __forceinline__ float rcp_t(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double rcp_t(double x) { return 1.0 / x; }
 
+// The plane's two transforms, each between registers and one of memory and LDS: with
+// t transposed ([f2][f1]) the second one's results leave the registers as runs of
+// consecutive rows, and the inverse pass reads them the same way.  A plane then
+// crosses the LDS once; rows transformed in LDS and copied out from there took
+// another round trip and a barrier.  The inverse pass moves 49 GB for 8256 pairs at
+// 72^3 complex64 at 4.8 TB/s, the forward one is bound by VALU issue (5.4 ms of it)
+// and stores together: forward 11.7 -> 9.9 ms, inverse 11.0 -> 10.2 ms.  One solve
+// at 72^3 complex128 8.7 -> 7.1 us.
 template <typename T, int N1, int N2>
 __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_fwd(PairDev<T> d, int total) {
   using C = cplx<T>;
   using Cfg = PairPlaneCfg<T, N1, N2>;
   constexpr int NP = N1 * N2;
-  constexpr int S = Cfg::LANES, M1 = N1 / S;
+  constexpr int S = Cfg::LANES, M1 = N1 / S, M2 = N2 / S;
   const long N = (long)d.n0 * NP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  C *lds = reinterpret_cast<C *>(smem_raw);
   const int tid = threadIdx.x;
   const int line = (tid >> 6) * Cfg::LPW + (tid & 63) % Cfg::LPW;
   const int q = (tid & 63) / Cfg::LPW, qo = line_out_q<N1, S>(q);  // part of the line, its output position
@@ -139,10 +172,10 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_f
     const GAS C *ph = gp(d.phi) + (size_t)i * N + plane;
     const GAS C *hf = nullptr;
     if (d.hf) hf = gp(d.hf) + (size_t)gp(d.jlist)[jj] * N + plane;
+    const int z = line < N2 ? line : N2 - 1, y1 = line < N1 ? line : N1 - 1;
+    C v[M1], w[M2];
     {
       // column z = line along i1: part q holds y = S n + q
-      const int z = line < N2 ? line : N2 - 1;
-      C v[M1];
       if (hf) {
 #pragma unroll
         for (int n = 0; n < M1; ++n) {
@@ -155,20 +188,18 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_f
         for (int n = 0; n < M1; ++n) v[n] = ph[(S * n + q) * N2 + z];
       }
       line_dit<N1, -1, C, S>(v, q);
-      if (line < N2) {
+    }
+    // row f1 = line along i2: part q holds z = S n + q
+    lds_exchange<T, Cfg::HALVES>(
+        smem_raw, v, line < N2, qo * Cfg::STRIDE + z, [](int k) { return line_out_j<N1, S>(k) * Cfg::STRIDE; },
+        y1 * Cfg::STRIDE + q, [](int n) { return S * n; }, w);
+    {
+      line_dit<N2, -1, C, S>(w, q);
+      const auto rt = make_rsrc(d.t + ((size_t)jj * d.nst + i) * N + plane, (unsigned)(NP * sizeof(C)));
+      const unsigned vo = line < N1 ? (unsigned)((line_out_q<N2, S>(q) * N1 + line) * sizeof(C)) : kOOB;
 #pragma unroll
-        for (int k = 0; k < M1; ++k) lds[(line_out_j<N1, S>(k) + qo) * Cfg::STRIDE + z] = v[k];
-      }
+      for (int k = 0; k < M2; ++k) bstore(rt, vo, (unsigned)(line_out_j<N2, S>(k) * N1 * sizeof(C)), w[k]);
     }
-    __syncthreads();
-    lds_row_fft_split<C, N1, N2, -1, S>(lds, line, q);
-    __syncthreads();
-    GAS C *tp = gw(d.t) + ((size_t)jj * d.nst + i) * N + plane;
-    for (int e = tid; e < NP; e += Cfg::THREADS) {
-      const int y = e / N2, z = e - y * N2;
-      tp[e] = lds[y * Cfg::STRIDE + z];
-    }
-    __syncthreads();
   }
 }
 
@@ -216,7 +247,10 @@ __global__ void __launch_bounds__(256) k_pair_xline(PairDev<T> d, int total) {
     line_dit<N0, -1, C, S>(v, q);
     __builtin_amdgcn_sched_barrier(0);  // keep the kernel factors out of the FFT's live range
     // frequency f = line_out_j(k) + qo; G + q = m0 b0 + (m1 b1 + m2 b2 + q)
-    const int i1 = Lc / N2, i2 = Lc - (Lc / N2) * N2;
+    // square planes hold (f2, f1), planes with n1 != n2 (f1, f2)
+    const bool tr = CUBE || d.transposed;
+    const int w = tr ? N1 : N2, hi = Lc / w, lo = Lc - hi * w;
+    const int i1 = tr ? lo : hi, i2 = tr ? hi : lo;
     const T m1 = (T)(i1 >= (N1 + 1) / 2 ? i1 - N1 : i1), m2 = (T)(i2 >= (N2 + 1) / 2 ? i2 - N2 : i2);
     T u[3];
 #pragma unroll
@@ -241,21 +275,19 @@ __global__ void __launch_bounds__(256) k_pair_xline(PairDev<T> d, int total) {
   }
 }
 
-// inverse 2D transform of one pair plane in place, the same decomposition as
-// the forward pass: the column transform reads t straight from memory, the
-// row transform runs from LDS.  k_pair_reduce then forms sum_j c_j hf_j t_j.
+// inverse 2D transform of one pair plane in place: the plane is whole in LDS before
+// the first store.  k_pair_reduce(_both) then forms sum_j c_j hf_j t_j.
 template <typename T, int N1, int N2>
 __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_inv(PairDev<T> d, int total) {
   using C = cplx<T>;
   using Cfg = PairPlaneCfg<T, N1, N2>;
   constexpr int NP = N1 * N2;
-  constexpr int S = Cfg::LANES, M1 = N1 / S;
+  constexpr int S = Cfg::LANES, M1 = N1 / S, M2 = N2 / S;
   const long N = (long)d.n0 * NP;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  C *lds = reinterpret_cast<C *>(smem_raw);
   const int tid = threadIdx.x;
   const int line = (tid >> 6) * Cfg::LPW + (tid & 63) % Cfg::LPW;
-  const int q = (tid & 63) / Cfg::LPW, qo = line_out_q<N1, S>(q);
+  const int q = (tid & 63) / Cfg::LPW;
   // one work item per work-group, the grid being the work count: a grid-stride loop
   // here made the complex128 96-point kernels spill to scratch
   {
@@ -267,26 +299,26 @@ __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_i
     const int jj = r / d.n0;
     if (pair_skipped(d, jj, i)) return;  // uniform over the work-group
     const size_t plane = (size_t)i0 * NP;
-    GAS C *tp = gw(d.t) + ((size_t)jj * d.nst + i) * N + plane;
+    const auto rt = make_rsrc(d.t + ((size_t)jj * d.nst + i) * N + plane, (unsigned)(NP * sizeof(C)));
+    const int z = line < N2 ? line : N2 - 1, y1 = line < N1 ? line : N1 - 1;
+    C v[M2], w[M1];
     {
-      const int z = line < N2 ? line : N2 - 1;
-      C v[M1];
+      // row f1 = line along i2: part q holds f2 = S n + q
+      const unsigned vo = (unsigned)((q * N1 + y1) * sizeof(C));
 #pragma unroll
-      for (int n = 0; n < M1; ++n) v[n] = tp[(S * n + q) * N2 + z];
-      line_dit<N1, +1, C, S>(v, q);
-      if (line < N2) {
+      for (int n = 0; n < M2; ++n) bload(rt, vo, (unsigned)(S * n * N1 * sizeof(C)), v[n]);
+      line_dit<N2, +1, C, S>(v, q);
+    }
+    // column z = line along i1: part q holds f1 = S n + q
+    lds_exchange<T, Cfg::HALVES>(
+        smem_raw, v, line < N1, y1 * Cfg::STRIDE + line_out_q<N2, S>(q), [](int k) { return line_out_j<N2, S>(k); },
+        q * Cfg::STRIDE + z, [](int n) { return S * n * Cfg::STRIDE; }, w);
+    {
+      line_dit<N1, +1, C, S>(w, q);
+      const unsigned vo = line < N2 ? (unsigned)((line_out_q<N1, S>(q) * N2 + line) * sizeof(C)) : kOOB;
 #pragma unroll
-        for (int k = 0; k < M1; ++k) lds[(line_out_j<N1, S>(k) + qo) * Cfg::STRIDE + z] = v[k];
-      }
+      for (int k = 0; k < M1; ++k) bstore(rt, vo, (unsigned)(line_out_j<N1, S>(k) * N2 * sizeof(C)), w[k]);
     }
-    __syncthreads();
-    lds_row_fft_split<C, N1, N2, +1, S>(lds, line, q);
-    __syncthreads();
-    for (int e = tid; e < NP; e += Cfg::THREADS) {
-      const int y = e / N2, z = e - y * N2;
-      tp[e] = lds[y * Cfg::STRIDE + z];
-    }
-    __syncthreads();
   }
 }
 
@@ -594,6 +626,7 @@ template <typename T, int S0, int S> void run_pairs(inqx_ham_s *h, const PairArg
   d.n0 = g.n[0];
   d.n1 = g.n[1];
   d.n2 = g.n[2];
+  d.transposed = S > 0 ? 1 : 0;
   for (int r = 0; r < 3; ++r)
     for (int c = 0; c < 3; ++c) d.b[r][c] = (T)g.b[r][c];
   for (int c = 0; c < 3; ++c) d.q[c] = (T)a.gshift[c];
