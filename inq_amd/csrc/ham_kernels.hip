@@ -540,6 +540,13 @@ __global__ void __launch_bounds__(xpass_threads<T>(N0)) k_xpass_project(const Sp
 // over all lm of an atom).  Writes D P per (group, l, state) for the energy
 // record and per (slot, state, l) -- every slot of the group -- so that the
 // apply pass loads a tile's values as contiguous records.
+//
+// The bound is latency: a slot's loads, and as many dependent rounds of them as a
+// lane has slots (a sphere of 10 points across has 80 to 100).  16 lanes share an
+// item, four of a wave and the four waves; with 4 lanes 128
+// items of 32^3 complex128 took 10.8 us (now 6.2), 624 of three groups 19.1 (10.4),
+// 8192 of 72^3 complex128 15.7 (12.2).
+constexpr int kRedItems = 16;  // (group, state) items per work-group
 template <typename T>
 __global__ void __launch_bounds__(256) k_kb_reduce(const SphereBlock<T> *blocks, const int *prefix, int nblocks,
                                                    int total, HamDev hd) {
@@ -549,13 +556,14 @@ __global__ void __launch_bounds__(256) k_kb_reduce(const SphereBlock<T> *blocks,
     if (wg >= total) return;
     const int b = find_block(prefix, nblocks, wg);
     const SphereBlock<T> B = blocks[b];
-    // four lanes per (group, state): lane quarter qr sums the slots qr, qr + 4,
-    // ... of every sibling group; the quarters are combined by two butterfly
-    // exchanges (every lane ends with the same sum, in a fixed order), and lane
-    // qr then writes channel qr
-    const int item = (wg - gp(prefix)[b]) * (blockDim.x >> 2) + (threadIdx.x >> 2);
-    const int qr = threadIdx.x & 3;
-    const bool live = item < hd.natoms * B.nst;  // uniform over the four lanes of an item
+    // 16 lanes per (group, state): part wave * 4 + qr sums the slots part, part + 16,
+    // ... of every sibling group; a wave's four parts are combined by two butterfly
+    // exchanges, the waves' through LDS (every lane ends with the same sum, in a
+    // fixed order); lane qr of every wave then holds channel qr
+    __shared__ double2 red[4][kRedItems][kCoeffCols];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, it = lane >> 2, qr = lane & 3;
+    const int item = (wg - gp(prefix)[b]) * kRedItems + it, part0 = wave * 4 + qr;
+    const bool live = item < hd.natoms * B.nst;  // uniform over the lanes of an item
     const int ic = live ? item : 0;
     const int a = ic / B.nst, s = ic - a * B.nst;
     // the projections of every group of this group's projector (siblings),
@@ -573,9 +581,9 @@ __global__ void __launch_bounds__(256) k_kb_reduce(const SphereBlock<T> *blocks,
       if (gq < ng) {
         const int q0 = gp(hd.atom_slots)[g0 + gq], q1 = gp(hd.atom_slots)[g0 + gq + 1];
         // two of this lane's slots per step, their loads in flight together
-        for (int q = q0 + qr; q < q1; q += 8) {
+        for (int q = q0 + part0; q < q1; q += 32) {
           const int sl0 = gp(hd.atom_slot_list)[q];
-          const int sl1 = gp(hd.atom_slot_list)[min(q + 4, q1 - 1)];
+          const int sl1 = gp(hd.atom_slot_list)[min(q + 16, q1 - 1)];
           C v0[kMaxNlm], v1[kMaxNlm];
 #pragma unroll
           for (int l = 0; l < kMaxNlm; ++l) {
@@ -587,7 +595,7 @@ __global__ void __launch_bounds__(256) k_kb_reduce(const SphereBlock<T> *blocks,
             pr[gq][l] += (double)v0[l].x;
             pi[gq][l] += (double)v0[l].y;
           }
-          if (q + 4 < q1) {
+          if (q + 16 < q1) {
 #pragma unroll
             for (int l = 0; l < kMaxNlm; ++l) {
               pr[gq][l] += (double)v1[l].x;
@@ -607,10 +615,27 @@ __global__ void __launch_bounds__(256) k_kb_reduce(const SphereBlock<T> *blocks,
         pr[q][l] += __shfl_xor(pr[q][l], 2, 64);
         pi[q][l] += __shfl_xor(pi[q][l], 2, 64);
       }
+#pragma unroll
+    for (int q = 0; q < kMaxGroups; ++q)
+#pragma unroll
+      for (int l = 0; l < kMaxNlm; ++l)
+        if (l == qr) red[wave][it][q * kMaxNlm + l] = double2{pr[q][l], pi[q][l]};
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kMaxGroups; ++q)
+      if (q < ng) {
+#pragma unroll
+        for (int l = 0; l < kMaxNlm; ++l) {
+          const double2 r0 = red[0][it][q * kMaxNlm + l], r1 = red[1][it][q * kMaxNlm + l];
+          const double2 r2 = red[2][it][q * kMaxNlm + l], r3 = red[3][it][q * kMaxNlm + l];
+          pr[q][l] = (r0.x + r1.x) + (r2.x + r3.x);
+          pi[q][l] = (r0.y + r1.y) + (r2.y + r3.y);
+        }
+      }
     if (!live) return;
     const int me = a - g0;  // this group among its siblings
     const int l = qr;       // the channel this lane writes
-    if (B.proj) {
+    if (B.proj && wave == 0) {
       double xr = 0.0, xi = 0.0;
 #pragma unroll
       for (int q = 0; q < kMaxGroups; ++q)
@@ -632,10 +657,10 @@ __global__ void __launch_bounds__(256) k_kb_reduce(const SphereBlock<T> *blocks,
         di += D[q * kMaxNlm + m] * pi[q][m];
       }
     const C r{(T)(dr * hd.kb_scale), (T)(di * hd.kb_scale)};
-    gw(B.dp)[((size_t)a * kMaxNlm + l) * B.nst + s] = r;
+    if (wave == 0) gw(B.dp)[((size_t)a * kMaxNlm + l) * B.nst + s] = r;
     GAS C *dps = gw(B.dps);
     const int q0 = gp(hd.atom_slots)[a], q1 = gp(hd.atom_slots)[a + 1];
-    for (int q = q0; q < q1; ++q) dps[((size_t)gp(hd.atom_slot_list)[q] * B.nst + s) * kMaxNlm + l] = r;
+    for (int q = q0 + wave; q < q1; q += 4) dps[((size_t)gp(hd.atom_slot_list)[q] * B.nst + s) * kMaxNlm + l] = r;
   }
 }
 
@@ -1855,7 +1880,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
         px[i + 1] = px[i] + x_tiles_padded(h->kb.ntile) * ((nst[i] + nw - 1) / nw);
       else
         px[i + 1] = px[i] + ld->ntile_line * ((nst[i] + 3) / 4);
-      pr[i + 1] = pr[i] + (std::max(1, h->kb.natoms) * nst[i] + 63) / 64;  // 64 (group, state) items per work-group
+      pr[i + 1] = pr[i] + (std::max(1, h->kb.natoms) * nst[i] + kRedItems - 1) / kRedItems;
     }
     int nwin = 1;
     for (int i = 0; i < nblocks; ++i) nwin = std::max(nwin, bases[i]->nwin_max);
