@@ -153,8 +153,9 @@ int inqx_ham_prepare(inqx_ham ham, inqx_basis basis, int nst, int precision);
  * plane batch.  Allocates scratch states; do not call during graph capture. */
 int inqx_ham_autotune_batch(inqx_ham ham, int nblocks, const inqx_basis *bases, const int *nst, int precision,
                             const char *cache_path, int *shape, double *best_ms);
-/* sets the plane-pass batch directly (planes per work-group; 0: the largest the
- * grid's LDS budget allows, larger values are capped to it) */
+/* sets the plane-pass batch directly (planes per work-group; 0: the most that leave
+ * every compute unit a work-group; values above the largest the grid's LDS budget
+ * allows are capped to it) */
 int inqx_ham_set_plane_batch(inqx_ham ham, int precision, int planes);
 /* the single-block form (no cache); best_xwaves / best_ms may be NULL */
 int inqx_ham_autotune(inqx_ham ham, inqx_basis basis, int nst, int precision, int *best_xwaves, double *best_ms);

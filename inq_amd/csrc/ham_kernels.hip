@@ -1711,6 +1711,29 @@ static void dispatch_passes(int n0, int n1, int n2, inqx_ham_s *h, LaunchData &l
   }
 }
 
+// x-pass waves (states) per work-group where the caller set none.  Four share a
+// tile's tables well and leave the LDS to several work-groups.
+//  * Two where four would leave CUs without a work-group: the passes are latency
+//    bound there (16 states at 32^3 complex128 41.9 us with four, 40.2 with two).
+//  * Eight where the tables are so large that the LDS holds more waves that way (d
+//    channels on 40 x 48 x 60 complex64, 40 states: 205 -> 192 us, 32 atoms of them
+//    at 60^3 204 -> 182), up to the waves the registers allow.
+//  * Two for complex128 lines from 72 points where two such groups fit the LDS: the
+//    registers hold one wave per SIMD, and a second group's line loads run while the
+//    first waits at its barrier (128 states at 72^3 918 -> 872 us, 96^3 508 -> 501;
+//    where the LDS holds one group of two, 16 states at 72^3 take 163 us against 128).
+// lds(n): bytes of a work-group of n waves; groups(n): the launch's work-groups
+template <typename T, typename FL, typename FG>
+static int auto_xwaves(int maxwaves, int n0, int maxnst, int num_cu, FL lds, FG groups) {
+  const bool dbl = std::is_same<T, double>::value;
+  const int cap = dbl ? (n0 < 72 ? 8 : 4) : n0 <= 48 ? 16 : n0 <= 72 ? 12 : 8;  // resident waves of a CU by VGPRs
+  const auto resident = [&](int n) { return std::min(cap, n * (160 * 1024 / std::max(1, lds(n)))); };
+  if (groups(4) < num_cu) return 2;
+  if (dbl && n0 >= 72 && resident(2) == cap) return 2;
+  if (maxwaves >= 8 && maxnst >= 8 && groups(8) >= num_cu && resident(8) > resident(4)) return 8;
+  return 4;
+}
+
 template <typename T>
 void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *nst, const void *const *psi,
                   void *const *hpsi, const ApplyOpts *opts) {
@@ -1792,11 +1815,24 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
     std::vector<int> pp(nblocks + 1, 0), px(nblocks + 1, 0), pr(nblocks + 1, 0);
     int plane_p = max_plane_batch(g.n, prec);
     // the launch shape's plane batch (autotuned), at most what the LDS budget allows
-    if (h->plane_batch[prec] > 0) plane_p = std::min(plane_p, h->plane_batch[prec]);
+    // or the most planes that still give every CU a work-group: fewer, longer ones are
+    // a longer chain of barriers (16 states at 32^3 complex128, 368 planes: 41.9 us
+    // with 4 in a group, 39.6 with 1)
+    if (h->plane_batch[prec] > 0) {
+      plane_p = std::min(plane_p, h->plane_batch[prec]);
+    } else {
+      const auto groups = [&](int p) {
+        long n = 0;
+        for (int i = 0; i < nblocks; ++i) n += (long)bases[i]->nslot * ((nst[i] + p - 1) / p);
+        return n;
+      };
+      while (plane_p > 1 && groups(plane_p) < h->ctx->c.num_cu) --plane_p;
+    }
     ld->plane_batch = plane_p;
     // waves (states) per x-pass work-group within the LDS budget
     const int cs = (int)sizeof(cplx<T>);
-    int nw = std::max(1, std::min(xpass_threads<T>(g.n[0]) / 64, h->xwaves[prec]));  // states (waves) per x-pass work-group
+    const int maxwaves = xpass_threads<T>(g.n[0]) / 64;
+    int nw = std::max(1, std::min(maxwaves, h->xwaves[prec]));  // states (waves) per x-pass work-group
     ld->mode = mode;
     ld->observables = opts->observables;
     ld->ntile_line = (g.n[1] * g.n[2] + 31) / 32;
@@ -1825,6 +1861,15 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
       xp.li = x.li - x.cs;
       xp.wave0 = x.wave0 - x.cs;
       xp.wave_bytes = xp.aux + 64 * kMaxNlm * cs;
+      if (h->xwaves[prec] == 0) {
+        const auto groups = [&](int n) {
+          long c = 0;
+          for (int i = 0; i < nblocks; ++i) c += (long)h->kb.ntile * ((nst[i] + n - 1) / n);
+          return c;
+        };
+        nw = auto_xwaves<T>(maxwaves, g.n[0], *std::max_element(nst, nst + nblocks), h->ctx->c.num_cu,
+                         [&](int n) { return x.wave0 + n * x.wave_bytes; }, groups);
+      }
       constexpr int kLdsMax = 160 * 1024;
       INQX_CHECK(x.wave0 + x.wave_bytes <= kLdsMax && xp.wave0 + xp.wave_bytes <= kLdsMax, INQX_ERR_UNSUPPORTED,
                  "KB tile too dense for LDS");

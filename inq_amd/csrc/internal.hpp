@@ -330,8 +330,10 @@ struct inqx_ham_s {
   std::vector<inqx_basis> bases;
   int pinned = 0;  // > 0 while a captured graph uses the projector tables
   // launch shape of the x-pass kernels per precision: states (waves) per work-group
-  int xwaves[2] = {4, 4};  // states per x-pass work-group (complex128, complex64)
-  // plane-pass planes (states) per work-group per precision; 0: the largest the grid allows
+  // (complex128, complex64); 0: by the work and the LDS (ham_kernels.hip, auto_xwaves)
+  int xwaves[2] = {0, 0};
+  // plane-pass planes (states) per work-group per precision; 0: the most that leave
+  // every CU a work-group
   int plane_batch[2] = {0, 0};
   // exact-exchange workspaces: real-space states, hf states, accumulator, pair planes
   inqx::DevMem exx_phi, exx_hf, exx_w, exx_t, exx_jlist, exx_coef;
