@@ -321,7 +321,9 @@ def contractions(ctx, reps=10):
     """The dense contractions on the matrix cores: the overlap S = vol phi^H phi
     (operations::overlap) and the rotation phi R (operations::rotate) at the
     Si64 block (128 x 67 691) and the Si216 block (432 x 228 487).  8 n^2 K flop
-    each (complex multiply-add), timed per kernel with the library's HIP events;
+    for the rotation (complex multiply-add), 4 n (n + 1) K for the overlap of a
+    block with itself (Hermitian: its lower triangle), timed per kernel with the
+    library's HIP events;
     utilisation is against the dense FP32 / FP64 MFMA peak."""
     from inq_amd import DeviceArray
     from inq_amd import operations as ops
@@ -342,12 +344,12 @@ def contractions(ctx, reps=10):
                 ops.rotate(ctx, rot, d)
             kt = ctx.kernel_times()
             ctx.profile(False)
-            flop = 8.0 * n * n * K
+            flops = {"overlap": 4.0 * n * (n + 1) * K, "rotate": 8.0 * n * n * K}
             res = {}
             sfx = "f32" if prec == "fp32" else "f64"
             for kind, key in (("overlap", f"overlap_mfma_{sfx}"), ("rotate", f"rotate_mfma_{sfx}")):
                 cnt, ms = kt[key]
-                tf = flop / (ms / cnt * 1e-3) / 1e12
+                tf = flops[kind] / (ms / cnt * 1e-3) / 1e12
                 res[kind] = {"us": ms / cnt * 1e3, "tflops": tf, "frac_of_mfma_peak": tf / MFMA_PEAK_TFLOPS[prec]}
             cnt, ms = kt[f"overlap_reduce_{sfx}"]
             res["overlap"]["reduce_us"] = ms / cnt * 1e3
