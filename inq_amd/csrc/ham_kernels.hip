@@ -1169,15 +1169,20 @@ void build_kb_tables(inqx_ham_s *h) {
         return (m.i0 * g.n[1] + L / g.n[2]) * (g.n[2] + 1) + L % g.n[2];
       };
       std::vector<std::vector<size_t>> by(kb.natoms);
-      for (size_t k = 0; k < mem.size(); ++k) by[mem[k].a].push_back(k);
+      // point by point, as the groups of a projector list the sphere's points
+      for (int a = 0; a < kb.natoms; ++a) by[a].resize((size_t)h->projs[gproj[a]].npts());
+      for (size_t k = 0; k < mem.size(); ++k) by[mem[k].a][mem[k].p] = k;
       std::vector<int> row(kb.natoms + 1, 0), off;
       std::vector<float> v32;
       std::vector<double> v64;
       std::vector<float> spos;
+      const size_t most = mem.size() + 64 * (size_t)kb.natoms;
+      off.reserve(most);
+      v32.reserve(kMaxNlm * most);
+      v64.reserve(kMaxNlm * most);
+      spos.reserve(4 * most);
       for (int a = 0; a < kb.natoms; ++a) {
         row[a] = (int)(off.size() / 64);
-        // the groups of a projector list the sphere's points in the same order
-        std::sort(by[a].begin(), by[a].end(), [&](size_t x, size_t y) { return mem[x].p < mem[y].p; });
         for (size_t k : by[a]) {
           off.push_back(offset(mem[k]));
           for (int q = 0; q < kMaxNlm; ++q) {
@@ -1199,12 +1204,14 @@ void build_kb_tables(inqx_ham_s *h) {
       std::vector<std::vector<char>> used;
       std::vector<std::vector<int>> cls;
       bool twice = false;
+      std::vector<int> last((size_t)g.n[0] * g.n[1] * (g.n[2] + 1), -1);  // last projector that holds the point
       for (int a = 0; a < kb.natoms; a += sib[2 * a + 1]) {
         std::vector<int> pts;
         for (size_t k : by[a]) pts.push_back(offset(mem[k]));
-        std::vector<int> s = pts;
-        std::sort(s.begin(), s.end());
-        if (std::unique(s.begin(), s.end()) != s.end()) twice = true;
+        for (int o : pts) {
+          if (last[o] == a) twice = true;
+          last[o] = a;
+        }
         size_t c = 0;
         for (; c < cls.size(); ++c)
           if (std::none_of(pts.begin(), pts.end(), [&](int o) { return used[c][o] != 0; })) break;
@@ -1227,14 +1234,27 @@ void build_kb_tables(inqx_ham_s *h) {
         first.push_back((int)(item.size() / 4));
       }
       kb.sg_classes = twice ? 0 : (int)cls.size();
-      upload(kb.sg_row, row, st);
-      upload(kb.sg_off, off, st);
       kb.pos_host[1].swap(spos);
       kb.pos[1].release();
-      upload(kb.sg_b32, v32, st);
-      upload(kb.sg_b64, v64, st);
-      upload(kb.sg_item, item, st);
-      upload(kb.sg_class, first, st);
+      std::vector<char> all;  // the tables in one allocation and one copy
+      const auto put = [&](const void *p, size_t bytes) {
+        const size_t at = (all.size() + 255) / 256 * 256;
+        all.resize(at + bytes);
+        if (bytes) std::memcpy(all.data() + at, p, bytes);
+        return at;
+      };
+      const size_t at_row = put(row.data(), sizeof(int) * row.size()), at_off = put(off.data(), sizeof(int) * off.size());
+      const size_t at32 = put(v32.data(), sizeof(float) * v32.size()), at64 = put(v64.data(), sizeof(double) * v64.size());
+      const size_t at_item = put(item.data(), sizeof(int) * item.size());
+      const size_t at_class = put(first.data(), sizeof(int) * first.size());
+      upload(kb.sg, all, st);
+      const char *base = kb.sg.as<char>();
+      kb.sg_row = reinterpret_cast<const int *>(base + at_row);
+      kb.sg_off = reinterpret_cast<const int *>(base + at_off);
+      kb.sg_b32 = base + at32;
+      kb.sg_b64 = base + at64;
+      kb.sg_item = reinterpret_cast<const int *>(base + at_item);
+      kb.sg_class = reinterpret_cast<const int *>(base + at_class);
       INQX_HIP(hipStreamSynchronize(st));
     }
     ent_cs.swap(cs2);

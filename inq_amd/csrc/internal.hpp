@@ -190,7 +190,9 @@ struct KBTables {
   // rows of the projectors (first group's row, first group, groups, rows between
   // groups) in classes of projectors that share no point.  sg_classes = 0: a
   // projector's sphere holds a point twice (periodic images), not offered
-  DevMem sg_row, sg_off, sg_b32, sg_b64, sg_item, sg_class;
+  DevMem sg;  // one allocation: sg_row, sg_off, ... below point into it
+  const int *sg_row = nullptr, *sg_off = nullptr, *sg_item = nullptr, *sg_class = nullptr;
+  const void *sg_b32 = nullptr, *sg_b64 = nullptr;
   int sg_classes = 0;
   long sg_nrec = 0;
   // float4 position of every record of the two orders, for the per-basis phase

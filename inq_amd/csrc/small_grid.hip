@@ -305,11 +305,11 @@ void launch_small_apply(inqx_ham_s *h, const SphereBlock<T> *blk, const int *ite
   d.dp_off = d.part_off + (int)part_bytes(prec, d.natoms);
   const int lds = d.dp_off + (int)sizeof(cplx<T>) * kMaxNlm * d.natoms;
   INQX_CHECK(lds <= kLdsBytes, INQX_ERR_UNSUPPORTED, "the cube does not fit the LDS");
-  d.g_row = kb.sg_row.as<int>();
-  d.g_off = kb.sg_off.as<int>();
-  d.g_b = prec == INQX_FP64 ? kb.sg_b64.p : kb.sg_b32.p;
-  d.g_item = kb.sg_item.p;
-  d.g_class = kb.sg_class.as<int>();
+  d.g_row = kb.sg_row;
+  d.g_off = kb.sg_off;
+  d.g_b = prec == INQX_FP64 ? kb.sg_b64 : kb.sg_b32;
+  d.g_item = kb.sg_item;
+  d.g_class = kb.sg_class;
   d.classes = has_kb ? kb.sg_classes : 0;
   d.coeff = kb.coeff.as<double>();
   d.group_sib = kb.group_sib.as<int>();
