@@ -250,8 +250,11 @@ __global__ void __launch_bounds__(kTriThreads) k_tridiag_eig(const double *dd, c
       if (rank[i] != round) continue;
       const double x = lv[i];
       // LU with partial pivoting of T - x I (columns of this lane: index j * n + i)
+      // the back substitution reads both super-diagonals to the last row, where they are
+      // multiplied by 0: they are written there too, as scratch may hold NaN
       U0[i] = d[0] - x;
-      if (n > 1) U1[i] = er[0];
+      U1[i] = n > 1 ? er[0] : 0.0;
+      U2[(size_t)(n - 1) * n + i] = 0.0;
       for (int j = 0; j + 1 < n; ++j) {
         const size_t aj = (size_t)j * n + i, aj1 = (size_t)(j + 1) * n + i;
         const double b = er[j], a1 = d[j + 1] - x, c1 = j + 2 < n ? er[j + 1] : 0.0;
