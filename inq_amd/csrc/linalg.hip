@@ -194,13 +194,14 @@ __device__ __forceinline__ int xcd_logical(int b, int G) {
 // S = vol A^H B split over K: a work-group sums one chunk of K for one 64 x 64
 // tile.  The grid is sized to run as one round of equal work-groups (up to four
 // per CU), so none waits for a last partial round.  FP32 products accumulate over
-// at most kOvRun complex values before they are added in FP64 (WIDE: chunks
+// at most `run` complex values before they are added in FP64 (WIDE: chunks
 // longer than that keep FP64 sums in registers and write FP64 partial tiles).
 // HERM (A and B the same states): only the tiles on and below the diagonal.
 // Measured, before -> now: 432 states x 228487 with themselves, complex64, 3.38 ->
 // 1.87 ms (112 TFLOP/s over the products done); 128 x 67691 93 -> 67 us complex64,
 // two different blocks of it in complex128 176 -> 166 us (53 of 67 TFLOP/s).
-constexpr int kOvRun = 1024;        // complex values per FP32 accumulation
+constexpr int kOvRunMin = 128, kOvRunMax = 1024;  // complex values per FP32 accumulation
+constexpr int kOvRunSplit = 1024;   // the contractions of all tiles are cut in so many runs between the two
 constexpr int kOvChunkMin = 128;    // complex values per work-group at least
 constexpr int kOvChunkGood = 256;   // enough stages to hide a work-group's start and end
 
@@ -208,6 +209,8 @@ struct OvPlan {
   int tiles_i, tiles_j, tiles;  // tiles: all, or those on and below the diagonal
   int nchunk;
   long chunk;  // complex values, a multiple of the stage
+  int run;     // complex64: complex values per FP32 accumulation, a multiple of the stage
+  bool wide;   // complex64: FP64 sums within a chunk
 };
 // work-groups per CU in the one round: what the registers hold
 static int overlap_slots(bool f64, bool wide) { return f64 || wide ? 3 : 4; }
@@ -215,13 +218,20 @@ static OvPlan overlap_plan(int n1, int n2, long K, bool herm, int cus, bool f64)
   OvPlan p;
   p.tiles_i = (n1 + kMT - 1) / kMT;
   p.tiles_j = (n2 + kMT - 1) / kMT;
-  p.tiles = herm ? p.tiles_i * (p.tiles_i + 1) / 2 : p.tiles_i * p.tiles_j;
+  const int all = p.tiles_i * p.tiles_j;
+  p.tiles = herm ? p.tiles_i * (p.tiles_i + 1) / 2 : all;
   const int stage = f64 ? kStage<double> : kStage<float>;
+  const auto stages = [&](long c) { return (c + stage - 1) / stage * stage; };
+  // The rounding of an FP32 sum grows with its length, so the length does not follow
+  // the launch shape below: small contractions end after 128 values, the longest
+  // after 1024 (error of a norm over 30000 values: 1.5e-8 rms with 128, 4.3e-8 with 368)
+  const long want_run = (kOvRunSplit + all - 1) / all;
+  p.run = (int)stages(std::min<long>(kOvRunMax, std::max<long>(kOvRunMin, (K + want_run - 1) / want_run)));
   for (int m = 4; m >= 1; --m) {
     const long want = std::max<long>(1, (long)m * cus / p.tiles);
-    if (m > overlap_slots(f64, K > want * kOvRun)) continue;
-    long c = std::max<long>((K + want - 1) / want, kOvChunkMin);
-    p.chunk = (c + stage - 1) / stage * stage;
+    p.chunk = stages(std::max<long>((K + want - 1) / want, kOvChunkMin));
+    p.wide = !f64 && p.chunk > p.run;
+    if (m > overlap_slots(f64, p.wide)) continue;
     if (p.chunk >= kOvChunkGood) break;
   }
   p.nchunk = (int)((K + p.chunk - 1) / p.chunk);
@@ -240,7 +250,8 @@ __device__ __forceinline__ void lower_tile(int t, int &ti, int &tj) {
 template <typename T, typename P, bool WIDE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WIDE || sizeof(T) == 8 ? 3 : 4)))
 k_overlap_partial(const T *A, const T *B, int n1, int n2, long K, int tiles,
-                                                         int tiles_j, int herm, long chunk, P *partial) {
+                                                         int tiles_j, int herm, long chunk, int run,
+                                                         P *partial) {
   constexpr int KC = kStage<T>, CV = 16 / (2 * (int)sizeof(T)), kTile = kMT * kRowStride;
   __shared__ __align__(16) unsigned char sm[2][2][kTile];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -298,7 +309,7 @@ k_overlap_partial(const T *A, const T *B, int n1, int n2, long K, int tiles,
     }
   };
   const long kw = k0 + (k1 - k0) / KC * KC;  // end of the whole stages
-  int buf = 0, run = 0;
+  int buf = 0, summed = 0;
   if (k0 < kw) {
     load(k0);
     store(0);
@@ -308,8 +319,8 @@ k_overlap_partial(const T *A, const T *B, int n1, int n2, long K, int tiles,
     const bool more = k + KC < kw;
     if (more) load(k + KC);
     mac(buf);
-    if (WIDE && (run += KC) >= kOvRun) {
-      run = 0;
+    if (WIDE && (summed += KC) >= run) {
+      summed = 0;
       widen();
     }
     buf ^= 1;
@@ -872,8 +883,7 @@ void launch_overlap(Ctx &cx, int prec, int n1, int n2, long K, const void *A, co
   const bool herm = A == B && n1 == n2;
   const bool f64 = prec == INQX_FP64;
   const OvPlan p = overlap_plan(n1, n2, K, herm, cx.num_cu, f64);
-  const bool wide = !f64 && p.chunk > kOvRun;  // FP64 partial tiles of FP32 products
-  const size_t es = f64 || wide ? 8 : 4;
+  const size_t es = f64 || p.wide ? 8 : 4;
   partial.ensure(es * (size_t)p.nchunk * p.tiles * kMT * kMT * 2);
   const long grid = (long)p.nchunk * p.tiles;
   INQX_CHECK(grid <= INT32_MAX / kMT, INQX_ERR_ARG, "overlap: too many tiles");
@@ -883,13 +893,13 @@ void launch_overlap(Ctx &cx, int prec, int n1, int n2, long K, const void *A, co
     ProfScope ps(cx, f64 ? "overlap_mfma_f64" : "overlap_mfma_f32");
     if (f64)
       hipLaunchKernelGGL((k_overlap_partial<double, double, false>), g, dim3(256), 0, cx.stream, (const double *)A,
-                         (const double *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, partial.as<double>());
-    else if (wide)
+                         (const double *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, p.run, partial.as<double>());
+    else if (p.wide)
       hipLaunchKernelGGL((k_overlap_partial<float, double, true>), g, dim3(256), 0, cx.stream, (const float *)A,
-                         (const float *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, partial.as<double>());
+                         (const float *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, p.run, partial.as<double>());
     else
       hipLaunchKernelGGL((k_overlap_partial<float, float, false>), g, dim3(256), 0, cx.stream, (const float *)A,
-                         (const float *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, partial.as<float>());
+                         (const float *)B, n1, n2, K, p.tiles, p.tiles_j, h, p.chunk, p.run, partial.as<float>());
   }
   INQX_HIP(hipGetLastError());
   ProfScope ps(cx, f64 ? "overlap_reduce_f64" : "overlap_reduce_f32");
