@@ -1375,7 +1375,10 @@ __global__ void __launch_bounds__(256) k_phase_table(const float4 *pos, int n, d
 // the tables of the blocks with k + A != 0, in the x passes' record order or in
 // that of small_grid.hip.  The missing ones of a launch share one allocation (a
 // hipMalloc each was most of a batch's first application) and one wait, as a table
-// outlives a change of the context's stream.
+// outlives a change of the context's stream.  All tables a basis holds are of one
+// (A, generation): the first that is rebuilt for another one drops the rest.  A basis
+// pinned by a captured graph therefore takes the first table of a further precision
+// or order, which the graph does not read, and refuses the rebuild of any it has.
 template <typename T>
 static void ensure_phase_tables(inqx_ham_s *h, int nblocks, Basis *const *bases, bool small) {
   KBTables &kb = h->kb;
@@ -1387,7 +1390,7 @@ static void ensure_phase_tables(inqx_ham_s *h, int nblocks, Basis *const *bases,
     const Basis::PhaseTable &t = b.ph[w][prec];
     if (b.kcov[0] + h->A[0] == 0.0 && b.kcov[1] + h->A[1] == 0.0 && b.kcov[2] + h->A[2] == 0.0) continue;
     if (t.gen == kb.gen && t.A[0] == h->A[0] && t.A[1] == h->A[1] && t.A[2] == h->A[2]) continue;
-    INQX_CHECK(b.pinned == 0, INQX_ERR_STATE, "basis tables are pinned by a captured propagation graph");
+    INQX_CHECK(b.pinned == 0 || !t.p, INQX_ERR_STATE, "basis tables are pinned by a captured propagation graph");
     if (std::find(todo.begin(), todo.end(), &b) == todo.end()) todo.push_back(&b);
   }
   if (todo.empty()) return;
@@ -1398,6 +1401,9 @@ static void ensure_phase_tables(inqx_ham_s *h, int nblocks, Basis *const *bases,
   for (size_t i = 0; i < todo.size(); ++i) {
     Basis &b = *todo[i];
     Basis::PhaseTable &t = b.ph[w][prec];
+    for (auto &order : b.ph)
+      for (Basis::PhaseTable &o : order)
+        if (o.p && (o.gen != kb.gen || o.A[0] != h->A[0] || o.A[1] != h->A[1] || o.A[2] != h->A[2])) o = {};
     t.store = store;
     t.p = store->as<char>() + per * i;
     t.gen = -1;
