@@ -1162,101 +1162,6 @@ void build_kb_tables(inqx_ham_s *h) {
       base += 64L * rows;
       kb.maxchunk = std::max(kb.maxchunk, rows);
     }
-    // small grids (small_grid.hip): the entries by group at their offsets in the padded cube
-    if (dev && small_grid(g.n)) {
-      auto offset = [&](const Mem &m) {
-        const int L = m.tile * kTile + m.lane;
-        return (m.i0 * g.n[1] + L / g.n[2]) * (g.n[2] + 1) + L % g.n[2];
-      };
-      std::vector<std::vector<size_t>> by(kb.natoms);
-      // point by point, as the groups of a projector list the sphere's points
-      for (int a = 0; a < kb.natoms; ++a) by[a].resize((size_t)h->projs[gproj[a]].npts());
-      for (size_t k = 0; k < mem.size(); ++k) by[mem[k].a][mem[k].p] = k;
-      std::vector<int> row(kb.natoms + 1, 0), off;
-      std::vector<float> v32;
-      std::vector<double> v64;
-      std::vector<float> spos;
-      const size_t most = mem.size() + 64 * (size_t)kb.natoms;
-      off.reserve(most);
-      v32.reserve(kMaxNlm * most);
-      v64.reserve(kMaxNlm * most);
-      spos.reserve(4 * most);
-      for (int a = 0; a < kb.natoms; ++a) {
-        row[a] = (int)(off.size() / 64);
-        for (size_t k : by[a]) {
-          off.push_back(offset(mem[k]));
-          for (int q = 0; q < kMaxNlm; ++q) {
-            v32.push_back(eb32[kMaxNlm * k + q]);
-            v64.push_back(eb64[kMaxNlm * k + q]);
-          }
-          for (int q = 0; q < 4; ++q) spos.push_back(epos[4 * k + q]);
-        }
-        while (off.size() % 64) {  // padding: offset -1, zero projector values
-          off.push_back(-1);
-          v32.insert(v32.end(), kMaxNlm, 0.0f);
-          v64.insert(v64.end(), kMaxNlm, 0.0);
-          spos.insert(spos.end(), 4, 0.0f);
-        }
-      }
-      row[kb.natoms] = (int)(off.size() / 64);
-      kb.sg_nrec = (long)off.size();
-      // classes of projectors that share no point, each projector in the first that takes it
-      std::vector<std::vector<char>> used;
-      std::vector<std::vector<int>> cls;
-      bool twice = false;
-      std::vector<int> last((size_t)g.n[0] * g.n[1] * (g.n[2] + 1), -1);  // last projector that holds the point
-      for (int a = 0; a < kb.natoms; a += sib[2 * a + 1]) {
-        std::vector<int> pts;
-        for (size_t k : by[a]) pts.push_back(offset(mem[k]));
-        for (int o : pts) {
-          if (last[o] == a) twice = true;
-          last[o] = a;
-        }
-        size_t c = 0;
-        for (; c < cls.size(); ++c)
-          if (std::none_of(pts.begin(), pts.end(), [&](int o) { return used[c][o] != 0; })) break;
-        if (c == cls.size()) {
-          cls.emplace_back();
-          used.emplace_back((size_t)g.n[0] * g.n[1] * (g.n[2] + 1), 0);
-        }
-        cls[c].push_back(a);
-        for (int o : pts) used[c][o] = 1;
-      }
-      std::vector<int> item, first(1, 0);
-      for (auto &list : cls) {
-        for (int a : list)
-          for (int r = row[a]; r < row[a + 1]; ++r) {
-            item.push_back(r);
-            item.push_back(a);
-            item.push_back(sib[2 * a + 1]);
-            item.push_back(row[a + 1] - row[a]);
-          }
-        first.push_back((int)(item.size() / 4));
-      }
-      kb.sg_classes = twice ? 0 : (int)cls.size();
-      kb.pos_host[1].swap(spos);
-      kb.pos[1].release();
-      std::vector<char> all;  // the tables in one allocation and one copy
-      const auto put = [&](const void *p, size_t bytes) {
-        const size_t at = (all.size() + 255) / 256 * 256;
-        all.resize(at + bytes);
-        if (bytes) std::memcpy(all.data() + at, p, bytes);
-        return at;
-      };
-      const size_t at_row = put(row.data(), sizeof(int) * row.size()), at_off = put(off.data(), sizeof(int) * off.size());
-      const size_t at32 = put(v32.data(), sizeof(float) * v32.size()), at64 = put(v64.data(), sizeof(double) * v64.size());
-      const size_t at_item = put(item.data(), sizeof(int) * item.size());
-      const size_t at_class = put(first.data(), sizeof(int) * first.size());
-      upload(kb.sg, all, st);
-      const char *base = kb.sg.as<char>();
-      kb.sg_row = reinterpret_cast<const int *>(base + at_row);
-      kb.sg_off = reinterpret_cast<const int *>(base + at_off);
-      kb.sg_b32 = base + at32;
-      kb.sg_b64 = base + at64;
-      kb.sg_item = reinterpret_cast<const int *>(base + at_item);
-      kb.sg_class = reinterpret_cast<const int *>(base + at_class);
-      INQX_HIP(hipStreamSynchronize(st));
-    }
     ent_cs.swap(cs2);
     eb32.swap(b32);
     eb64.swap(b64);
@@ -1265,6 +1170,7 @@ void build_kb_tables(inqx_ham_s *h) {
   kb.nent = (long)ent_cs.size() / 2;
   kb.pos_host[0].swap(epos);
   kb.pos[0].release();
+  kb.sg_built = false;
   ++kb.gen;
   std::vector<int> atom_slots(kb.natoms + 1, 0), atom_slot_list;
   for (int a = 0; a < kb.natoms; ++a) {
@@ -1303,6 +1209,109 @@ void build_kb_tables(inqx_ham_s *h) {
   kb.built = true;
 }
 
+// The projector records of a grid whose cube fits the LDS (small_grid.hip), by group
+// at their offsets in the padded cube.  Built for the first H that runs there: a
+// precision whose cube does not fit, the energy record and the transforms read none.
+// False where a projector's sphere holds a point twice (periodic images).
+static bool small_tables(inqx_ham_s *h) {
+  KBTables &kb = h->kb;
+  if (kb.sg_built) return kb.sg_classes > 0;
+  const Grid &g = h->g;
+  hipStream_t st = h->ctx->c.stream;
+  const size_t cube = (size_t)g.n[0] * g.n[1] * (g.n[2] + 1);
+  // records padded to rows of 64 per group: offset -1, zero projector values
+  std::vector<int> row(1, 0), off, item, first(1, 0);
+  std::vector<float> v32, spos;
+  std::vector<double> v64;
+  std::vector<int> pts;
+  // classes of projectors that share no point, each projector in the first that takes it
+  std::vector<std::vector<char>> used;
+  std::vector<std::vector<int>> cls;  // [class] first group, groups, rows of a group of its projectors
+  bool twice = false;
+  std::vector<int> last(cube, -1);  // last projector that holds the point
+  for (int j = 0; j < (int)h->projs.size(); ++j) {
+    const Projector &P = h->projs[j];
+    const long np = P.npts(), padded = (np + 63) / 64 * 64;
+    const int ng = (P.nlm + kMaxNlm - 1) / kMaxNlm, a0 = (int)row.size() - 1;
+    pts.clear();
+    for (long p = 0; p < np; ++p) {
+      const int *c = &P.coords[3 * p], o = (c[0] * g.n[1] + c[1]) * (g.n[2] + 1) + c[2];
+      pts.push_back(o);
+      if (last[o] == j) twice = true;
+      last[o] = j;
+    }
+    for (int q = 0; q < ng; ++q) {
+      for (long p = 0; p < padded; ++p) {
+        const bool ok = p < np;
+        off.push_back(ok ? pts[p] : -1);
+        for (int l = 0; l < kMaxNlm; ++l) {
+          const int ch = kMaxNlm * q + l;
+          const double v = ok && ch < P.nlm ? P.matrix[(size_t)ch * np + p] : 0.0;
+          v32.push_back((float)v);
+          v64.push_back(v);
+        }
+        for (int d = 0; d < 3; ++d) spos.push_back(ok ? P.relpos[3 * (size_t)p + d] : 0.0f);
+        spos.push_back(0.0f);
+      }
+      row.push_back((int)(off.size() / 64));
+    }
+    size_t c = 0;
+    for (; c < cls.size(); ++c)
+      if (std::none_of(pts.begin(), pts.end(), [&](int o) { return used[c][o] != 0; })) break;
+    if (c == cls.size()) {
+      cls.emplace_back();
+      used.emplace_back(cube, 0);
+    }
+    cls[c].insert(cls[c].end(), {a0, ng, (int)(padded / 64)});
+    for (int o : pts) used[c][o] = 1;
+  }
+  kb.sg_nrec = (long)off.size();
+  for (auto &list : cls) {
+    for (size_t k = 0; k < list.size(); k += 3)
+      for (int r = 0; r < list[k + 2]; ++r) item.insert(item.end(), {row[list[k]] + r, list[k], list[k + 1], list[k + 2]});
+    first.push_back((int)(item.size() / 4));
+  }
+  kb.sg_classes = twice ? 0 : (int)cls.size();
+  kb.pos_host[1].swap(spos);
+  kb.pos[1].release();
+  std::vector<char> all;  // the tables in one allocation and one copy
+  const auto put = [&](const void *p, size_t bytes) {
+    const size_t at = (all.size() + 255) / 256 * 256;
+    all.resize(at + bytes);
+    if (bytes) std::memcpy(all.data() + at, p, bytes);
+    return at;
+  };
+  const size_t at_row = put(row.data(), sizeof(int) * row.size()), at_off = put(off.data(), sizeof(int) * off.size());
+  const size_t at32 = put(v32.data(), sizeof(float) * v32.size()), at64 = put(v64.data(), sizeof(double) * v64.size());
+  const size_t at_item = put(item.data(), sizeof(int) * item.size());
+  const size_t at_class = put(first.data(), sizeof(int) * first.size());
+  upload(kb.sg, all, st);
+  const char *base = kb.sg.as<char>();
+  kb.sg_row = reinterpret_cast<const int *>(base + at_row);
+  kb.sg_off = reinterpret_cast<const int *>(base + at_off);
+  kb.sg_b32 = base + at32;
+  kb.sg_b64 = base + at64;
+  kb.sg_item = reinterpret_cast<const int *>(base + at_item);
+  kb.sg_class = reinterpret_cast<const int *>(base + at_class);
+  INQX_HIP(hipStreamSynchronize(st));
+  kb.sg_built = true;
+  return kb.sg_classes > 0;
+}
+
+// a basis' sphere in the padded cube of a small grid: the points' offsets, then those
+// of the rows that hold points
+static void ensure_cube_tables(inqx_ham_s *h, Basis &b) {
+  if (b.d_cube.p) return;
+  const int n2 = h->g.n[2], n2p = n2 + 1;
+  std::vector<int> at(b.npw);
+  for (long i = 0; i < b.npw; ++i) at[i] = b.gidx[i] / n2 * n2p + b.gidx[i] % n2;
+  for (long i = 0; i < b.npw; ++i)
+    if (i == 0 || b.gidx[i] / n2 != b.gidx[i - 1] / n2) at.push_back(b.gidx[i] / n2 * n2p);
+  b.ncube_rows = (int)(at.size() - b.npw);
+  upload(b.d_cube, at, h->ctx->c.stream);
+  INQX_HIP(hipStreamSynchronize(h->ctx->c.stream));
+}
+
 void ensure_basis_device(inqx_ham_s *h, Basis &b) {
   hipStream_t st = h->ctx->c.stream;
   if (!b.d_pw_lw.p) {
@@ -1317,15 +1326,6 @@ void ensure_basis_device(inqx_ham_s *h, Basis &b) {
         const int y = b.pw_yz[q] / g.n[2], z = b.pw_yz[q] - y * g.n[2];
         lw[q] = (Grid::sym(y, g.n[1]) - ss[4] + 1) * n2p + z;
       }
-    }
-    std::vector<int> co, cr;  // offsets in the padded cube of a small grid
-    if (small_grid(g.n)) {
-      for (long i = 0; i < b.npw; ++i) co.push_back(b.gidx[i] / g.n[2] * n2p + b.gidx[i] % g.n[2]);
-      for (long i = 0; i < b.npw; ++i)
-        if (i == 0 || b.gidx[i] / g.n[2] != b.gidx[i - 1] / g.n[2]) cr.push_back(b.gidx[i] / g.n[2] * n2p);
-      b.ncube_rows = (int)cr.size();
-      upload(b.d_cube_off, co, st);
-      upload(b.d_cube_rows, cr, st);
     }
     upload(b.d_slot_seg, b.slot_seg, st);
     upload(b.d_rows, b.rows, st);
@@ -1786,7 +1786,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
   // run instead are launch and latency bound there (16 states at 20^3 complex128
   // 39 us against 25; 1024 states 190 against 97).  The energy record needs the x passes' dipole sums.
   const bool small = mode == 0 && !opts->observables && small_grid_fits(g.n, prec, has_kb ? h->kb.natoms : 0) &&
-                     (!has_kb || h->kb.sg_classes > 0);
+                     (!has_kb || small_tables(h));
   LaunchKey key;
   key.k.push_back((uintptr_t)prec);
   key.k.push_back((uintptr_t)mode);
@@ -1799,6 +1799,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
   if (has_kb) ensure_phase_tables<T>(h, nblocks, bases, small);
   for (int i = 0; i < nblocks; ++i) {
     ensure_basis_device(h, *bases[i]);
+    if (small) ensure_cube_tables(h, *bases[i]);
     ensure_workspace(h, *bases[i], nst[i], prec);
     key.k.push_back((uintptr_t)bases[i]);
     key.k.push_back((uintptr_t)nst[i]);
@@ -1924,8 +1925,8 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
       d.rs = mode == 1 || mode == 2 ? reinterpret_cast<cplx<T> *>(opts->rs[i]) : nullptr;
       d.rs_layout = opts->rs_layout;
       d.accumulate = opts->accumulate ? 1 : 0;
-      d.cube_off = B.d_cube_off.as<int>();
-      d.cube_rows = B.d_cube_rows.as<int>();
+      d.cube_off = small ? B.d_cube.as<int>() : nullptr;
+      d.cube_rows = small ? d.cube_off + B.npw : nullptr;
       d.ncube_rows = B.ncube_rows;
       d.acc1 = opts->acc1 ? reinterpret_cast<cplx<T> *>(opts->acc1[i]) : nullptr;
       d.acc2 = opts->acc2 ? reinterpret_cast<cplx<T> *>(opts->acc2[i]) : nullptr;

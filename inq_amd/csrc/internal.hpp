@@ -188,11 +188,13 @@ struct KBTables {
   // the same records for grids whose cube fits the LDS (small_grid.hip): by group,
   // each padded to rows of 64 (LDS offset; projector values; position), and the
   // rows of the projectors (first group's row, first group, groups, rows between
-  // groups) in classes of projectors that share no point.  sg_classes = 0: a
-  // projector's sphere holds a point twice (periodic images), not offered
+  // groups) in classes of projectors that share no point; built for the first H
+  // that reads them.  sg_classes = 0: a projector's sphere holds a point twice
+  // (periodic images), not offered
   DevMem sg;  // one allocation: sg_row, sg_off, ... below point into it
   const int *sg_row = nullptr, *sg_off = nullptr, *sg_item = nullptr, *sg_class = nullptr;
   const void *sg_b32 = nullptr, *sg_b64 = nullptr;
+  bool sg_built = false;
   int sg_classes = 0;
   long sg_nrec = 0;
   // float4 position of every record of the two orders, for the per-basis phase
@@ -278,7 +280,7 @@ struct Basis {
   int nwin_max = 0;           // longest row window of a plane
   std::vector<int> rows, pw_yz;
   DevMem d_slot_seg, d_rows, d_pw_lw, d_kin64, d_kin32;
-  DevMem d_cube_off, d_cube_rows;  // small grids (small_grid.hip)
+  DevMem d_cube;  // small grids (small_grid.hip), on first use: offsets of the points, then of the rows
   int ncube_rows = 0;
   DevMem d_g2h;  // (1/2)|G|^2 per sphere point, FP64, no k shift (preconditioner)
   DevMem d_gidx; // flattened FFT index per sphere point (layout conversions), on first use
@@ -382,7 +384,6 @@ template <typename T>
 void launch_rect_forward(Ctx &cx, const SphereBlock<T> *blk, const int *pref, int nblocks, int total, int pb,
                          int pstr, int n1, int n2, const double *cf);
 // small_grid.hip: H on blocks whose cube fits one work-group's LDS, a work-group per state
-bool small_grid(const int *n);
 bool small_grid_fits(const int *n, int prec, int natoms);
 template <typename T>
 void launch_small_apply(inqx_ham_s *h, const SphereBlock<T> *blk, const int *items, int total, bool has_kb,

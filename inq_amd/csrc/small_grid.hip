@@ -273,16 +273,12 @@ size_t part_bytes(int prec, int natoms) { return 2 * kMaxNlm * sizeof(double) * 
 
 }  // namespace
 
-// the lengths are built and the cube fits in the smaller precision
-bool small_grid(const int *n) {
-  return small_length(n[0]) && small_length(n[1]) && small_length(n[2]) && cube_bytes(n, INQX_FP32) <= kLdsBytes;
-}
-
-// the cube, the projection sums and D P fit the LDS
+// the lengths are built and the cube, the projection sums and D P fit the LDS
 bool small_grid_fits(const int *n, int prec, int natoms) {
-  return small_grid(n) && cube_bytes(n, prec) + 16 + part_bytes(prec, natoms) +
-                              (prec == INQX_FP64 ? 16 : 8) * (size_t)kMaxNlm * natoms <=
-                          (size_t)kLdsBytes;
+  return small_length(n[0]) && small_length(n[1]) && small_length(n[2]) &&
+         cube_bytes(n, prec) + 16 + part_bytes(prec, natoms) +
+                 (prec == INQX_FP64 ? 16 : 8) * (size_t)kMaxNlm * natoms <=
+             (size_t)kLdsBytes;
 }
 
 template <typename T>
