@@ -503,19 +503,18 @@ __global__ void __launch_bounds__(256) k_pair_reduce(PairDev<T> d, long nvec) {
 // of pair (s, j)'s, exchange_operator.hpp:144-160 with real kernels).
 //
 // The bound is the read of t, 3 MB a pair at 72^3 complex64; two kernels, one for
-// each sum, read it twice.  A work-group holds 64 points; wave k holds the states
-// i = base + u kRedWaves + k (u < U): their values and their w sums stay in
+// each sum, read it twice.  A work-group holds 64 points; wave k of W holds the
+// states i = base + u W + k (u < U): their values and their w sums stay in
 // registers while the rows jj stream by, a row's loads all in flight at once.  The
-// waves' parts of wb_j meet in LDS every kRedRows rows.  w_i is added in jj order
+// waves' parts of wb_j meet in LDS every red_rows rows.  w_i is added in jj order
 // and wb_j belongs to one chunk, so splitting the j range into chunks gives the
 // same bits.  128 states, 72^3 complex64 (8256 pairs): 12.9 -> 6.7 ms.
-constexpr int kRedWaves = 8;
 template <typename T> constexpr int red_rows() { return sizeof(T) == 4 ? 8 : 4; }
 
-template <typename T, int U>
-__global__ void __launch_bounds__(64 * kRedWaves) k_pair_reduce_both(PairDev<T> d, long N) {
+template <typename T, int W, int U>
+__global__ void __launch_bounds__(64 * W) k_pair_reduce_both(PairDev<T> d, long N) {
   using C = cplx<T>;
-  constexpr int W = kRedWaves, R = red_rows<T>();
+  constexpr int R = red_rows<T>();
   __shared__ C part[R][W][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long p = (long)blockIdx.x * 64 + lane, pc = p < N ? p : N - 1;
@@ -569,16 +568,15 @@ __global__ void __launch_bounds__(64 * kRedWaves) k_pair_reduce_both(PairDev<T> 
         part[jj - r0][wave][lane] = b;
       }
       __syncthreads();
-      // wave k adds row r0 + k of the tile
-      const int jj = r0 + wave;
-      if (wave < R && jj < r1) {
+      // wave k adds the rows r0 + k, r0 + k + W, ... of the tile
+      for (int jj = r0 + wave; jj < r1; jj += W) {
         const int j = gp(d.jlist)[jj];
         if (j > base && p < N) {
           C s = gw(d.wb)[(size_t)j * N + p];
 #pragma unroll
           for (int k = 0; k < W; ++k) {
-            s.x += part[wave][k][lane].x;
-            s.y += part[wave][k][lane].y;
+            s.x += part[jj - r0][k][lane].x;
+            s.y += part[jj - r0][k][lane].y;
           }
           gw(d.wb)[(size_t)j * N + p] = s;
         }
@@ -593,16 +591,20 @@ __global__ void __launch_bounds__(64 * kRedWaves) k_pair_reduce_both(PairDev<T> 
   }
 }
 
-// states per wave: enough for the block in one pass over the rows (more would be
-// empty loads), at most what the registers hold; further states take further passes
+// Waves and states per wave: enough for the block in one pass over the rows (more
+// would be empty loads and idle waves), at most eight and what the registers hold;
+// further states take further passes.  Two states at 128^3 complex64: 150 us with
+// eight waves, 35 with one (44 in the two kernels that read the pairs twice).
 template <typename T> void launch_pair_reduce_both(Ctx &cx, const PairDev<T> &d, long N) {
   constexpr int UMAX = sizeof(T) == 4 ? 16 : 8;
-  const dim3 grid((unsigned)((N + 63) / 64)), wg(64 * kRedWaves);
-  const int need = (d.nst + kRedWaves - 1) / kRedWaves;
-  if (need <= 2) hipLaunchKernelGGL((k_pair_reduce_both<T, 2>), grid, wg, 0, cx.stream, d, N);
-  else if (need <= 4) hipLaunchKernelGGL((k_pair_reduce_both<T, 4>), grid, wg, 0, cx.stream, d, N);
-  else if (need <= 8) hipLaunchKernelGGL((k_pair_reduce_both<T, 8>), grid, wg, 0, cx.stream, d, N);
-  else hipLaunchKernelGGL((k_pair_reduce_both<T, UMAX>), grid, wg, 0, cx.stream, d, N);
+  const dim3 grid((unsigned)((N + 63) / 64));
+  if (d.nst <= 2) hipLaunchKernelGGL((k_pair_reduce_both<T, 1, 2>), grid, dim3(64), 0, cx.stream, d, N);
+  else if (d.nst <= 4) hipLaunchKernelGGL((k_pair_reduce_both<T, 2, 2>), grid, dim3(128), 0, cx.stream, d, N);
+  else if (d.nst <= 8) hipLaunchKernelGGL((k_pair_reduce_both<T, 4, 2>), grid, dim3(256), 0, cx.stream, d, N);
+  else if (d.nst <= 16) hipLaunchKernelGGL((k_pair_reduce_both<T, 8, 2>), grid, dim3(512), 0, cx.stream, d, N);
+  else if (d.nst <= 32) hipLaunchKernelGGL((k_pair_reduce_both<T, 8, 4>), grid, dim3(512), 0, cx.stream, d, N);
+  else if (d.nst <= 64) hipLaunchKernelGGL((k_pair_reduce_both<T, 8, 8>), grid, dim3(512), 0, cx.stream, d, N);
+  else hipLaunchKernelGGL((k_pair_reduce_both<T, 8, UMAX>), grid, dim3(512), 0, cx.stream, d, N);
   INQX_HIP(hipGetLastError());
 }
 
