@@ -1739,24 +1739,48 @@ static void dispatch_passes(int n0, int n1, int n2, inqx_ham_s *h, LaunchData &l
 
 // x-pass waves (states) per work-group where the caller set none.  Four share a
 // tile's tables well and leave the LDS to several work-groups.
-//  * Two where four would leave CUs without a work-group: the passes are latency
-//    bound there (16 states at 32^3 complex128 41.9 us with four, 40.2 with two).
-//  * Eight where the tables are so large that the LDS holds more waves that way (d
-//    channels on 40 x 48 x 60 complex64, 40 states: 205 -> 192 us, 32 atoms of them
-//    at 60^3 204 -> 182), up to the waves the registers allow.
-//  * Two for complex128 lines from 72 points where two such groups fit the LDS: the
-//    registers hold one wave per SIMD, and a second group's line loads run while the
-//    first waits at its barrier (128 states at 72^3 918 -> 872 us, 96^3 508 -> 501;
-//    where the LDS holds one group of two, 16 states at 72^3 take 163 us against 128).
-// lds(n): bytes of a work-group of n waves; groups(n): the launch's work-groups
-template <typename T, typename FL, typename FG>
-static int auto_xwaves(int maxwaves, int n0, int maxnst, int num_cu, FL lds, FG groups) {
+//  * Two in complex64 where four leave CUs without a work-group and the busiest CU has
+//    fewer states with two (8 states, 40^3, d channels: 67.6 us with four, 57.0 with
+//    two; 20 states of them at 36^3, where groups of two come one after another: 71 and
+//    89).
+//  * Two in complex128 where every CU gets at most one such group (16 states at 32^3
+//    41.9 and 40.2 us; 8 at 48^3, 288 groups of two: 46.2 and 48.6).
+//  * Two for complex128 lines from 72 points where two such groups fit a CU's LDS: the
+//    second one's line loads run while the first waits at its barrier (96 states at
+//    72^3, k != 0: 644 and 629 us, 40 at 96^3 729 and 685; where one group of two
+//    fits, 688 and 962; at 60 and 64 points, which also have one wave per SIMD, two are
+//    1 % faster to 7 % slower).
+//  * Eight where the tables are so large that one group of four fits a CU and one of
+//    eight as well, and there are eight states for every CU (d channels on 40 x 48 x 60
+//    complex64, 96 states: 413 and 381 us; 20 states at 48^3, 216 groups of eight: 116
+//    and 137).  Where two groups of four fit, eight are slower (40 states at 48^3
+//    complex64 79 and 97), and where groups of four fill a few rounds and groups of
+//    eight do not (96 states on 32^3, three rounds and one and a half: 161 and 176;
+//    128 on 48^3, nine and four and a half: 354 and 323).
+// maxn: states of the largest block; tile, padded: tiles of a group of states, and with
+// those that complete the XCDs' round; lds(n): bytes of a work-group of n waves;
+// groups(n), full(n): groups of n states, and those that have n
+template <typename T, typename FL, typename FG, typename FF>
+static int auto_xwaves(int maxwaves, int n0, int maxn, int num_cu, long tiles, long padded, FL lds, FG groups, FF full) {
   const bool dbl = std::is_same<T, double>::value;
-  const int cap = dbl ? (n0 < 72 ? 8 : 4) : n0 <= 48 ? 16 : n0 <= 72 ? 12 : 8;  // resident waves of a CU by VGPRs
-  const auto resident = [&](int n) { return std::min(cap, n * (160 * 1024 / std::max(1, lds(n)))); };
-  if (groups(4) < num_cu) return 2;
-  if (dbl && n0 >= 72 && resident(2) == cap) return 2;
-  if (maxwaves >= 8 && maxnst >= 8 && groups(8) >= num_cu && resident(8) > resident(4)) return 8;
+  // waves of a CU that the compiled kernels' registers allow (more at the shortest
+  // complex128 lines, 12 in complex64 at 28 points)
+  const int cap = dbl ? (n0 < 60 ? 8 : 4) : n0 <= 54 ? 16 : n0 <= 72 ? 12 : n0 <= 108 ? 8 : 4;
+  const auto per_cu = [&](int n) { return std::max(1, std::min(160 * 1024 / std::max(1, lds(n)), cap / n)); };
+  const auto slots = [&](int n) { return (long)num_cu * per_cu(n); };
+  // rounds of resident work-groups; one on an eighth of the CUs or fewer adds little
+  const auto rounds = [&](int n) {
+    return std::max(1L, (8 * tiles * groups(n) + 7 * slots(n) - 1) / (8 * slots(n)));
+  };
+  const auto busiest = [&](int n) {  // states of the busiest slot, one group after another
+    const long r = rounds(n);
+    return n * (r - 1) + (tiles * full(n) > (r - 1) * slots(n) ? n : maxn % n);
+  };
+  if (tiles * groups(4) < num_cu && (dbl ? padded * groups(2) <= num_cu : busiest(2) < busiest(4))) return 2;
+  if (dbl && n0 >= 72 && 2 * per_cu(2) == cap) return 2;
+  if (maxwaves >= 8 && maxn >= 8 && tiles * groups(8) >= num_cu && lds(8) <= 160 * 1024 && per_cu(4) == 1 &&
+      !(tiles * groups(4) % slots(4) == 0 && busiest(8) > busiest(4) && rounds(8) < 3))
+    return 8;
   return 4;
 }
 
@@ -1889,13 +1913,16 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
       xp.wave0 = x.wave0 - x.cs;
       xp.wave_bytes = xp.aux + 64 * kMaxNlm * cs;
       if (h->xwaves[prec] == 0) {
-        const auto groups = [&](int n) {
+        const auto count = [&](auto per_block) {
           long c = 0;
-          for (int i = 0; i < nblocks; ++i) c += (long)h->kb.ntile * ((nst[i] + n - 1) / n);
+          for (int i = 0; i < nblocks; ++i) c += per_block(nst[i]);
           return c;
         };
-        nw = auto_xwaves<T>(maxwaves, g.n[0], *std::max_element(nst, nst + nblocks), h->ctx->c.num_cu,
-                         [&](int n) { return x.wave0 + n * x.wave_bytes; }, groups);
+        nw = auto_xwaves<T>(
+            maxwaves, g.n[0], *std::max_element(nst, nst + nblocks), h->ctx->c.num_cu, h->kb.ntile,
+            x_tiles_padded(h->kb.ntile), [&](int n) { return x.wave0 + n * x.wave_bytes; },
+            [&](int n) { return count([n](int ns) { return (ns + n - 1) / n; }); },
+            [&](int n) { return count([n](int ns) { return ns / n; }); });
       }
       constexpr int kLdsMax = 160 * 1024;
       INQX_CHECK(x.wave0 + x.wave_bytes <= kLdsMax && xp.wave0 + xp.wave_bytes <= kLdsMax, INQX_ERR_UNSUPPORTED,
