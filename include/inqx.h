@@ -146,11 +146,13 @@ int inqx_ham_prepare(inqx_ham ham, inqx_basis basis, int nst, int precision);
  * launch sequence, as inqx_ham_apply_batch runs them) for every launch shape
  * (x-pass states per work-group 1, 2, 4 or 8, times plane-pass planes per
  * work-group from the largest the grid's LDS budget allows down to 1) and
- * keeps the fastest for this Hamiltonian and precision.  cache_path: a text
- * file of earlier results, one line per (device, precision, grid, KB size,
- * blocks) key; a hit applies the stored shape without timing, a miss times and
- * appends (NULL: no cache).  shape[2] (out, may be NULL): x-pass states,
- * plane batch.  Allocates scratch states; do not call during graph capture. */
+ * keeps the fastest for this Hamiltonian and precision.  On a grid whose cube fits
+ * the LDS the plane and x passes are timed all the same, which the energies,
+ * transforms and densities run there; best_ms is the H application as it runs.
+ * cache_path: a text file of earlier results, one line per (device, precision,
+ * grid, KB size, blocks) key; a hit applies the stored shape without timing, a
+ * miss times and appends (NULL: no cache).  shape[2] (out, may be NULL): x-pass
+ * states, plane batch.  Allocates scratch states; do not call during graph capture. */
 int inqx_ham_autotune_batch(inqx_ham ham, int nblocks, const inqx_basis *bases, const int *nst, int precision,
                             const char *cache_path, int *shape, double *best_ms);
 /* sets the plane-pass batch directly (planes per work-group; 0: the most that leave

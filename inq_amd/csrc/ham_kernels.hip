@@ -1809,8 +1809,8 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
   // of states: fewer than the CUs leave some idle, but the five passes they would
   // run instead are launch and latency bound there (16 states at 20^3 complex128
   // 39 us against 25; 1024 states 190 against 97).  The energy record needs the x passes' dipole sums.
-  const bool small = mode == 0 && !opts->observables && small_grid_fits(g.n, prec, has_kb ? h->kb.natoms : 0) &&
-                     (!has_kb || small_tables(h));
+  const bool small = mode == 0 && !opts->observables && !opts->passes &&
+                     small_grid_fits(g.n, prec, has_kb ? h->kb.natoms : 0) && (!has_kb || small_tables(h));
   LaunchKey key;
   key.k.push_back((uintptr_t)prec);
   key.k.push_back((uintptr_t)mode);
@@ -1818,6 +1818,7 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
   key.k.push_back((uintptr_t)(opts->accumulate ? 1 : 0));
   key.k.push_back((uintptr_t)h->xwaves[prec]);
   key.k.push_back((uintptr_t)h->plane_batch[prec]);
+  key.k.push_back((uintptr_t)(small ? 1 : 0));
   if (mode == 1 || mode == 2)
     for (int i = 0; i < nblocks; ++i) key.k.push_back((uintptr_t)opts->rs[i]);
   if (has_kb) ensure_phase_tables<T>(h, nblocks, bases, small);

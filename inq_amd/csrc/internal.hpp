@@ -260,6 +260,7 @@ struct ApplyOpts {
   // 3: one block's density (psi -> *density)
   int mode = 0;
   const DensityOut *density = nullptr;
+  bool passes = false;          // mode 0: the plane and x passes also where the cube fits the LDS
   void *const *rs = nullptr;    // per block real-space arrays for modes 1 and 2
   int rs_layout = 0;            // 0: [nst][N], 1: [N][nst]
   bool accumulate = false;      // mode 2: hpsi += result
