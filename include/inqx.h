@@ -161,7 +161,8 @@ int inqx_ham_autotune_batch(inqx_ham ham, int nblocks, const inqx_basis *bases, 
 int inqx_ham_set_plane_batch(inqx_ham ham, int precision, int planes);
 /* the single-block form (no cache); best_xwaves / best_ms may be NULL */
 int inqx_ham_autotune(inqx_ham ham, inqx_basis basis, int nst, int precision, int *best_xwaves, double *best_ms);
-/* sets the x-pass shape directly (1, 2, 4 or 8 states per work-group) */
+/* sets the x-pass shape directly (1, 2, 4 or 8 states per work-group; 0, the default:
+ * chosen for each launch by its states and the LDS) */
 int inqx_ham_set_launch_shape(inqx_ham ham, int precision, int xwaves);
 
 /* ------------------------------------------------------------ H |psi> */

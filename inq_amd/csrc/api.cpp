@@ -605,8 +605,8 @@ int inqx_ham_set_launch_shape(inqx_ham h, int precision, int xwaves) {
   API_BEGIN
   INQX_CHECK(h, INQX_ERR_ARG, "null Hamiltonian");
   INQX_CHECK(precision == INQX_FP64 || precision == INQX_FP32, INQX_ERR_ARG, "bad precision");
-  INQX_CHECK(xwaves == 1 || xwaves == 2 || xwaves == 4 || xwaves == 8, INQX_ERR_ARG,
-             "x-pass shape must be 1, 2, 4 or 8");
+  INQX_CHECK(xwaves == 0 || xwaves == 1 || xwaves == 2 || xwaves == 4 || xwaves == 8, INQX_ERR_ARG,
+             "x-pass shape must be 0 (automatic), 1, 2, 4 or 8");
   INQX_CHECK(h->pinned == 0, INQX_ERR_STATE, "Hamiltonian pinned by a captured propagation graph");
   if (h->xwaves[precision] != xwaves) {
     h->xwaves[precision] = xwaves;
