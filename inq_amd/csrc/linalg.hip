@@ -532,7 +532,10 @@ k_rotate(const cplx<T> *Mm, int ld, const cplx<T> *Cm, int nr, int nc, long K,
 //                  to the unused upper tile (c0, i)
 //   k_chol_finish  moves the panels from the upper to the lower triangle
 // One launch per panel instead of three, and tiles of 32 also for the small
-// blocks: n = 128 150 -> 83 us, n = 432 690 -> 290 us.
+// blocks: n = 128 150 -> 83 us, n = 432 690 -> 290 us.  Up to n = 64 one work-group
+// did it in one launch before; two launches without k_chol_finish, and a last tile
+// that takes the steps of its rows only: n = 33 42 us then, 44 now, n = 40 48
+// and 44, n = 64 69 and 54.
 // info[0] = 0 or the first non-positive leading minor (LAPACK convention); the first
 // launch writes it, and every later launch returns at once when it is set.
 constexpr int kChB = 32;
@@ -669,7 +672,9 @@ __device__ __forceinline__ void panel_step(double2 (&x)[4], const ctile &Lk, con
   if (c == own) x[q] = v;
 }
 
-__global__ void __launch_bounds__(256) k_chol_step(double *S, int n, int c0, int *info) {
+// whole: the matrix has two panels, so this work-group is the only one; it leaves L in
+// place instead of k_chol_finish
+__global__ void __launch_bounds__(256) k_chol_step(double *S, int n, int c0, int whole, int *info) {
   __shared__ ctile Lk, Li, Lj;
   __shared__ double rd[kChB];
   __shared__ double2 col[2][2 * kChB];
@@ -707,7 +712,17 @@ __global__ void __launch_bounds__(256) k_chol_step(double *S, int n, int c0, int
   }
   __syncthreads();
   GAS double2 *g = (GAS double2 *)lgw(S);
-  if (tj == 0) {
+  if (whole) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + 256 * u, k = e >> 5, m = e & 31;
+      const double2 zero{0.0, 0.0};
+      if (i0 + k < n) g[(long)(i0 + k) * n + c0 + m] = Li[k][m];
+      if (i0 + m < n) g[(long)(c0 + k) * n + i0 + m] = zero;
+      if (m > k) g[(long)(c0 + k) * n + c0 + m] = zero;
+      if (m > k && i0 + m < n) g[(long)(i0 + k) * n + i0 + m] = zero;
+    }
+  } else if (tj == 0) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {  // L_i^H to the upper tile (c0, i0)
       const int e = tid + 256 * u, k = e >> 5, m = e & 31;
@@ -734,7 +749,10 @@ __global__ void __launch_bounds__(256) k_chol_step(double *S, int n, int c0, int
   }
   if (!next) return;
   __syncthreads();
-  if (tid < 64) factor_tile<kChB>(Lj, col, S, n, i0, info, false);
+  if (tid >= 64) return;
+  if (n - i0 <= 8) factor_tile<8>(Lj, col, S, n, i0, info, false);
+  else if (n - i0 <= 16) factor_tile<16>(Lj, col, S, n, i0, info, false);
+  else factor_tile<kChB>(Lj, col, S, n, i0, info, false);
 }
 
 __global__ void __launch_bounds__(256) k_chol_finish(double *S, int n, const int *info) {
@@ -767,9 +785,30 @@ __global__ void __launch_bounds__(256) k_chol_finish(double *S, int n, const int
 //   k_trinv_diag   one wave per diagonal tile: lane (column c, half h) keeps the
 //                  rows 2 q + h of its column of X; tiles above the diagonal zeroed
 //   k_trinv_merge  one 32 x 32 tile of T = L_21 X_11 or of X_21 = -X_22 T
-// forward substitution of one column of the inverse of a tile, its first STEPS rows
+// the inverse of the diagonal tile of b <= STEPS rows at r0, in one wave
 template <int STEPS>
-__device__ __forceinline__ void invert_steps(const ctile &t, const double2 (&id)[kChB], double2 (&x)[kChB / 2], int h) {
+__device__ __forceinline__ void invert_tile(ctile &t, double2 (&id)[kChB], const GAS double2 *lg, GAS double2 *g, int n,
+                                            int r0, int b) {
+  const int lane = threadIdx.x;
+#pragma unroll 4
+  for (int u = 0; u < STEPS / 2; ++u) {
+    const int e = lane + 64 * u, i = e >> 5, j = e & 31;
+    double2 v{i == j ? 1.0 : 0.0, 0.0};  // identity past the last row
+    if (i < b && j <= i) v = lg[(long)(r0 + i) * n + r0 + j];
+    t[i][j] = v;
+  }
+  __syncthreads();
+  if (lane < STEPS) {
+    const double2 l = t[lane][lane];
+    const double m = 1.0 / (l.x * l.x + l.y * l.y);
+    id[lane] = double2{l.x * m, -l.y * m};
+  }
+  __syncthreads();
+  const int c = lane & 31, h = lane >> 5;
+  double2 x[STEPS / 2];
+#pragma unroll
+  for (int q = 0; q < STEPS / 2; ++q) x[q] = double2{2 * q + h == c ? 1.0 : 0.0, 0.0};
+  // forward substitution, a column of the inverse per lane pair
 #pragma unroll
   for (int j = 0; j < STEPS; ++j) {
     __builtin_amdgcn_sched_barrier(0);  // one step's values in registers at a time
@@ -790,8 +829,17 @@ __device__ __forceinline__ void invert_steps(const ctile &t, const double2 (&id)
       }
     __builtin_amdgcn_sched_barrier(0);
   }
+#pragma unroll
+  for (int q = 0; q < STEPS / 2; ++q) t[2 * q + h][c] = x[q];  // its column, read by no other lane's steps now
+  __syncthreads();
+#pragma unroll 4
+  for (int u = 0; u < STEPS / 2; ++u) {
+    const int e = lane + 64 * u, i = e >> 5, j = e & 31;
+    if (i < b && j < b) g[(long)(r0 + i) * n + r0 + j] = j <= i ? t[i][j] : double2{0.0, 0.0};
+  }
 }
 
+// X = L^{-1}: the diagonal tiles; tiles above the diagonal zeroed
 __global__ void __launch_bounds__(64) k_trinv_diag(const double *L, int n, double *X) {
   __shared__ ctile t;
   __shared__ double2 id[kChB];  // 1 / L[i][i]
@@ -808,35 +856,10 @@ __global__ void __launch_bounds__(64) k_trinv_diag(const double *L, int n, doubl
     return;
   }
   const int b = min(kChB, n - r0);
-#pragma unroll 4
-  for (int u = 0; u < 16; ++u) {
-    const int e = lane + 64 * u, i = e >> 5, j = e & 31;
-    double2 v{i == j ? 1.0 : 0.0, 0.0};  // identity past the last row
-    if (i < b && j <= i) v = lg[(long)(r0 + i) * n + r0 + j];
-    t[i][j] = v;
-  }
-  __syncthreads();
-  if (lane < kChB) {
-    const double2 l = t[lane][lane];
-    const double m = 1.0 / (l.x * l.x + l.y * l.y);
-    id[lane] = double2{l.x * m, -l.y * m};
-  }
-  __syncthreads();
-  const int c = lane & 31, h = lane >> 5;
-  double2 x[kChB / 2];
-#pragma unroll
-  for (int q = 0; q < kChB / 2; ++q) x[q] = double2{2 * q + h == c ? 1.0 : 0.0, 0.0};
-  if (b <= 8) invert_steps<8>(t, id, x, h);
-  else if (b <= 16) invert_steps<16>(t, id, x, h);
-  else invert_steps<kChB>(t, id, x, h);
-#pragma unroll
-  for (int q = 0; q < kChB / 2; ++q) t[2 * q + h][c] = x[q];  // its column, read by no other lane's steps now
-  __syncthreads();
-#pragma unroll 4
-  for (int u = 0; u < 16; ++u) {
-    const int e = lane + 64 * u, i = e >> 5, j = e & 31;
-    if (i < b && j < b) g[(long)(r0 + i) * n + r0 + j] = j <= i ? t[i][j] : double2{0.0, 0.0};
-  }
+  if (b <= 2) invert_tile<2>(t, id, lg, g, n, r0, b);
+  else if (b <= 8) invert_tile<8>(t, id, lg, g, n, r0, b);
+  else if (b <= 16) invert_tile<16>(t, id, lg, g, n, r0, b);
+  else invert_tile<kChB>(t, id, lg, g, n, r0, b);
 }
 
 // pair blockIdx.z of blocks of `blk` rows; tile (blockIdx.y, blockIdx.x) of its
@@ -1080,9 +1103,11 @@ void launch_cholesky(Ctx &cx, int n, double *S, int *info) {
   if (nb == 1) return;
   for (int b = 0; b + 1 < nb; ++b) {
     const int m = nb - 1 - b;  // tile rows of the trailing triangle
-    hipLaunchKernelGGL(k_chol_step, dim3(m * (m + 1) / 2), dim3(256), 0, cx.stream, S, n, kChB * b, info);
+    hipLaunchKernelGGL(k_chol_step, dim3(m * (m + 1) / 2), dim3(256), 0, cx.stream, S, n, kChB * b, nb == 2 ? 1 : 0,
+                       info);
     INQX_HIP(hipGetLastError());
   }
+  if (nb == 2) return;
   hipLaunchKernelGGL(k_chol_finish, dim3(nb * (nb + 1) / 2), dim3(256), 0, cx.stream, S, n, (const int *)info);
   INQX_HIP(hipGetLastError());
 }
