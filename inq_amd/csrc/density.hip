@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256) k_line_density(const cplx<T> *t1, int m_l
       }
       v[n] = x;
     }
-    line_dit<N0, +1, C, S>(v, q);
+    line_dit<N0, +1, C, S, true>(v, q);
 #pragma unroll
     for (int k = 0; k < M; ++k) {
       const double re = (double)(v[k].x * scale), im = (double)(v[k].y * scale);

@@ -358,7 +358,8 @@ template <int N, int SIGN, typename C> struct fft_split {
   }
 };
 
-template <int N, int SIGN, typename C> struct fft_quad {
+// ONE: dit's last butterflies take W_N^k part_turn(q) as one rounded factor (complex64)
+template <int N, int SIGN, typename C, bool ONE = false> struct fft_quad {
   static_assert(N % 4 == 0, "four-lane lines need a length divisible by 4");
   static constexpr int Q = N / 4;
   using T = decltype(C{}.x);
@@ -367,6 +368,23 @@ template <int N, int SIGN, typename C> struct fft_quad {
     const T r = (T)0.70710678118654752440;
     const C w = q >= 2 ? C{r, (T)SIGN * r} : C{(T)1, (T)0};
     return quarter_if<SIGN>(w, (q & 1) != 0);
+  }
+  // v W_N^k part_turn(q).  Two factors round once more than one that is chosen from the
+  // two a part's half may have.  Density in complex64, rms error with two factors, with
+  // one and with two lanes per line: 1.49e-7, 1.43e-7 and 1.38e-7 at 24^3, 1.93e-7,
+  // 1.87e-7 and 1.82e-7 at 64^3 (the choice costs its line pass 0 to 6 %).  The pair
+  // planes, bound by VALU issue, keep two: the choice cost 9 to 36 % there, and their
+  // solves' error is the same either way within 4 % (2.57e-7 and 2.47e-7 at 72^3, 2.08e-7
+  // and 2.14e-7 at 80^3; 2.48e-7 and 2.17e-7 with two lanes)
+  static __device__ __forceinline__ C part_twmul(C v, int k, int q, C rho) {
+    if constexpr (ONE && sizeof(T) == 4) {
+      const bool hi = q >= 2;
+      const T c = hi ? (T)kTw<N>.c[k + N / 8] : (T)kTw<N>.c[k];
+      const T s = hi ? (T)SIGN * (T)kTw<N>.s[k + N / 8] : (T)SIGN * (T)kTw<N>.s[k];
+      return quarter_if<SIGN>(C{v.x * c - v.y * s, v.x * s + v.y * c}, (q & 1) != 0);
+    } else {
+      return twmul<N, SIGN>(cmul(v, rho), k);
+    }
   }
   // decimation in time: part q holds x[4n + q] (n < Q)
   static __device__ __forceinline__ void dit(C (&v)[Q], int q) {
@@ -390,7 +408,7 @@ template <int N, int SIGN, typename C> struct fft_quad {
       for (int k = 0; k < Q / 2; ++k) {
         C e = v[k], o = v[k + Q / 2];
         cswap16(e, o);
-        const C t = twmul<N, SIGN>(cmul(o, rho), k);
+        const C t = part_twmul(o, k, q, rho);
         v[k] = cadd(e, t);
         v[k + Q / 2] = csub(e, t);
       }

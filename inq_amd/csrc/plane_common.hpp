@@ -129,11 +129,11 @@ __device__ __forceinline__ void plane_row_split(C *row, bool upper, bool ok) {
 }
 
 // the transform of a line split over S lanes (part q of the line): input
-// x[S n + q], output order line_out_j + line_out_q (fft_reg.hpp)
-template <int N, int SIGN, typename C, int S>
+// x[S n + q], output order line_out_j + line_out_q; ONE as in fft_quad (fft_reg.hpp)
+template <int N, int SIGN, typename C, int S, bool ONE = false>
 __device__ __forceinline__ void line_dit(C (&v)[N / S], int q) {
   if constexpr (S == 2) fft_split<N, SIGN, C>::dit(v, q != 0);
-  else fft_quad<N, SIGN, C>::dit(v, q);
+  else fft_quad<N, SIGN, C, ONE>::dit(v, q);
 }
 // the mirror: input in line_dit's output order, output x[S k + q] (line_dit's input order)
 template <int N, int SIGN, typename C, int S>
