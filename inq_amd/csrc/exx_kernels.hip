@@ -79,6 +79,7 @@ template <typename T, int N1, int N2> struct PairPlaneCfg {
   // planes within 1 %
   static constexpr bool HALVES = N1 * STRIDE * (int)sizeof(cplx<T>) > 40 * 1024;
   static constexpr int LDS = N1 * STRIDE * (int)sizeof(cplx<T>) / (HALVES ? 2 : 1);
+  static_assert(LDS <= 160 * 1024, "a plane, or half of its values, fits a CU's LDS");
 };
 template <typename T, int N1, int N2> constexpr int pair_plane_maxt() { return PairPlaneCfg<T, N1, N2>::MAXT; }
 
@@ -149,6 +150,8 @@ __device__ __forceinline__ double rcp_t(double x) { return 1.0 / x; }
 // 72^3 complex64 at 4.8 TB/s, the forward one is bound by VALU issue (5.4 ms of it)
 // and stores together: forward 11.7 -> 9.9 ms, inverse 11.0 -> 10.2 ms.  One solve
 // at 72^3 complex128 8.7 -> 7.1 us.
+// A plain Poisson solve runs in place (phi = t): the work-group's loads are all in
+// registers before its first barrier (in lds_exchange), and its stores follow it.
 template <typename T, int N1, int N2>
 __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_fwd(PairDev<T> d, int total) {
   using C = cplx<T>;
@@ -275,8 +278,9 @@ __global__ void __launch_bounds__(256) k_pair_xline(PairDev<T> d, int total) {
   }
 }
 
-// inverse 2D transform of one pair plane in place: the plane is whole in LDS before
-// the first store.  k_pair_reduce(_both) then forms sum_j c_j hf_j t_j.
+// inverse 2D transform of one pair plane in place, as in the forward pass: every load of
+// the work-group precedes its first barrier, every store follows it.
+// k_pair_reduce(_both) then forms sum_j c_j hf_j t_j.
 template <typename T, int N1, int N2>
 __global__ void __launch_bounds__((pair_plane_maxt<T, N1, N2>())) k_pair_plane_inv(PairDev<T> d, int total) {
   using C = cplx<T>;
@@ -859,22 +863,15 @@ bool pair_grid_supported(const int *n) {
 }
 
 namespace {
-// square planes whose LDS plane passes do not fit the CU's 160 KB (complex128
-// from 100 points) run the column and row kernels instead
-template <typename T, int S0, int S> void run_pairs_square(inqx_ham_s *h, const PairArgs &a) {
-  if constexpr (PairPlaneCfg<T, S, S>::LDS > 160 * 1024) run_pairs<T, S0, 0>(h, a);
-  else run_pairs<T, S0, S>(h, a);
-}
-
 template <typename T, int S0> void pairs_n12(inqx_ham_s *h, const PairArgs &a) {
   if (h->g.n[1] != h->g.n[2]) {
     run_pairs<T, S0, 0>(h, a);
     return;
   }
   switch (h->g.n[1]) {
-#define CASE(S)                          \
-  case S:                                \
-    run_pairs_square<T, S0, S>(h, a);    \
+#define CASE(S)                   \
+  case S:                         \
+    run_pairs<T, S0, S>(h, a);    \
     break;
     INQX_SIZES(CASE)
 #undef CASE
