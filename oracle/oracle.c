@@ -555,24 +555,29 @@ static void projections(const orc_ham *h, int nst, const double *kcov, const cpl
 }
 
 /* project (gemm 2, projector_all.hpp:215-272) + apply (scatter-add with
- * exp(-i k.pos), projector_all.hpp:276-288).  Serial over projectors so that
- * overlapping spheres accumulate in a fixed order. */
+ * exp(-i k.pos), projector_all.hpp:276-288).  Serial over projectors and over a
+ * projector's points, parallel over states: overlapping spheres, and a sphere that
+ * holds a point twice through periodic images, accumulate in a fixed order. */
 static void kb_apply(const orc_ham *h, int nst, const double *kcov, const cplx *dproj, int nlm_stride,
                      cplx *hphi) {
   const grid_t *g = &h->g;
   for (int a = 0; a < h->nproj; ++a) {
     const proj_t *p = &h->proj[a];
     const cplx *pa = dproj + (long)a * nlm_stride * nst;
-#pragma omp parallel for schedule(static)
-    for (long ip = 0; ip < p->npts; ++ip) {
-      cplx ph = kb_phase(kcov, p->relpos + 3 * ip, -1.0);
-      cplx *dst = hphi + pidx(g, p->coords + 3 * ip) * nst;
-      for (int s = 0; s < nst; ++s) {
-        cplx t = 0.0;
-        for (int l = 0; l < p->nlm; ++l) t += p->matrix[(long)l * p->npts + ip] * pa[l * nst + s];
-        dst[s] += ph * t;
-      }
+    cplx *ph = (cplx *)malloc(sizeof(cplx) * (size_t)(p->npts > 0 ? p->npts : 1));
+#pragma omp parallel
+    {
+#pragma omp for schedule(static)
+      for (long ip = 0; ip < p->npts; ++ip) ph[ip] = kb_phase(kcov, p->relpos + 3 * ip, -1.0);
+#pragma omp for schedule(static)
+      for (int s = 0; s < nst; ++s)
+        for (long ip = 0; ip < p->npts; ++ip) {
+          cplx t = 0.0;
+          for (int l = 0; l < p->nlm; ++l) t += p->matrix[(long)l * p->npts + ip] * pa[l * nst + s];
+          hphi[pidx(g, p->coords + 3 * ip) * nst + s] += ph[ip] * t;
+        }
     }
+    free(ph);
   }
 }
 
