@@ -292,8 +292,11 @@ int inqx_ctx_destroy(inqx_ctx ctx) {
       ctx->c.event_pool.push_back(p.second.second);
     }
     for (auto e : ctx->c.event_pool) (void)hipEventDestroy(e);
+    ctx->c.pending.clear();
+    ctx->c.event_pool.clear();
   }
-  delete ctx;
+  ctx->closed = true;
+  if (ctx->hams == 0) delete ctx;
   return INQX_OK;
 }
 
@@ -398,6 +401,7 @@ int inqx_ham_create(inqx_ctx ctx, const double lattice[9], const int n[3], inqx_
     delete h;
     INQX_CHECK(false, INQX_ERR_ARG, "the lattice volume is not positive");
   }
+  ++ctx->hams;
   *out = h;
   API_END(ctx)
 }
@@ -411,7 +415,9 @@ int inqx_ham_destroy(inqx_ham h) {
   invalidate_launch_cache(h);
   release_ks_work(h);
   for (auto b : h->bases) b->b.ham = nullptr;
+  inqx_ctx ctx = h->ctx;
   delete h;
+  if (--ctx->hams == 0 && ctx->closed) delete ctx;
   return INQX_OK;
 }
 

@@ -4,7 +4,6 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
-
 #include <cstdint>
 #include <cstdio>
 #include <map>
@@ -320,6 +319,10 @@ struct Basis {
 
 struct inqx_ctx_s {
   inqx::Ctx c;
+  // Hamiltonians hold their context: destroyed before one of them (a garbage collector's
+  // order), it is released with the last
+  std::atomic<int> hams{0};
+  std::atomic<bool> closed{false};
 };
 
 struct inqx_ham_s {
