@@ -583,6 +583,7 @@ int inqx_ham_prepare(inqx_ham h, inqx_basis bs, int nst, int precision) {
   INQX_CHECK(precision == INQX_FP64 || precision == INQX_FP32, INQX_ERR_ARG, "bad precision");
   if (!h->kb.built) build_kb_tables(h);
   ensure_basis_device(h, bs->b);
+  ensure_small_apply(h, bs->b, precision);
   ensure_workspace(h, bs->b, nst, precision);
   API_END(ctx)
 }

@@ -1312,6 +1312,15 @@ static void ensure_cube_tables(inqx_ham_s *h, Basis &b) {
   INQX_HIP(hipStreamSynchronize(h->ctx->c.stream));
 }
 
+// the tables of H on a grid whose cube fits the LDS at this precision; false elsewhere
+static bool small_apply_tables(inqx_ham_s *h, int prec) {
+  const int natoms = h->kb.natoms;
+  return small_grid_fits(h->g.n, prec, natoms) && (natoms == 0 || small_tables(h));
+}
+void ensure_small_apply(inqx_ham_s *h, Basis &b, int prec) {
+  if (small_apply_tables(h, prec)) ensure_cube_tables(h, b);
+}
+
 void ensure_basis_device(inqx_ham_s *h, Basis &b) {
   hipStream_t st = h->ctx->c.stream;
   if (!b.d_pw_lw.p) {
@@ -1805,12 +1814,14 @@ void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *ns
     INQX_CHECK(opts->rs != nullptr, INQX_ERR_ARG, "transform without real-space arrays");
   }
   const bool has_kb = mode == 0 && h->kb.natoms > 0;
-  // a cube that fits the LDS runs as one work-group per state, whatever the number
-  // of states: fewer than the CUs leave some idle, but the five passes they would
-  // run instead are launch and latency bound there (16 states at 20^3 complex128
-  // 39 us against 25; 1024 states 190 against 97).  The energy record needs the x passes' dipole sums.
-  const bool small = mode == 0 && !opts->observables && !opts->passes &&
-                     small_grid_fits(g.n, prec, has_kb ? h->kb.natoms : 0) && (!has_kb || small_tables(h));
+  // a cube that fits the LDS runs as one work-group per state.  The number of states
+  // does not enter, so that a block's bits do not depend on how many are applied with
+  // it.  16 states at 20^3 complex128 39 us in five passes and 25, 1024 states 190 and 97,
+  // 512 at 24^3 complex64 with 40 atoms 2311 and 165; the longest chains of one
+  // work-group lose to five passes that spread few states over the chip: one state at
+  // 20^3 complex128 without projectors 15 and 18, eight at 24^3 complex64 with 40 atoms
+  // 73 and 81.  The energy record needs the x passes' dipole sums.
+  const bool small = mode == 0 && !opts->observables && !opts->passes && small_apply_tables(h, prec);
   LaunchKey key;
   key.k.push_back((uintptr_t)prec);
   key.k.push_back((uintptr_t)mode);

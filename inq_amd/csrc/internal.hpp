@@ -374,6 +374,8 @@ template <typename T>
 void launch_apply(inqx_ham_s *h, int nblocks, Basis *const *bases, const int *nst, const void *const *psi,
                   void *const *hpsi, const ApplyOpts *opts = nullptr);
 void ensure_basis_device(inqx_ham_s *h, Basis &b);
+// what H of the basis reads on a grid whose cube fits the LDS (nothing elsewhere)
+void ensure_small_apply(inqx_ham_s *h, Basis &b, int prec);
 void ensure_workspace(inqx_ham_s *h, Basis &b, int nst, int prec);
 bool grid_supported(const int *n);
 int max_plane_batch(const int *n, int prec);
