@@ -138,8 +138,10 @@ int inqx_basis_size(inqx_basis basis, long *npw);
 int inqx_basis_gindex(inqx_basis basis, int *gidx);
 /* 1/2 |G+k+A|^2 per sphere point (host, FP64) */
 int inqx_basis_kinetic(inqx_basis basis, double *kin);
-/* allocate the workspaces apply needs for nst states at a precision, so that
- * later calls allocate nothing (required before hipGraph capture) */
+/* allocate the workspaces and tables apply needs for nst states at a precision, so
+ * that later calls allocate nothing (required before hipGraph capture), but for the
+ * projector phases of a block with k + A != 0 and the descriptor of a launch, which
+ * the first application on those states builds */
 int inqx_ham_prepare(inqx_ham ham, inqx_basis basis, int nst, int precision);
 
 /* launch-shape autotuner: times the H application of the given blocks (one
