@@ -76,11 +76,16 @@ __device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, unsigned voff, 
   i2 q = {__float_as_int(v.x), __float_as_int(v.y)};
   __builtin_amdgcn_raw_buffer_store_b64(q, r, voff, soff, 0);
 }
+// The wave-uniform offset of a 16-byte store is added to the lane's.  gfx950 wants two wait
+// states between a store of more than 8 bytes and a VALU write of its data registers;
+// the compiler keeps them where the store's offset field is constant and none where it
+// is an SGPR, and the next value of a line then overwrote data that the store had yet to
+// read: at 54^3 one line in 10^5 held a wrong value.
 __device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, cplx<double> v) {
   typedef int i4 __attribute__((ext_vector_type(4)));
   const long long a = __double_as_longlong(v.x), b = __double_as_longlong(v.y);
   i4 q = {(int)a, (int)(a >> 32), (int)b, (int)(b >> 32)};
-  __builtin_amdgcn_raw_buffer_store_b128(q, r, voff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(q, r, voff + soff, 0, 0);
 }
 
 // a per-lane buffer offset beyond every record: loads return 0, stores are dropped
