@@ -45,6 +45,7 @@ __device__ __forceinline__ int find_block(const int *prefix, int nblocks, int wg
 }
 
 // ---- raw buffer access: per-lane byte offset in a VGPR, wave-uniform part in an SGPR
+// (complex128 stores: see there)
 // the base and size of a buffer resource are wave-uniform by construction;
 // readfirstlane makes that explicit so the resource stays in SGPRs
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, unsigned bytes) {
